@@ -27,6 +27,15 @@
  *  hm_col_kernel   one workgroup per column: the log10 sum over genes of
  *                  those contributions, the likelihood and pi0's sum
  *                  (eqtlbma_hm.cpp:617-868).
+ * Configs model: every one of those sums is linear in the 10^raw of a gene's
+ * SNPs, and the SNPs of a gene all weigh 1/P, so the EM and the likelihood
+ * walk of --getci need a gene's SNPs only through
+ *   A[k][l] = log10 (1/P) sum_p 10^raw[p][k][l],
+ * which no parameter enters.  hm_collapse_kernel reads the raw ABFs once per
+ * call and leaves one pseudo-SNP A per gene; the passes then run on those.
+ * A gene with a raw ABF that is not finite keeps its SNPs (the reference's
+ * NaN rules are not linear), and a pass whose weights are NaN or negative
+ * (SQUAREM's proposals) runs on the SNPs themselves.
  * The host then normalises the new weights exactly as the reference does
  * (log10 sums with the previous weight added, divided by their log10 sum)
  * and runs the reference's iteration logic; one pass per EM iteration, all
@@ -35,9 +44,11 @@
  * NaN first element makes the sum NaN), NaN terms are skipped, and a result
  * within DBL_EPSILON of zero is zero.
  */
+#include <algorithm>
 #include <cfloat>
 #include <cmath>
 #include <cstring>
+#include <string>
 #include <vector>
 
 #include "eqbf_internal.h"
@@ -58,7 +69,7 @@ __device__ inline double hm_wave_lws(double v, double w, bool valid, double firs
   double m = (valid && !isnan(v)) ? v : -INFINITY;
   for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
   if (isnan(first)) m = NAN;
-  double s = (valid && !isnan(v)) ? w * exp10(v - m) : 0.0;
+  double s = (valid && !isnan(v)) ? w * dm::exp10_sum(v - m) : 0.0;
   for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
   return hm_finish(m, s);
 }
@@ -104,7 +115,7 @@ __global__ void __launch_bounds__(HM_NT) hm_pair_kernel(const HmDev h) {
         if (r[l] > m) m = r[l];
       double s = 0.0;
       for (int l = 0; l < L; ++l)
-        if (!isnan(r[l])) s += grid[l] * exp10(r[l] - m);
+        if (!isnan(r[l])) s += grid[l] * dm::exp10_sum(r[l] - m);
       h.cfg[(size_t)p * K + k] = hm_finish(m, s);
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -120,7 +131,7 @@ __global__ void __launch_bounds__(HM_NT) hm_pair_kernel(const HmDev h) {
     if (isnan(first)) m = NAN;
     double s = 0.0;
     for (int k = lane; k < K; k += 64)
-      if (!isnan(c[k])) s += dw[k] * exp10(c[k] - m);
+      if (!isnan(c[k])) s += dw[k] * dm::exp10_sum(c[k] - m);
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
     if (lane == 0) h.snp[p] = hm_finish(m, s);
     if (h.lik_only) return;
@@ -132,7 +143,7 @@ __global__ void __launch_bounds__(HM_NT) hm_pair_kernel(const HmDev h) {
       double ss = 0.0;
       for (int k = 0; k < K; ++k) {
         const double v = R[(size_t)k * L + l];
-        if (!isnan(v)) ss += dw[k] * exp10(v - mm);
+        if (!isnan(v)) ss += dw[k] * dm::exp10_sum(v - mm);
       }
       h.grd[(size_t)p * L + l] = hm_finish(mm, ss);
     }
@@ -175,7 +186,7 @@ __global__ void __launch_bounds__(HM_NT) hm_pair_kernel(const HmDev h) {
       if (t[k] > mm) mm = t[k];
     double ss = 0.0;
     for (int k = 0; k < HM_TYPES_KMAX && k < K; ++k)
-      if (!isnan(t[k])) ss += dw[k] * exp10(t[k] - mm);
+      if (!isnan(t[k])) ss += dw[k] * dm::exp10_sum(t[k] - mm);
     h.grd[(size_t)p * L + l] = hm_finish(mm, ss);
   }
   /* the SNP's BF over the types */
@@ -186,7 +197,7 @@ __global__ void __launch_bounds__(HM_NT) hm_pair_kernel(const HmDev h) {
       if (c[k] > m) m = c[k];
     double s = 0.0;
     for (int k = 0; k < K; ++k)
-      if (!isnan(c[k])) s += dw[k] * exp10(c[k] - m);
+      if (!isnan(c[k])) s += dw[k] * dm::exp10_sum(c[k] - m);
     h.snp[p] = hm_finish(m, s);
   }
 }
@@ -200,7 +211,7 @@ __device__ inline double hm_lws_seq(const double* v, int n, int stride, const do
   double s = 0.0;
   for (int i = 0; i < n; ++i) {
     const double x = v[i * stride];
-    if (!isnan(x)) s += w[i] * exp10(x - m);
+    if (!isnan(x)) s += w[i] * dm::exp10_sum(x - m);
   }
   return hm_finish(m, s);
 }
@@ -340,14 +351,14 @@ __global__ void __launch_bounds__(HM_NT) __attribute__((amdgpu_waves_per_eu(4, 8
         double s0 = 0.0, s1 = 0.0;
         int l = 0;
         for (; l + 1 < L; l += 2) {
-          const double t0 = exp10(x[l] - M), t1 = exp10(x[l + 1] - M);
+          const double t0 = dm::exp10_sum(x[l] - M), t1 = dm::exp10_sum(x[l + 1] - M);
           x[l] = t0;
           x[l + 1] = t1;
           s0 += wg[l] * t0;
           s1 += wg[l + 1] * t1;
         }
         if (l < L) {
-          const double t0 = exp10(x[l] - M);
+          const double t0 = dm::exp10_sum(x[l] - M);
           x[l] = t0;
           s0 += wg[l] * t0;
         }
@@ -359,7 +370,7 @@ __global__ void __launch_bounds__(HM_NT) __attribute__((amdgpu_waves_per_eu(4, 8
         double sum = 0.0;
         for (int l = 0; l < L; ++l) {
           const double v = x[l];
-          if (!isnan(v)) sum += wg[l] * exp10(v - m);
+          if (!isnan(v)) sum += wg[l] * dm::exp10_sum(v - m);
         }
         c = hm_finish(m, sum);
       }
@@ -418,7 +429,7 @@ __device__ double hm_block_lws(const double* v, int64_t n, int64_t stride, doubl
   double s = 0.0;
   for (int64_t i = tid; i < n; i += HM_NT) {
     const double x = v[i * stride];
-    if (!isnan(x)) s += w * exp10(x - m);
+    if (!isnan(x)) s += w * dm::exp10_sum(x - m);
   }
   for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
   __syncthreads();
@@ -450,8 +461,8 @@ __global__ void __launch_bounds__(HM_NT) hm_gene_kernel(const HmDev h) {
       ol = row[NC];
     } else {
       const double m = gbf > 0.0 ? gbf : 0.0;
-      double s = pi0 * exp10(0.0 - m);
-      if (!isnan(gbf)) s += (1 - pi0) * exp10(gbf - m);
+      double s = pi0 * dm::exp10_sum(0.0 - m);
+      if (!isnan(gbf)) s += (1 - pi0) * dm::exp10_sum(gbf - m);
       ol = hm_finish(m, s);
       row[NC] = ol;
     }
@@ -509,10 +520,10 @@ __global__ void __launch_bounds__(HM_NT) hm_gene_kernel(const HmDev h) {
       int64_t i = wv;
       for (; i + NW < np; i += 2 * NW) {
         const double x0 = v[i * stride], x1 = v[(i + NW) * stride];
-        if (!isnan(x0)) sum += w * exp10(x0 - m);
-        if (!isnan(x1)) sum1 += w * exp10(x1 - m);
+        if (!isnan(x0)) sum += w * dm::exp10_sum(x0 - m);
+        if (!isnan(x1)) sum1 += w * dm::exp10_sum(x1 - m);
       }
-      if (i < np && !isnan(v[i * stride])) sum += w * exp10(v[i * stride] - m);
+      if (i < np && !isnan(v[i * stride])) sum += w * dm::exp10_sum(v[i * stride] - m);
       sum += sum1;
     }
     part[wv][lane] = sum;
@@ -524,6 +535,146 @@ __global__ void __launch_bounds__(HM_NT) hm_gene_kernel(const HmDev h) {
     }
     __syncthreads();
   }
+}
+
+/* ---- configs model: a gene's SNPs summed once ------------------------------
+ * Workgroup b takes the pairs [b ch, (b + 1) ch), thread -> (row group, column
+ * of the K L values), and leaves for each gene g that it meets the running
+ * reference m and the sum of 10^(v - m) per column in part[b + g] (b + g grows
+ * by at least one from a segment to the next, so no two segments share it).
+ * m starts at the segment's first value and is moved, with the sum, when a
+ * value lies 16 decades above it: sums stay below 10^22 and what underflows
+ * is 300 decades below a term that does not.  A value that is not finite
+ * leaves a NaN sum.
+ *
+ * Bound by the one read of the raw ABFs; 18 FP64 instructions a value.  On
+ * 1.5e6 pairs of 31 x 10 values 0.70 ms (5.3 TB/s), after which a pass takes
+ * about 35 us; a pass over the SNPs took 2.0 ms. */
+constexpr int HM_COLL_NT = 512;
+constexpr int HM_COLL_U = 8; /* values in flight per thread */
+
+__global__ void __launch_bounds__(HM_COLL_NT) hm_collapse_kernel(const double* __restrict__ raw,
+                                                                 const int64_t* __restrict__ off, int64_t NP,
+                                                                 int64_t G, int KL, int cols, int ch,
+                                                                 double2* __restrict__ part) {
+  __shared__ double2 red[HM_COLL_NT];
+  const int groups = blockDim.x / cols; /* row groups */
+  const int grp = threadIdx.x / cols, c = threadIdx.x - grp * cols;
+  const int col = blockIdx.y * cols + c;
+  const bool on = grp < groups && col < KL;
+  const int64_t p0 = (int64_t)blockIdx.x * ch, p1 = min(p0 + ch, NP);
+  /* the gene of pair p0: the last one with off <= p0 */
+  int64_t g = 0, hi = G;
+  while (hi - g > 1) {
+    const int64_t mid = (g + hi) >> 1;
+    if (off[mid] <= p0)
+      g = mid;
+    else
+      hi = mid;
+  }
+  for (int64_t at = p0; at < p1 && g < G; ++g) {
+    const int64_t s0 = max(at, off[g]), s1 = min(off[g + 1], p1);
+    if (s1 <= s0) continue;
+    double m = 0.0, s = 0.0, z = 0.0;
+    if (on && s0 + grp < s1) {
+      const double* v = raw + (size_t)(s0 + grp) * KL + col;
+      const size_t step = (size_t)groups * KL;
+      int64_t r = s0 + grp;
+      m = *v;
+      auto move = [&](double top) { /* a new reference, where a value asks for one */
+        if (top > m + 16.0) {
+          s *= dm::exp10_sum(m - top);
+          m = top;
+        }
+      };
+      auto add = [&](double x) {
+        s += dm::exp10_core(fmax(x - m, -400.0));
+        z = fma(0.0, x, z);
+      };
+      for (; r + (HM_COLL_U - 1) * (int64_t)groups < s1; r += HM_COLL_U * (int64_t)groups, v += HM_COLL_U * step) {
+        double x[HM_COLL_U];
+#pragma unroll
+        for (int u = 0; u < HM_COLL_U; ++u) x[u] = v[u * step];
+        double top = x[0];
+#pragma unroll
+        for (int u = 1; u < HM_COLL_U; ++u) top = fmax(top, x[u]);
+        move(top);
+#pragma unroll
+        for (int u = 0; u < HM_COLL_U; ++u) add(x[u]);
+      }
+      for (; r < s1; r += groups, v += step) {
+        const double x = *v;
+        move(x);
+        add(x);
+      }
+      s += z;
+    }
+    if (groups > 1) { /* over the row groups */
+      red[threadIdx.x] = make_double2(m, s);
+      __syncthreads();
+      if (grp == 0 && on)
+        for (int k = 1; k < groups && s0 + k < s1; ++k) {
+          const double2 o = red[k * cols + c];
+          if (o.x > m) {
+            s = s * dm::exp10_sum(m - o.x) + o.y;
+            m = o.x;
+          } else {
+            s += o.y * dm::exp10_sum(o.x - m);
+          }
+        }
+      __syncthreads();
+    }
+    if (grp == 0 && on) part[(size_t)(blockIdx.x + g) * KL + col] = make_double2(m, s);
+    at = s1;
+  }
+}
+
+/* A[k][l] of each gene from its segments, into row g; flag[g] = 1 when a sum
+ * is NaN, and the offsets of one row per gene */
+__global__ void __launch_bounds__(HM_NT) hm_collapse_merge_kernel(const int64_t* __restrict__ off, int64_t G, int KL,
+                                                                  int ch, const double2* __restrict__ part,
+                                                                  double* __restrict__ out, int* __restrict__ flag,
+                                                                  int64_t* __restrict__ off1) {
+  const int64_t g = blockIdx.x, p0 = off[g], p1 = off[g + 1];
+  bool bad = p1 <= p0; /* a gene without SNPs keeps its empty row range */
+  if (p1 > p0) {
+    const int64_t b0 = p0 / ch, b1 = (p1 - 1) / ch;
+    const double lp = log10((double)(p1 - p0));
+    for (int c = threadIdx.x; c < KL; c += HM_NT) {
+      double2 a = part[(size_t)(b0 + g) * KL + c];
+      for (int64_t b = b0 + 1; b <= b1; ++b) {
+        const double2 o = part[(size_t)(b + g) * KL + c];
+        if (o.x > a.x) {
+          a.y = a.y * dm::exp10_sum(a.x - o.x) + o.y;
+          a.x = o.x;
+        } else {
+          a.y += o.y * dm::exp10_sum(o.x - a.x);
+        }
+      }
+      if (!isfinite(a.y) || !isfinite(a.x)) bad = true;
+      out[(size_t)g * KL + c] = a.x + (log10(a.y) - lp);
+    }
+  }
+  const int any = __syncthreads_or(bad);
+  if (threadIdx.x == 0) {
+    flag[g] = any;
+    off1[g] = g;
+    if (g == G - 1) off1[G] = G;
+  }
+}
+
+/* rows of the genes: the pseudo-SNP, or the gene's own SNPs where flagged */
+__global__ void __launch_bounds__(HM_NT) hm_collapse_copy_kernel(const double* __restrict__ raw,
+                                                                 const int64_t* __restrict__ off,
+                                                                 const double* __restrict__ one,
+                                                                 const int* __restrict__ flag,
+                                                                 const int64_t* __restrict__ off1, int KL,
+                                                                 double* __restrict__ out) {
+  const int64_t g = blockIdx.x;
+  const int64_t n = (off1[g + 1] - off1[g]) * KL;
+  const double* src = flag[g] ? raw + (size_t)off[g] * KL : one + (size_t)g * KL;
+  double* dst = out + (size_t)off1[g] * KL;
+  for (int64_t i = threadIdx.x; i < n; i += HM_NT) dst[i] = src[i];
 }
 
 /* over genes: log10 sum of each contribution column (weights 1), the sum
@@ -576,14 +727,99 @@ double h_lws(const double* v, const double* w, size_t n) {
   return std::fabs(r) <= DBL_EPSILON ? 0.0 : r;
 }
 
+/* Rows that the passes run over: every SNP, or the genes' sums */
+struct HmRows {
+  const double* raw = nullptr;
+  const int64_t* off = nullptr;
+  int64_t NP = 0;
+  double *cfg = nullptr, *grd = nullptr, *num = nullptr, *snp = nullptr;
+};
+
 struct HmRun {
   eqbf_ctx* ctx;
   hipStream_t st;
   HmDev h;
+  HmRows snps, sums; /* sums.raw: null when the SNPs were not summed */
   const eqbf_hm_opts* o;
   bool types;
   int NC;
   std::vector<double> hpar, hred;
+
+  /* makes the passes run over `r`; its per-row buffers on first use */
+  int use(HmRows& r, const char* prefix) {
+    if (!r.cfg) {
+      const std::string p(prefix);
+      const size_t n = (size_t)r.NP + 1; /* an empty last gene's first row is looked at */
+      r.cfg = (double*)ctx_buf(ctx, p + "cfg", n * h.K * sizeof(double));
+      r.grd = (double*)ctx_buf(ctx, p + "grd", n * h.L * sizeof(double));
+      r.num = types ? (double*)ctx_buf(ctx, p + "num", n * h.K * h.S * sizeof(double)) : nullptr;
+      r.snp = (double*)ctx_buf(ctx, p + "snp", n * sizeof(double));
+      if (!r.cfg || !r.grd || (types && !r.num) || !r.snp) return EQBF_ERR_HIP;
+    }
+    h.raw = r.raw;
+    h.off = r.off;
+    h.NP = r.NP;
+    h.cfg = r.cfg;
+    h.grd = r.grd;
+    h.num = r.num;
+    h.snp = r.snp;
+    return EQBF_OK;
+  }
+
+  /* Configs model: each gene's SNPs summed into one row (hm_collapse_kernel).
+   * Worth its one read where a gene has two SNPs or more on average: an EM is
+   * at least three passes. */
+  int collapse() {
+    const int64_t NP = snps.NP, G = h.G;
+    if (types || NP < 2 * G) return EQBF_OK;
+    const int KL = h.K * h.L;
+    /* columns a workgroup covers, and the whole waves that hold its row groups */
+    const int ny = (KL + HM_COLL_NT - 1) / HM_COLL_NT, cols = (KL + ny - 1) / ny;
+    const int nt = (std::max(1, HM_COLL_NT / cols) * cols + 63) / 64 * 64;
+    /* about 16 workgroups per CU, none with less than 16 pairs per row group */
+    const int64_t share = (NP * ny + 16 * (int64_t)ctx->n_cu - 1) / (16 * (int64_t)std::max(ctx->n_cu, 1));
+    const int ch = (int)std::min<int64_t>(std::max<int64_t>(share, 16 * (int64_t)(nt / cols)), 1 << 16);
+    const int64_t nb = (NP + ch - 1) / ch;
+    double2* part = (double2*)ctx_buf(ctx, "hm_part", (size_t)(nb + G) * KL * sizeof(double2));
+    double* one = (double*)ctx_buf(ctx, "hm_one", (size_t)G * KL * sizeof(double));
+    int64_t* off1 = (int64_t*)ctx_buf(ctx, "hm_off1", (size_t)(G + 1) * sizeof(int64_t));
+    int* flag = (int*)ctx_buf(ctx, "hm_flag", (size_t)G * sizeof(int));
+    if (!part || !one || !off1 || !flag) return EQBF_ERR_HIP;
+    {
+      ProfScope ps(ctx, "hm_collapse_kernel", st);
+      hipLaunchKernelGGL(hm_collapse_kernel, dim3((unsigned)nb, (unsigned)ny), dim3(nt), 0, st, snps.raw, snps.off, NP,
+                         G, KL, cols, ch, part);
+    }
+    hipLaunchKernelGGL(hm_collapse_merge_kernel, dim3((unsigned)G), dim3(HM_NT), 0, st, snps.off, G, KL, ch, part, one,
+                       flag, off1);
+    EQBF_HIP(ctx, hipGetLastError());
+    std::vector<int> hf(G);
+    EQBF_HIP(ctx, hipMemcpyAsync(hf.data(), flag, G * sizeof(int), hipMemcpyDeviceToHost, st));
+    EQBF_HIP(ctx, hipStreamSynchronize(st));
+    sums.raw = one;
+    sums.off = off1;
+    sums.NP = G;
+    if (std::find(hf.begin(), hf.end(), 1) == hf.end()) return EQBF_OK;
+    /* some genes keep their SNPs */
+    std::vector<int64_t> ho(G + 1), h1(G + 1, 0);
+    EQBF_HIP(ctx, hipMemcpyAsync(ho.data(), snps.off, (G + 1) * sizeof(int64_t), hipMemcpyDeviceToHost, st));
+    EQBF_HIP(ctx, hipStreamSynchronize(st));
+    for (int64_t g = 0; g < G; ++g) h1[g + 1] = h1[g] + (hf[g] ? ho[g + 1] - ho[g] : 1);
+    if (h1[G] > NP - NP / 4) { /* most do: no rows worth keeping */
+      sums = HmRows();
+      return EQBF_OK;
+    }
+    double* rows = (double*)ctx_buf(ctx, "hm_rows1", (size_t)std::max<int64_t>(h1[G], 1) * KL * sizeof(double));
+    if (!rows) return EQBF_ERR_HIP;
+    EQBF_HIP(ctx, hipMemcpyAsync(off1, h1.data(), (G + 1) * sizeof(int64_t), hipMemcpyHostToDevice, st));
+    hipLaunchKernelGGL(hm_collapse_copy_kernel, dim3((unsigned)G), dim3(HM_NT), 0, st, snps.raw, snps.off, one, flag,
+                       off1, KL, rows);
+    EQBF_HIP(ctx, hipGetLastError());
+    EQBF_HIP(ctx, hipStreamSynchronize(st)); /* h1 is read by the copy */
+    sums.raw = rows;
+    sums.NP = h1[G];
+    return EQBF_OK;
+  }
 
   int upload(const HmParams& P) {
     const int K = h.K, L = h.L, S = h.S;
@@ -605,6 +841,8 @@ struct HmRun {
       if (d > 0) lo_d = std::min(lo_d, d);
     }
     h.range = bad ? -1.0 : 290.0 + std::log10(lo_g) + std::log10(lo_d);
+    int rc = use(!bad && sums.raw ? sums : snps, !bad && sums.raw ? "hms_" : "hm_");
+    if (rc) return rc;
     EQBF_HIP(ctx, hipMemcpyAsync((void*)h.par, hpar.data(), hpar.size() * sizeof(double), hipMemcpyHostToDevice, st));
     return EQBF_OK;
   }
@@ -891,9 +1129,9 @@ int hm_setup(eqbf_ctx* ctx, HmRun& R, const double* raw_dev, int64_t n_pairs, co
   R.types = types;
   HmDev& h = R.h;
   memset(&h, 0, sizeof h);
-  h.raw = raw_dev;
-  h.off = off_dev;
-  h.NP = n_pairs;
+  R.snps.raw = raw_dev;
+  R.snps.off = off_dev;
+  R.snps.NP = n_pairs;
   h.G = G;
   h.K = o->dim;
   h.L = o->n_grid;
@@ -909,13 +1147,9 @@ int hm_setup(eqbf_ctx* ctx, HmRun& R, const double* raw_dev, int64_t n_pairs, co
     h.tp = (int)std::min<size_t>(std::min<size_t>(16, room / per), (size_t)(HM_PRE * HM_NT) / (h.K * h.L));
   }
   h.par = (const double*)ctx_buf(ctx, "hm_par", (size_t)(1 + h.L + h.K + h.K * h.S) * sizeof(double));
-  h.cfg = (double*)ctx_buf(ctx, "hm_cfg", (size_t)n_pairs * h.K * sizeof(double));
-  h.grd = (double*)ctx_buf(ctx, "hm_grd", (size_t)n_pairs * h.L * sizeof(double));
-  h.num = types ? (double*)ctx_buf(ctx, "hm_num", (size_t)n_pairs * h.K * h.S * sizeof(double)) : nullptr;
-  h.snp = (double*)ctx_buf(ctx, "hm_snp", (size_t)n_pairs * sizeof(double));
   h.rows = (double*)ctx_buf(ctx, "hm_rows", (size_t)G * (R.NC + 3) * sizeof(double));
   h.red = (double*)ctx_buf(ctx, "hm_red", (size_t)(R.NC + 2) * sizeof(double));
-  if (!h.par || !h.cfg || !h.grd || (types && !h.num) || !h.snp || !h.rows || !h.red) return EQBF_ERR_HIP;
+  if (!h.par || !h.rows || !h.red) return EQBF_ERR_HIP;
   return EQBF_OK;
 }
 
@@ -948,6 +1182,7 @@ int hm_em_run(eqbf_ctx* ctx, const double* raw_dev, int64_t n_pairs, const int64
   int rc = hm_setup(ctx, R, raw_dev, n_pairs, off_dev, G, o, st);
   if (rc) return rc;
   if ((rc = hm_check_params(ctx, o, p))) return rc;
+  if ((rc = R.collapse())) return rc;
   HmParams P;
   hm_load(o, p, P);
   double l = NAN;
@@ -1150,6 +1385,7 @@ extern "C" int eqbf_hm_ci(eqbf_ctx* ctx, const double* raw, int64_t n_pairs, con
   if ((rc = hm_upload(ctx, raw, n_pairs, gene_offset, n_genes, opts, &d_raw, &d_off))) return rc;
   HmRun R;
   if ((rc = hm_setup(ctx, R, d_raw, n_pairs, d_off, n_genes, opts, ctx->stream))) return rc;
+  if ((rc = R.collapse())) return rc;
   HmParams P;
   hm_load(opts, params, P);
   return hm_ci(R, P, left, right);

@@ -275,6 +275,31 @@ __device__ inline double tz_eval(const double* __restrict__ tz, int nu, double a
   return h00 * w0 + h10 * d0 + h01 * w1 + h11 * d1;
 }
 
+/* 10^x for -400 <= x <= 308 (0 below 10^-324; NaN stays NaN): 2^k 2^f with k
+ * the nearest integer of x log2 10, taken from the low bits of the sum with
+ * 1.5 2^52, and f good to 2^-53 of its own size through log2 10 in two parts;
+ * 2^f = 1 + f q(f), q the interpolant of (2^f - 1)/f at 11 Chebyshev nodes on
+ * [-1/2, 1/2] (2.0e-17 relative). */
+__device__ __forceinline__ double exp10_core(double x) {
+  const double t = fma(x, 0x1.a934f0979a371p+1, 0x1.8p52);
+  const double k = t - 0x1.8p52;
+  const double f = fma(x, 0x1.7f2495fb7fa6dp-53, fma(x, 0x1.a934f0979a371p+1, -k));
+  double q = fma(0x1.e9d3fe3952179p-32, f, 0x1.e6063f7217bc6p-28);
+  q = fma(q, f, 0x1.b524fae627834p-24);
+  q = fma(q, f, 0x1.62bfd47773353p-20);
+  q = fma(q, f, 0x1.ffcbfc670dcd4p-17);
+  q = fma(q, f, 0x1.430913096fd9fp-13);
+  q = fma(q, f, 0x1.5d87fe78a5276p-10);
+  q = fma(q, f, 0x1.3b2ab6fba1ddap-7);
+  q = fma(q, f, 0x1.c6b08d704a0c2p-5);
+  q = fma(q, f, 0x1.ebfbdff82c598p-3);
+  q = fma(q, f, 0x1.62e42fefa39efp-1);
+  return __builtin_amdgcn_ldexp(fma(q, f, 1.0), __double2loint(t));
+}
+
+/* 10^x for any x <= 308, -inf and NaN included: the terms of a log10 sum */
+__device__ __forceinline__ double exp10_sum(double x) { return exp10_core(x < -400.0 ? -400.0 : x); }
+
 }  // namespace dm
 
 /* Index of raw ABF (row, p) of n_raw rows and NP pairs: [n_raw][NP], or in

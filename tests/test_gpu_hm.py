@@ -188,3 +188,25 @@ def test_hm_wide_ranges_and_tiny_weights_vs_oracle(eng, orc):
         fin = np.isfinite(b)
         assert np.array_equal(np.isfinite(a), fin)
         assert np.max(np.abs(a[fin] - b[fin]), initial=0) <= 1e-10
+
+
+@pytest.mark.parametrize("K,L,G,pmax,odd", [
+    (1, 1, 7, 900, None), (3, 25, 40, 60, None), (31, 10, 30, 90, None), (40, 20, 6, 70, None),
+    (31, 10, 30, 90, "nan"), (3, 5, 12, 40, "inf"), (5, 4, 20, 30, "rising"),
+])
+def test_hm_gene_sums_vs_oracle(eng, orc, K, L, G, pmax, odd):
+    """Configs model with each gene's SNPs summed once: row groups and column
+    blocks of every width, genes over several workgroups, genes that keep
+    their SNPs (a NaN or -inf among finite ones) next to summed ones, and
+    values that climb by hundreds of decades."""
+    raw, off = _case(77 + K, G, K, L, pmin=1, pmax=pmax)
+    if odd == "nan":
+        raw[off[3] + 1, 1, 2] = np.nan
+        raw[off[9], K - 1, 1] = np.nan
+    elif odd == "inf":
+        raw[off[2], 1, 1] = -np.inf
+    elif odd == "rising":
+        for g in range(G):
+            raw[off[g]:off[g + 1]] += np.linspace(-200, 60, off[g + 1] - off[g])[:, None, None]
+    prm = orc.HmParams(0.5, np.full(L, 1 / L), cfg=np.full(K, 1 / K))
+    _em_both(eng, orc, raw, off, prm, thresh=1e-3, maxit=6)
