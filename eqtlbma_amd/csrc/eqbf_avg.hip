@@ -19,6 +19,9 @@
  *                    SNP BF over them and the first strict maximum; then,
  *                    when asked, post_dim and its argmax (:683-718) and the
  *                    configs model's subgroup posteriors (:722-745)
+ *   avg_rows_kernel  the same for the configs model where every grid point is
+ *                    kept and a row fits a lane's registers (at most 16
+ *                    points, 64 configurations)
  *   avg_gene_kernel  one wave per gene, lanes over its SNPs: the gene BF
  *                    (Gene::avg_raw_bfs, :598-622), gene_post (:634-643),
  *                    post_the (:647-662), post_an (:664-680)
@@ -66,6 +69,7 @@ struct AvgArgs {
   double pi0;
   int64_t NP, G;
   int D, S, L, nk, types, want;
+  double gw_row[16]; /* the grid weights as kernel arguments, where L fits and every point is kept */
 };
 
 /* sum over the subgroups of log10(q 10^x + 1 - q) at kept grid point i,
@@ -114,34 +118,91 @@ __global__ void __launch_bounds__(256) avg_grid_kernel(const double* __restrict_
   out[r] = l10_round(mx + log10(sum));
 }
 
-/* reductions over the aligned group of w lanes (w a power of two <= 64) */
-__device__ inline double gmax(double v, int w) {
-  for (int o = w >> 1; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
+/* Value of the lane that a step of a butterfly over aligned groups pairs this
+ * one with: within 16 lanes by data-parallel moves (quads by permutation, the
+ * halves mirrored, which pairs equal partial results), 16 and 32 apart through
+ * LDS. */
+template <int STEP>
+__device__ __forceinline__ int partner(int v) {
+  if (STEP == 1) return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, true);  /* quad [1,0,3,2] */
+  if (STEP == 2) return __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, true);  /* quad [2,3,0,1] */
+  if (STEP == 4) return __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, true); /* 8 lanes mirrored */
+  if (STEP == 8) return __builtin_amdgcn_update_dpp(0, v, 0x140, 0xF, 0xF, true); /* 16 lanes mirrored */
+  return __shfl_xor(v, STEP, 64);
+}
+template <int STEP>
+__device__ __forceinline__ double partner(double v) {
+  return __hiloint2double(partner<STEP>(__double2hiint(v)), partner<STEP>(__double2loint(v)));
+}
+/* reduction over the aligned group of w lanes (w a power of two <= 64), the
+ * result in every lane */
+template <class T, class F>
+__device__ __forceinline__ T greduce(T v, int w, F f) {
+  if (w > 1) v = f(v, partner<1>(v));
+  if (w > 2) v = f(v, partner<2>(v));
+  if (w > 4) v = f(v, partner<4>(v));
+  if (w > 8) v = f(v, partner<8>(v));
+  if (w > 16) v = f(v, partner<16>(v));
+  if (w > 32) v = f(v, partner<32>(v));
   return v;
 }
-__device__ inline double gsum(double v, int w) {
-  for (int o = w >> 1; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+__device__ __forceinline__ double gmax(double v, int w) {
+  return greduce(v, w, [](double a, double b) { return fmax(a, b); });
+}
+__device__ __forceinline__ double gsum(double v, int w) {
+  return greduce(v, w, [](double a, double b) { return a + b; });
 }
 
 /* first index of the strict maximum scanning from index 0 (the reference's
- * "j == 0 || v[j] > v[best]"): v0 is the first value, (lmax, larg) the
- * lane's largest value and its first index (larg = n when it has none) */
-__device__ inline int first_max(double v0, double lmax, int larg, int n, int w) {
-  const double mx = gmax(lmax, w);
-  int cand = (larg < n && lmax == mx) ? larg : n;
-  for (int o = w >> 1; o > 0; o >>= 1) cand = min(cand, __shfl_xor(cand, o, 64));
+ * "j == 0 || v[j] > v[best]"): v0 is the first value, mx the group's largest,
+ * (lmax, larg) the lane's largest value and its first index (larg = n when it
+ * has none) */
+__device__ __forceinline__ int first_max(double v0, double mx, double lmax, int larg, int n, int w) {
+  const int cand = greduce((larg < n && lmax == mx) ? larg : n, w, [](int a, int b) { return min(a, b); });
   if (isnan(v0) || !(mx > v0)) return 0;
   return cand >= n ? 0 : cand;
 }
 
 constexpr int kAvgWaves = 4;
+constexpr int kAvgRow = 16; /* longest row that a lane holds in registers (AvgArgs::gw_row) */
+
+/* log10 sum_i w_i 10^r_i over a row of LV values that all are kept: the row in
+ * registers, 16-byte loads where VEC; a row with a value that is not finite
+ * goes through the general form */
+template <int LV, bool VEC>
+__device__ __forceinline__ double row_lws(const AvgArgs& a, const double* __restrict__ r) {
+  double x[LV];
+  if (VEC) {
+#pragma unroll
+    for (int i = 0; i + 1 < LV; i += 2) {
+      const double2 t = *reinterpret_cast<const double2*>(r + i);
+      x[i] = t.x;
+      x[i + 1] = t.y;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < LV; ++i) x[i] = r[i];
+  }
+  double mx = x[0], z = 0.0;
+#pragma unroll
+  for (int i = 0; i < LV; ++i) {
+    mx = fmax(mx, x[i]);
+    z = fma(0.0, x[i], z);
+  }
+  if (__builtin_expect(isnan(z), 0)) return grid_lws(a, [&](int i) { return r[i]; });
+  double sum = 0.0;
+#pragma unroll
+  for (int i = 0; i < LV; ++i) sum = fma(a.gw_row[i], dm::exp10_core(fmax(x[i] - mx, -400.0)), sum);
+  return l10_round(mx + log10(sum));
+}
 
 /* A group of w lanes per pair (w = the power of two >= dim, at most 64:
  * 64 / w pairs a wave), four waves a block striding over the pairs; lanes
  * over the dimensions.  Also writes post_dim, its best dimension and the
  * configs model's subgroup posteriors when asked: they need only the pair's
- * own values. */
+ * own values, and the posterior of a dimension is its term of the SNP's sum
+ * over that sum.  The general form: any number of dimensions, kept points and
+ * row lengths, both models. */
 __global__ void __launch_bounds__(64 * kAvgWaves) avg_pair_kernel(const AvgArgs a, int w) {
   const int lane = threadIdx.x & 63;
   const int gl = lane & (w - 1), g0 = lane - gl; /* lane in the group, group's first lane */
@@ -149,6 +210,9 @@ __global__ void __launch_bounds__(64 * kAvgWaves) avg_pair_kernel(const AvgArgs 
   const int D = a.D;
   const bool dims_post = (a.want & 16) || (!a.types && (a.want & 8));
   const bool sub_post = !a.types && (a.want & 8);
+  /* the lane's first dimension: its weight and subgroups stay in registers */
+  const double dw0 = gl < D ? a.dw[gl] : 0.0;
+  const uint64_t cs0 = sub_post && gl < D ? a.cs[gl] : 0;
   const int64_t step = (int64_t)gridDim.x * kAvgWaves * per_wave;
   for (int64_t pb = ((int64_t)blockIdx.x * kAvgWaves + (threadIdx.x >> 6)) * per_wave; pb < a.NP; pb += step) {
     const int64_t p = pb + lane / w;
@@ -174,25 +238,29 @@ __global__ void __launch_bounds__(64 * kAvgWaves) avg_pair_kernel(const AvgArgs 
     }
     const double d0 = __shfl(dk, g0, 64); /* the group's first lane holds dims[0] */
     /* maximum as the reference scans it: from the first value, strict > */
-    double mx = gmax(lmax, w);
+    const double top = gmax(lmax, w);
+    double mx = top;
     if (isnan(d0)) mx = NAN;
     if (!(mx > d0)) mx = d0;
-    const int best0 = first_max(d0, lmax, larg, D, w);
-    double sum = 0.0;
+    int best = a.types ? -1 : first_max(d0, top, lmax, larg, D, w);
+    /* the terms w_k 10^(d_k - mx) of the SNP's sum, the first one kept */
+    double sum = 0.0, tk = 0.0;
     for (int k = gl; on && k < D; k += w) {
       const double d = (k == gl) ? dk : dims[k];
-      if (!isnan(d)) sum += a.dw[k] * exp10(d - mx);
+      const double t = ((k == gl) ? dw0 : a.dw[k]) * dm::exp10_sum(d - mx);
+      if (k == gl) tk = t;
+      if (!isnan(d)) sum += t;
     }
     sum = gsum(sum, w);
     const double sbp = l10_round(mx + log10(sum));
-    int best = a.types ? -1 : best0;
     if (dims_post) {
       double* pd = a.post_dim + (size_t)p * D;
       double pmax = -INFINITY, pk = NAN;
       int parg = D;
       for (int k = gl; on && k < D; k += w) {
-        const double d = (k == gl) ? dk : dims[k];
-        double v = exp10(log10(a.dw[k]) + d - sbp);
+        const double wk = (k == gl) ? dw0 : a.dw[k];
+        const double t = (k == gl) ? tk : wk * dm::exp10_sum(dims[k] - mx);
+        double v = wk >= 0.0 ? t / sum : NAN; /* the reference takes the weight's logarithm */
         if (v > 1.0) v = 1.0;
         pd[k] = v;
         if (k == gl) pk = v;
@@ -201,12 +269,12 @@ __global__ void __launch_bounds__(64 * kAvgWaves) avg_pair_kernel(const AvgArgs 
           parg = k;
         }
       }
-      best = first_max(__shfl(pk, g0, 64), pmax, parg, D, w);
+      best = first_max(__shfl(pk, g0, 64), gmax(pmax, w), pmax, parg, D, w);
       if (sub_post) {
         for (int s = 0; s < a.S; ++s) {
           double acc = 0.0;
           for (int k = gl; on && k < D; k += w)
-            if ((a.cs[k] >> s) & 1ull) acc += (k == gl) ? pk : pd[k];
+            if ((((k == gl) ? cs0 : a.cs[k]) >> s) & 1ull) acc += (k == gl) ? pk : pd[k];
           acc = gsum(acc, w);
           if (on && gl == 0) a.post_sub[(size_t)p * a.S + s] = acc > 1.0 ? 1.0 : acc;
         }
@@ -217,6 +285,97 @@ __global__ void __launch_bounds__(64 * kAvgWaves) avg_pair_kernel(const AvgArgs 
       a.best_dim[p] = best;
     }
   }
+}
+
+/* Configs model with at most 64 dimensions and rows of LV values that are all
+ * kept: a wave takes n_it passes of 64 / w pairs, one lane per row.
+ *
+ * Bound by the FP64 instructions (11 exponentials and a logarithm per row and
+ * six reductions over the lanes of a pair) next to the one read of the raw
+ * values.  So a row is held in registers (16-byte loads where VEC), the SNP's
+ * logarithms wait in LDS until the wave has one for each of its lanes, and a
+ * posterior is its term over the sum instead of a logarithm and an exponential
+ * of its own.  On 9.0e5 pairs of 31 x 10 values with every posterior 0.67 ms
+ * (4.1 TB/s); the general form took 2.0 ms. */
+template <int LV, bool VEC>
+__global__ void __launch_bounds__(64 * kAvgWaves) __attribute__((amdgpu_waves_per_eu(4, 8)))
+avg_rows_kernel(const AvgArgs a, int w, int n_it) {
+  __shared__ double2 held[kAvgWaves][64]; /* maximum and sum of each pair of the wave */
+  __shared__ int hbest[kAvgWaves][64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int gl = lane & (w - 1), grp = lane / w, g0 = lane - gl;
+  const int per_wave = 64 / w, D = a.D;
+  const bool dims_post = a.want & (16 | 8), sub_post = a.want & 8;
+  const bool in = gl < D;
+  const double dw0 = in ? a.dw[gl] : 0.0;
+  const uint64_t cs0 = sub_post && in ? a.cs[gl] : 0;
+  const int64_t base = ((int64_t)blockIdx.x * kAvgWaves + wv) * (n_it * per_wave);
+  const int n_pairs = (int)min((int64_t)n_it * per_wave, max(a.NP - base, (int64_t)0));
+  for (int q = grp; q - grp < n_pairs; q += per_wave) {
+    const int64_t p = base + q;
+    const bool on = q < n_pairs && in; /* every lane takes part in the reductions */
+    double d = NAN;
+    if (on) {
+      d = row_lws<LV, VEC>(a, a.raw + ((size_t)p * D + gl) * LV);
+      a.dim_bf[(size_t)p * D + gl] = d;
+    }
+    const double d0 = __shfl(d, g0, 64);
+    /* maximum as the reference scans it: from the first value, strict > */
+    const double lmax = d > -INFINITY ? d : -INFINITY, top = gmax(lmax, w);
+    double mx = top;
+    if (isnan(d0)) mx = NAN;
+    if (!(mx > d0)) mx = d0;
+    const double t = dw0 * dm::exp10_sum(d - mx);
+    const double sum = gsum(isnan(d) ? 0.0 : t, w);
+    int best;
+    if (dims_post) {
+      double v = dw0 >= 0.0 ? t / sum : NAN; /* the reference takes the weight's logarithm */
+      if (v > 1.0) v = 1.0;
+      if (on) a.post_dim[(size_t)p * D + gl] = v;
+      const double pmax = v > -INFINITY && on ? v : -INFINITY;
+      best = first_max(__shfl(v, g0, 64), gmax(pmax, w), pmax, v > -INFINITY && on ? gl : D, D, w);
+      if (sub_post) {
+        /* lane s of the group keeps subgroup s */
+        double mine = 0.0;
+        for (int s = 0; s < a.S; ++s) {
+          const double acc = gsum(((cs0 >> s) & 1ull) ? v : 0.0, w);
+          if (w >= a.S) {
+            if (gl == s) mine = acc;
+          } else if (gl == 0 && q < n_pairs) {
+            a.post_sub[(size_t)p * a.S + s] = acc > 1.0 ? 1.0 : acc;
+          }
+        }
+        if (w >= a.S && gl < a.S && q < n_pairs) a.post_sub[(size_t)p * a.S + gl] = mine > 1.0 ? 1.0 : mine;
+      }
+    } else {
+      best = first_max(d0, top, lmax, d > -INFINITY ? gl : D, D, w);
+    }
+    if (gl == 0 && q < n_pairs) {
+      held[wv][q] = make_double2(mx, sum);
+      hbest[wv][q] = best;
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  if (lane < n_pairs) {
+    const double2 h = held[wv][lane];
+    a.snp_bf[base + lane] = l10_round(h.x + log10(h.y));
+    a.best_dim[base + lane] = hbest[wv][lane];
+  }
+}
+
+/* launch of the instance for rows of L values, LV counted down to it */
+template <int LV>
+void launch_avg_rows(const AvgArgs& a, int w, int n_it, hipStream_t st) {
+  if constexpr (LV > 1)
+    if (a.L != LV) return launch_avg_rows<LV - 1>(a, w, n_it, st);
+  const int64_t per_block = (int64_t)kAvgWaves * n_it * (64 / w);
+  const dim3 grid((unsigned)((a.NP + per_block - 1) / per_block)), block(64 * kAvgWaves);
+  if (LV % 2 == 0 && ((uintptr_t)a.raw & 15) == 0)
+    hipLaunchKernelGGL((avg_rows_kernel<LV, LV % 2 == 0>), grid, block, 0, st, a, w, n_it);
+  else
+    hipLaunchKernelGGL((avg_rows_kernel<LV, false>), grid, block, 0, st, a, w, n_it);
 }
 
 __global__ void __launch_bounds__(64) avg_gene_kernel(const AvgArgs a) {
@@ -333,6 +492,10 @@ int avg_bfs_run(eqbf_ctx* ctx, const double* raw, int64_t NP, const int64_t* off
   a.nk = o->n_keep;
   a.types = o->model == EQBF_AVG_TYPES;
   a.want = o->want;
+  /* rows that are kept whole and fit a lane's registers */
+  bool rows = !a.types && a.D <= 64 && a.L <= kAvgRow && a.nk == a.L;
+  for (int i = 0; i < a.nk && rows; ++i) rows = o->keep[i] == i;
+  for (int i = 0; i < a.L && rows; ++i) a.gw_row[i] = o->grid_weights[i];
   /* lanes per pair: the power of two >= dim, at most 64; enough blocks to
    * fill every CU several times over, each wave then strides over the pairs */
   int w = 1;
@@ -341,7 +504,16 @@ int avg_bfs_run(eqbf_ctx* ctx, const double* raw, int64_t NP, const int64_t* off
   const unsigned pblocks = (unsigned)std::min<int64_t>((NP + per_block - 1) / per_block, (int64_t)256 * 64);
   if (NP > 0) {
     ProfScope ps(ctx, "avg_pair_kernel", st);
-    hipLaunchKernelGGL(avg_pair_kernel, dim3(pblocks), dim3(64 * kAvgWaves), 0, st, a, w);
+    if (rows) {
+      /* passes per wave: as many as give every lane a pair, fewer while that
+       * leaves compute units without a workgroup */
+      const int64_t passes = (NP + 64 / w - 1) / (64 / w);
+      const int n_it = (int)std::max<int64_t>(
+          1, std::min<int64_t>(w, passes / ((int64_t)kAvgWaves * 4 * std::max(ctx->n_cu, 1))));
+      launch_avg_rows<kAvgRow>(a, w, n_it, st);
+    } else {
+      hipLaunchKernelGGL(avg_pair_kernel, dim3(pblocks), dim3(64 * kAvgWaves), 0, st, a, w);
+    }
   }
   if (G > 0) {
     ProfScope ps(ctx, "avg_gene_kernel", st);
@@ -395,21 +567,26 @@ struct AvgTables {
   uint64_t* cs = nullptr;
 };
 
-int avg_tables(eqbf_ctx* ctx, const eqbf_avg_opts* o, AvgTables& t, hipStream_t st) {
-  const int D = o->dim, S = o->n_subgroups;
-  t.gw = (double*)ctx_buf(ctx, "avg_gw", (size_t)o->n_grid * sizeof(double));
-  t.dw = (double*)ctx_buf(ctx, "avg_dw", (size_t)D * sizeof(double));
-  t.keep = (int32_t*)ctx_buf(ctx, "avg_keep", (size_t)o->n_keep * sizeof(int32_t));
-  t.cs = (uint64_t*)ctx_buf(ctx, "avg_cs", (size_t)D * sizeof(uint64_t));
-  t.sw = (double*)ctx_buf(ctx, "avg_sw", (size_t)D * std::max(S, 1) * sizeof(double));
-  if (!t.gw || !t.dw || !t.keep || !t.cs || !t.sw) return ctx_fail(ctx, EQBF_ERR_HIP, "allocating tables failed");
-  EQBF_HIP(ctx, hipMemcpyAsync(t.gw, o->grid_weights, (size_t)o->n_grid * sizeof(double), hipMemcpyHostToDevice, st));
-  EQBF_HIP(ctx, hipMemcpyAsync(t.dw, o->dim_weights, (size_t)D * sizeof(double), hipMemcpyHostToDevice, st));
-  EQBF_HIP(ctx, hipMemcpyAsync(t.keep, o->keep, (size_t)o->n_keep * sizeof(int32_t), hipMemcpyHostToDevice, st));
-  if (o->cfg_subgroups)
-    EQBF_HIP(ctx, hipMemcpyAsync(t.cs, o->cfg_subgroups, (size_t)D * sizeof(uint64_t), hipMemcpyHostToDevice, st));
-  if (o->sub_weights && S > 0)
-    EQBF_HIP(ctx, hipMemcpyAsync(t.sw, o->sub_weights, (size_t)D * S * sizeof(double), hipMemcpyHostToDevice, st));
+/* in one buffer and one copy (each small copy costs a few microseconds); `host`
+ * has to live until the stream has made it */
+int avg_tables(eqbf_ctx* ctx, const eqbf_avg_opts* o, AvgTables& t, std::vector<uint64_t>& host, hipStream_t st) {
+  const size_t D = o->dim, S = std::max(o->n_subgroups, 0), L = o->n_grid, nk = o->n_keep;
+  const size_t sw = o->sub_weights ? D * S : 0, cs = o->cfg_subgroups ? D : 0;
+  host.resize(L + D + cs + sw + (nk + 1) / 2);
+  uint64_t* h = host.data();
+  memcpy(h, o->grid_weights, L * sizeof(double));
+  memcpy(h + L, o->dim_weights, D * sizeof(double));
+  if (cs) memcpy(h + L + D, o->cfg_subgroups, D * sizeof(uint64_t));
+  if (sw) memcpy(h + L + D + cs, o->sub_weights, sw * sizeof(double));
+  memcpy(h + L + D + cs + sw, o->keep, nk * sizeof(int32_t));
+  uint64_t* d = (uint64_t*)ctx_buf(ctx, "avg_tables", host.size() * sizeof(uint64_t));
+  if (!d) return ctx_fail(ctx, EQBF_ERR_HIP, "allocating tables failed");
+  t.gw = (double*)d;
+  t.dw = (double*)(d + L);
+  t.cs = d + L + D;
+  t.sw = (double*)(d + L + D + cs);
+  t.keep = (int32_t*)(d + L + D + cs + sw);
+  EQBF_HIP(ctx, hipMemcpyAsync(d, h, host.size() * sizeof(uint64_t), hipMemcpyHostToDevice, st));
   return EQBF_OK;
 }
 
@@ -431,7 +608,8 @@ extern "C" int eqbf_avg_bfs_device(eqbf_ctx* ctx, const double* raw, int64_t NP,
   EQBF_HIP(ctx, hipSetDevice(ctx->device));
   hipStream_t st = stream ? (hipStream_t)stream : ctx->stream;
   AvgTables t;
-  if ((rc = avg_tables(ctx, o, t, st))) return rc;
+  std::vector<uint64_t> tables;
+  if ((rc = avg_tables(ctx, o, t, tables, st))) return rc;
   rc = avg_bfs_run(ctx, raw, NP, off, G, o, t.gw, t.keep, t.dw, t.cs, t.sw, out, st);
   if (rc) return rc;
   /* the host tables must outlive the copies */
@@ -469,7 +647,8 @@ extern "C" int eqbf_avg_bfs(eqbf_ctx* ctx, const double* raw, int64_t NP, const 
     EQBF_HIP(ctx, hipMemcpyAsync(d_raw, raw, (size_t)NP * R * o->n_grid * sizeof(double), hipMemcpyHostToDevice, st));
   EQBF_HIP(ctx, hipMemcpyAsync(d_off, off, (size_t)(G + 1) * sizeof(int64_t), hipMemcpyHostToDevice, st));
   AvgTables t;
-  if ((rc = avg_tables(ctx, o, t, st))) return rc;
+  std::vector<uint64_t> tables;
+  if ((rc = avg_tables(ctx, o, t, tables, st))) return rc;
   rc = avg_bfs_run(ctx, d_raw, NP, d_off, G, o, t.gw, t.keep, t.dw, t.cs, t.sw, &d, st);
   if (rc) return rc;
   auto back = [&](void* h, const void* dv, size_t bytes) -> int {

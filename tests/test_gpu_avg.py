@@ -115,3 +115,32 @@ def test_avg_types_all_posteriors(eng, orc):
     ref = orc.avg_bfs(raw, off, gw, **kw)
     _cmp(got, ref, ["dim_bf", "snp_bf", "gene_bf", "gene_post", "post_the", "post_an", "post_dim", "post_sub",
                     "best_dim"])
+
+
+@pytest.mark.parametrize("D,L,S,want", [
+    (1, 1, 1, "abcd"), (2, 2, 3, "abcd"), (3, 7, 2, ""), (5, 16, 4, "abcd"), (31, 10, 5, "abcd"), (31, 11, 5, "ac"),
+    (33, 3, 6, "abcd"), (64, 5, 6, "abcd"), (65, 10, 6, "abcd"), (7, 17, 3, "abcd"),
+])
+def test_avg_configs_rows_in_registers(eng, orc, D, L, S, want):
+    """Every point kept: rows that a lane holds whole (up to 16 values, 64
+    dimensions) and the sizes just past that; NaN first and other values,
+    -inf, wide ranges, a zero weight, more subgroups than dimensions."""
+    rng = np.random.default_rng(D * 100 + L)
+    off = _genes(rng, 30, 1, 40)
+    NP = int(off[-1])
+    raw = rng.normal(-0.4, 0.7, (NP, D, L))
+    raw[rng.choice(NP, 5, replace=False)] += rng.uniform(1, 150, (5, D, 1))
+    raw[rng.random(raw.shape) < 0.01] = np.nan
+    raw[3, 0, 0] = np.nan
+    raw[4, D - 1, L - 1] = -np.inf
+    raw[6, 0, :] = -0.3  # a tie between dimensions
+    cw = rng.dirichlet(np.ones(D))
+    if D > 2:
+        cw[1] = 0.0
+    kw = dict(cfg_w=cw, cfg_sub=rng.integers(1, 1 << S, D).astype(np.uint64), pi0=0.3,
+              want=tuple(want) + (("dims",) if "d" in want else ()), n_subgroups=S)
+    gw = rng.dirichlet(np.ones(L))
+    got, ref = eng.avg_bfs(raw, off, gw, **kw), orc.avg_bfs(raw, off, gw, **kw)
+    keys = ["dim_bf", "snp_bf", "gene_bf", "best_dim"]
+    keys += [k for w, k in zip("abc", ("gene_post", "post_the", "post_an")) if w in want]
+    _cmp(got, ref, keys + (["post_dim", "post_sub"] if "d" in want else []))
