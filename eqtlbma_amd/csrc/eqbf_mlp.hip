@@ -9,11 +9,11 @@
  * x Phi(x).  Gradients with respect to the BF16 weights are applied to the
  * master copy (straight-through).
  *
- * Kernels: one tiled product C = A . B (64 x 64 tile per 256-thread
- * workgroup, 4 x 4 outputs per thread, 16-deep LDS stages) with three
- * epilogues -- forward (bias, pre-activation and GELU stored), backward
+ * Kernels: one tiled product C = A . B on the FP32 matrix instructions with
+ * three epilogues -- forward (bias, pre-activation and GELU stored), backward
  * through the weights (times GELU'(z) of the layer below), and the weight
- * gradient -- plus bias-gradient, loss and Adam kernels.
+ * gradient, whose sum over the batch is split over workgroups (with the bias
+ * gradient as A's row sums) and then added up -- plus loss and Adam kernels.
  */
 #include <algorithm>
 #include <cmath>
@@ -38,6 +38,7 @@ struct eqbf_mlp {
   std::vector<float*> z, h; /* per layer: pre-activation, output          */
   float* dz0 = nullptr;     /* two gradient buffers of the widest layer    */
   float* dz1 = nullptr;
+  float* part = nullptr;    /* weight-gradient partial products            */
   float* xin = nullptr;     /* batch inputs, targets, loss scalar          */
   float* tgt = nullptr;
   float* wout = nullptr;
@@ -69,56 +70,84 @@ __device__ inline float ld<float>(const float* p, int64_t i) { return p[i]; }
 template <>
 __device__ inline float ld<uint16_t>(const uint16_t* p, int64_t i) { return bf16_to_f32(p[i]); }
 
-enum { EPI_FWD = 0, EPI_FWD_LINEAR = 1, EPI_BWD_DATA = 2, EPI_STORE = 3 };
+enum { EPI_FWD = 0, EPI_FWD_LINEAR = 1, EPI_BWD_DATA = 2, EPI_SPLIT = 3 };
 
-/* C[m][n] = sum_k A(m, k) B(k, n), A(m, k) = A[m*sam + k*sak], B(k, n) = B[k*sbk + n*sbn]. */
-template <typename TA, typename TB, int EPI>
-__global__ void __launch_bounds__(256) mlp_gemm_kernel(const TA* __restrict__ A, int64_t sam, int64_t sak,
-                                                       const TB* __restrict__ B, int64_t sbk, int64_t sbn, int M,
-                                                       int N, int K, const float* __restrict__ bias,
+/* C[m][n] = sum_k A(m, k) B(k, n) over the k of split blockIdx.z (all of them
+ * but for EPI_SPLIT, whose partial products go to C[z][M][N] and the row sums
+ * of A to C2[z][M]).  AK: A[m * lda + k], else A[k * lda + m]; BK: B[n * ldb +
+ * k], else B[k * ldb + n] -- consecutive threads load along the contiguous one.
+ *
+ * 32 x 64 outputs a workgroup, so that a batch of 2,000 rows over 256 units is
+ * 252 workgroups; 64 k a stage through LDS, the next stage's loads in
+ * registers meanwhile; FP32 matrix instructions (products and sums as an FP32
+ * multiply-add makes them), each wave 16 x 32.  2,000 rows, 256 to 256 units:
+ * forward 10 us (33), weight gradient with its bias 16 us (353 and 356 as one
+ * thread's sum over the rows). */
+constexpr int MLP_TM = 32, MLP_TN = 64, MLP_TK = 64;
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+template <typename TA, typename TB, bool AK, bool BK, int EPI>
+__global__ void __launch_bounds__(256) mlp_gemm_kernel(const TA* __restrict__ A, int64_t lda,
+                                                       const TB* __restrict__ B, int64_t ldb, int M, int N, int K,
+                                                       int ksplit, const float* __restrict__ bias,
                                                        float* __restrict__ C, float* __restrict__ C2,
                                                        const float* __restrict__ zprev) {
-  __shared__ float As[16][64 + 1];
-  __shared__ float Bs[16][64 + 1];
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-  float acc[4][4];
+  __shared__ float As[MLP_TK][MLP_TM + 1];
+  __shared__ float Bs[MLP_TK][MLP_TN + 1];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int m0 = blockIdx.x * MLP_TM, n0 = blockIdx.y * MLP_TN;
+  const int kb = blockIdx.z * ksplit, ke = min(K, kb + ksplit);
+  /* element i of the thread: k and row (column) of the stage's tiles */
+  auto ak = [&](int i) { return AK ? (tid & 63) : (tid >> 5) + 8 * i; };
+  auto am = [&](int i) { return AK ? (tid >> 6) + 4 * i : (tid & 31); };
+  auto bk = [&](int i) { return BK ? (tid & 63) : (tid >> 6) + 4 * i; };
+  auto bn = [&](int i) { return BK ? (tid >> 6) + 4 * i : (tid & 63); };
+  float ra[8], rb[16];
+  auto fetch = [&](int k0) { /* indexes held inside, so that the loads need no branches */
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    for (int e = threadIdx.x; e < 16 * 64; e += 256) {
-      const int kk = e >> 6, r = e & 63;
-      const int m = m0 + r, k = k0 + kk, n = n0 + r;
-      As[kk][r] = (m < M && k < K) ? ld<TA>(A, (int64_t)m * sam + (int64_t)k * sak) : 0.f;
-      Bs[kk][r] = (n < N && k < K) ? ld<TB>(B, (int64_t)k * sbk + (int64_t)n * sbn) : 0.f;
+    for (int i = 0; i < 8; ++i) {
+      const int m = m0 + am(i), k = k0 + ak(i), mc = min(m, M - 1), kc = min(k, ke - 1);
+      const float v = ld<TA>(A, AK ? mc * lda + kc : kc * lda + mc);
+      ra[i] = m < M && k < ke ? v : 0.f;
     }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int n = n0 + bn(i), k = k0 + bk(i), nc = min(n, N - 1), kc = min(k, ke - 1);
+      const float v = ld<TB>(B, BK ? nc * ldb + kc : kc * ldb + nc);
+      rb[i] = n < N && k < ke ? v : 0.f;
+    }
+  };
+  f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  float rowsum = 0.f;
+  const int wm = (wv >> 1) * 16, wn = (wv & 1) * 32, lr = lane & 15, lk = lane >> 4;
+  if (kb < ke) fetch(kb);
+  for (int k0 = kb; k0 < ke; k0 += MLP_TK) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) As[ak(i)][am(i)] = ra[i];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) Bs[bk(i)][bn(i)] = rb[i];
     __syncthreads();
+    if (k0 + MLP_TK < ke) fetch(k0 + MLP_TK);
 #pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      float a[4], b[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = As[kk][ty + 16 * i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = Bs[kk][tx + 16 * j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
+    for (int kk = 0; kk < MLP_TK; kk += 4) {
+      const float a = As[kk + lk][wm + lr];
+      acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, Bs[kk + lk][wn + lr], acc[0], 0, 0, 0);
+      acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, Bs[kk + lk][wn + 16 + lr], acc[1], 0, 0, 0);
     }
+    if (EPI == EPI_SPLIT && blockIdx.y == 0 && tid < MLP_TM)
+      for (int kk = 0; kk < MLP_TK; ++kk) rowsum += As[kk][tid];
     __syncthreads();
   }
+  if (EPI == EPI_SPLIT && blockIdx.y == 0 && tid < MLP_TM && m0 + tid < M)
+    C2[(int64_t)blockIdx.z * M + m0 + tid] = rowsum;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = m0 + ty + 16 * i;
-    if (m >= M) continue;
+  for (int j = 0; j < 2; ++j)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + tx + 16 * j;
-      if (n >= N) continue;
+    for (int i = 0; i < 4; ++i) {
+      const int m = m0 + wm + lk * 4 + i, n = n0 + wn + 16 * j + lr;
+      if (m >= M || n >= N) continue;
       const int64_t o = (int64_t)m * N + n;
-      float v = acc[i][j];
+      float v = acc[j][i];
       if (EPI == EPI_FWD || EPI == EPI_FWD_LINEAR) {
         v += bias[n];
         C[o] = v;                                    /* pre-activation */
@@ -126,19 +155,22 @@ __global__ void __launch_bounds__(256) mlp_gemm_kernel(const TA* __restrict__ A,
       } else if (EPI == EPI_BWD_DATA) {
         C[o] = v * gelu_d(zprev[o]);
       } else {
-        C[o] = v;
+        C[(int64_t)blockIdx.z * M * N + o] = v;
       }
     }
-  }
 }
 
-/* db[n] = sum_b dz[b][n] */
-__global__ void mlp_bias_grad_kernel(const float* __restrict__ dz, int64_t B, int N, float* __restrict__ db) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= N) return;
+/* dW and db from the partial products of the splits, in their order */
+__global__ void __launch_bounds__(256) mlp_split_sum_kernel(const float* __restrict__ pw, const float* __restrict__ pb,
+                                                            int splits, int64_t nw, int nb, float* __restrict__ dw,
+                                                            float* __restrict__ db) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= nw + nb) return;
+  const float* p = i < nw ? pw + i : pb + (i - nw);
+  const int64_t st = i < nw ? nw : nb;
   float s = 0.f;
-  for (int64_t b = 0; b < B; ++b) s += dz[b * N + n];
-  db[n] = s;
+  for (int z = 0; z < splits; ++z) s += p[z * st];
+  (i < nw ? dw[i] : db[i - nw]) = s;
 }
 
 /* Weighted squared error over the outputs and its gradient:
@@ -195,17 +227,28 @@ __global__ void mlp_gather_kernel(const float* __restrict__ xall, const float* _
   for (int k = threadIdx.x; k < nout; k += blockDim.x) t[b * nout + k] = tall[r * nout + k];
 }
 
-dim3 gemm_grid(int M, int N) { return dim3((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64)); }
+dim3 gemm_grid(int M, int N, int splits = 1) {
+  return dim3((unsigned)((M + MLP_TM - 1) / MLP_TM), (unsigned)((N + MLP_TN - 1) / MLP_TN), (unsigned)splits);
+}
+
+/* Splits of a weight gradient's sum over B rows and the rows of each: 128
+ * rows, fewer splits where they would not fit the scratch that ensure_batch
+ * made (MLP_SPLITS of the largest layer). */
+constexpr int MLP_SPLITS = 16;
+int split_rows(int64_t B) {
+  const int64_t r = std::max<int64_t>(128, (B + MLP_SPLITS - 1) / MLP_SPLITS);
+  return (int)((r + MLP_TK - 1) / MLP_TK * MLP_TK);
+}
 
 void free_mlp_buffers(eqbf_mlp* m) {
   for (float* q : m->z) (void)hipFree(q);
   for (float* q : m->h) (void)hipFree(q);
   m->z.clear();
   m->h.clear();
-  void* ps[] = {m->dz0, m->dz1, m->xin, m->tgt, m->wout, m->loss, m->idx};
+  void* ps[] = {m->dz0, m->dz1, m->part, m->xin, m->tgt, m->wout, m->loss, m->idx};
   for (void* q : ps)
     if (q) (void)hipFree(q);
-  m->dz0 = m->dz1 = m->xin = m->tgt = m->wout = nullptr;
+  m->dz0 = m->dz1 = m->part = m->xin = m->tgt = m->wout = nullptr;
   m->loss = nullptr;
   m->idx = nullptr;
   m->cap = 0;
@@ -227,6 +270,9 @@ int ensure_batch(eqbf_ctx* ctx, eqbf_mlp* m, int64_t B) {
   }
   EQBF_HIP(ctx, hipMalloc(&m->dz0, (size_t)B * wmax * sizeof(float)));
   EQBF_HIP(ctx, hipMalloc(&m->dz1, (size_t)B * wmax * sizeof(float)));
+  size_t wlargest = 0;
+  for (int l = 0; l < L; ++l) wlargest = std::max(wlargest, (size_t)m->dout[l] * (m->din[l] + 1));
+  EQBF_HIP(ctx, hipMalloc(&m->part, MLP_SPLITS * wlargest * sizeof(float)));
   EQBF_HIP(ctx, hipMalloc(&m->xin, (size_t)B * m->n_in * sizeof(float)));
   EQBF_HIP(ctx, hipMalloc(&m->tgt, (size_t)B * m->n_out * sizeof(float)));
   EQBF_HIP(ctx, hipMalloc(&m->wout, 64 * sizeof(float)));
@@ -247,12 +293,12 @@ void forward(eqbf_ctx* ctx, eqbf_mlp* m, int64_t B) {
     const float* b = m->p + m->boff[l];
     ProfScope ps(ctx, "mlp_gemm_kernel", st);
     if (l + 1 < L)
-      hipLaunchKernelGGL((mlp_gemm_kernel<float, uint16_t, EPI_FWD>), gemm_grid((int)B, N), dim3(256), 0, st, x,
-                         (int64_t)K, (int64_t)1, W, (int64_t)1, (int64_t)K, (int)B, N, K, b, m->z[l], m->h[l],
+      hipLaunchKernelGGL((mlp_gemm_kernel<float, uint16_t, true, true, EPI_FWD>), gemm_grid((int)B, N), dim3(256), 0,
+                         st, x, (int64_t)K, W, (int64_t)K, (int)B, N, K, K, b, m->z[l], m->h[l],
                          (const float*)nullptr);
     else
-      hipLaunchKernelGGL((mlp_gemm_kernel<float, uint16_t, EPI_FWD_LINEAR>), gemm_grid((int)B, N), dim3(256), 0, st,
-                         x, (int64_t)K, (int64_t)1, W, (int64_t)1, (int64_t)K, (int)B, N, K, b, m->z[l], m->h[l],
+      hipLaunchKernelGGL((mlp_gemm_kernel<float, uint16_t, true, true, EPI_FWD_LINEAR>), gemm_grid((int)B, N),
+                         dim3(256), 0, st, x, (int64_t)K, W, (int64_t)K, (int)B, N, K, K, b, m->z[l], m->h[l],
                          (const float*)nullptr);
     x = m->h[l];
   }
@@ -272,15 +318,18 @@ void backward(eqbf_ctx* ctx, eqbf_mlp* m, int64_t B) {
     const float* xin = l > 0 ? m->h[l - 1] : m->xin; /* [B][K] */
     {
       ProfScope ps(ctx, "mlp_gemm_kernel", st);
-      /* dW[n][k] = sum_b dz[b][n] x[b][k] */
-      hipLaunchKernelGGL((mlp_gemm_kernel<float, float, EPI_STORE>), gemm_grid(N, K), dim3(256), 0, st, dz,
-                         (int64_t)1, (int64_t)N, xin, (int64_t)K, (int64_t)1, N, K, (int)B, (const float*)nullptr,
-                         m->g + m->woff[l], (float*)nullptr, (const float*)nullptr);
-      hipLaunchKernelGGL(mlp_bias_grad_kernel, dim3((N + 255) / 256), dim3(256), 0, st, dz, B, N,
-                         m->g + m->boff[l]);
+      /* dW[n][k] = sum_b dz[b][n] x[b][k], db[n] = sum_b dz[b][n] */
+      const int rows = split_rows(B), splits = (int)((B + rows - 1) / rows);
+      float* pb = m->part + (int64_t)splits * N * K;
+      hipLaunchKernelGGL((mlp_gemm_kernel<float, float, false, false, EPI_SPLIT>), gemm_grid(N, K, splits), dim3(256),
+                         0, st, dz, (int64_t)N, xin, (int64_t)K, N, K, (int)B, rows, (const float*)nullptr, m->part,
+                         pb, (const float*)nullptr);
+      const int64_t nw = (int64_t)N * K;
+      hipLaunchKernelGGL(mlp_split_sum_kernel, dim3((unsigned)((nw + N + 255) / 256)), dim3(256), 0, st, m->part, pb,
+                         splits, nw, N, m->g + m->woff[l], m->g + m->boff[l]);
       if (l > 0) /* dz_below[b][k] = sum_n dz[b][n] W[n][k] * gelu'(z_below[b][k]) */
-        hipLaunchKernelGGL((mlp_gemm_kernel<float, uint16_t, EPI_BWD_DATA>), gemm_grid((int)B, K), dim3(256), 0, st,
-                           dz, (int64_t)N, (int64_t)1, m->w16 + m->woff[l], (int64_t)K, (int64_t)1, (int)B, K, N,
+        hipLaunchKernelGGL((mlp_gemm_kernel<float, uint16_t, true, false, EPI_BWD_DATA>), gemm_grid((int)B, K),
+                           dim3(256), 0, st, dz, (int64_t)N, m->w16 + m->woff[l], (int64_t)K, (int)B, K, N, N,
                            (const float*)nullptr, dnext, (float*)nullptr, m->z[l - 1]);
     }
     std::swap(dz, dnext);

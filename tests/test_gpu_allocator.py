@@ -194,3 +194,44 @@ def test_allocator_end_to_end_and_ablation(eng, orc):
     assert calls_f.sum() > 0
     assert agree >= 0.95
     al.close()
+
+
+@pytest.mark.parametrize("n_in,hidden,layers,n_out,B", [(24, 256, 3, 3, 2049), (5, 33, 1, 1, 1), (31, 65, 2, 7, 129),
+                                                        (3, 8, 0, 2, 300)])
+def test_network_sizes_off_the_tiles(eng, n_in, hidden, layers, n_out, B):
+    """Rows, units and splits of the batch that do not fill a tile."""
+    net = engine.Mlp(eng, n_in, hidden, layers, n_out, seed=3)
+    ref = mo.Mlp(n_in, hidden, layers, n_out)
+    rng = np.random.default_rng(B)
+    params = net.get_params()
+    x = rng.normal(size=(B, n_in)).astype(np.float32)
+    t = rng.normal(size=(B, n_out)).astype(np.float32)
+    w = rng.uniform(0.5, 2, n_out).astype(np.float32)
+    y, y_ref = net.forward(x), ref.forward(params, x)
+    assert np.max(np.abs(y - y_ref)) <= 1e-5 * max(1.0, np.max(np.abs(y_ref)))  # FP32 sums of up to 256 terms
+    loss, g = net.loss_grad(x, t, w)
+    loss_ref, g_ref = ref.loss_grad(params, x, t, w)
+    assert loss == pytest.approx(loss_ref, rel=1e-5)
+    assert np.linalg.norm(g - g_ref) <= 1e-5 * np.linalg.norm(g_ref)
+    net.close()
+
+
+@pytest.mark.parametrize("N,P", [(17, 9), (33, 40), (300, 20), (511, 700), (512, 65)])
+def test_ld_eigenvalues_sizes(eng, N, P):
+    """Samples and SNPs off the tiles, fewer SNPs than vectors; missing
+    genotypes (mean for the Gram matrix) and a constant SNP."""
+    hc = synth.plain(seed=N, S=1, N=N, n_genes=2, snps_per_gene=P)
+    g = hc.genotypes[0]
+    g[:, 3] = 1.0
+    g[min(N - 1, 5), 0] = np.nan
+    eig = eng.ld_eigenvalues(hc, 20)
+    for gi in range(hc.G):
+        X = g[:, hc.pair_snp[hc.pair_offset[gi]:hc.pair_offset[gi + 1]]].astype(np.float64)
+        Z = X - np.nanmean(X, axis=0)
+        sd = np.sqrt(np.nanmean(Z ** 2, axis=0))
+        Z = np.nan_to_num(Z)[:, sd > 0] / sd[sd > 0]
+        lam = np.sort(np.linalg.eigvalsh(Z @ Z.T / N))[::-1][:20]
+        lam = np.concatenate([lam, np.zeros(20 - len(lam))]) if len(lam) < 20 else lam
+        # leading ones converge fastest; the last ones of a flat spectrum after 20 iterations to a few per cent
+        assert np.allclose(eig[gi, :5], lam[:5], rtol=1e-2, atol=1e-4 * lam[0])
+        assert np.allclose(eig[gi], lam, rtol=6e-2, atol=1e-4 * lam[0])
