@@ -1076,116 +1076,225 @@ __global__ void config_masks_kernel(int bfs, int S, uint64_t* __restrict__ masks
   }
 }
 
-/* ---- plain FP64 path: one launch per gene, one thread per pair ------------------ */
-__device__ double abf_plain(uint64_t mask, int S, const double* st_b, const double* st_se, const double* st_t,
-                            const uint8_t* has, double phi2, double oma2) {
-  /* CalcLog10AbfUvlr with the reference's expressions */
-  double bn = 0, bd = 0, vb = 0, single = 0;
-  bool any_single = false;
-  for (int s = 0; s < S; ++s) {
-    if (!((mask >> s) & 1ull) || !has[s]) continue;
-    double bhat = st_b[s], varbhat = pow(st_se[s], 2), t = st_t[s];
-    double l;
-    if (fabs(t) < 1e-8) {
-      l = 0;
-    } else {
-      bn += bhat / (varbhat + phi2);
-      bd += 1 / (varbhat + phi2);
-      vb += 1 / (varbhat + phi2);
-      l = 0.5 * log10(varbhat) - 0.5 * log10(varbhat + phi2) + (0.5 * pow(t, 2) * phi2 / (varbhat + phi2)) / log(10.0);
-    }
-    single += l;
-    any_single = true;
-  }
-  (void)any_single;
-  double bbar = (bd != 0.0) ? bn / bd : 0.0;
-  vb = (vb != 0.0) ? 1 / vb : INFINITY;
-  if (bbar != 0.0 && vb < INFINITY) {
-    double T2 = pow(bbar, 2.0) / vb;
-    double lb = (T2 != 0) ? 0.5 * log10(vb) - 0.5 * log10(vb + oma2) + (0.5 * T2 * oma2 / (vb + oma2)) / log(10.0) : 0;
-    return lb + single;
-  }
-  return 0.0;
-}
-
-__device__ double l10ws_plain(const double* v, int n) {
-  double mx = v[0];
-  for (int i = 0; i < n; ++i)
-    if (v[i] > mx) mx = v[i];
-  double w = 1 / ((double)n), sum = 0;
-  for (int i = 0; i < n; ++i)
-    if (!isnan(v[i])) sum += w * pow(10.0, v[i] - mx);
-  double res = mx + log10(sum);
-  if (fabs(res) <= 2.220446049250313e-16) res = 0.0;
-  return res;
-}
-
+/* ---- FP64 path ---------------------------------------------------------------
+ * A workgroup of eight waves takes 64 pairs, lane = pair in every wave: the
+ * waves share out the subgroups of the summary statistics, then the rows (grid
+ * types and configurations) of the Bayes factors, so that a call of a few
+ * hundred pairs is not one thread's serial work: the FP64 re-checks of 24 genes'
+ * permutations (2,000 pairs, 300 samples, 5 subgroups, --bfs all) went from 4.0 to
+ * 0.25 ms a launch, where a thread took a pair with pow() and a logarithm per
+ * subgroup and row.  The statistics reach the
+ * rows through LDS as iv = 1 / se^2, b iv and t^2 / (2 ln 10), all zero for a
+ * subgroup that takes no part. */
 #define PLAIN_SMAX 64
 #define PLAIN_GMAX 128
+constexpr int P64_WAVES = 8;
+
+struct P64Lds {
+  double *iv, *biv, *e; /* [S][64] */
+};
+__device__ __forceinline__ P64Lds p64_lds(double* base, int S) {
+  return {base, base + S * 64, base + 2 * S * 64};
+}
+__host__ __device__ inline size_t p64_lds_bytes(int S) { return (size_t)S * 64 * 3 * sizeof(double); }
+
+/* one subgroup's standardised statistics (b, se, t), has: it has results */
+__device__ __forceinline__ void p64_put(const P64Lds& l, int at, bool has, double b, double se, double t) {
+  const bool on = has && !(fabs(t) < 1e-8); /* a NaN t takes part */
+  const double iv = on ? 1.0 / (se * se) : 0.0;
+  l.iv[at] = iv;
+  l.biv[at] = on ? b * iv : 0.0;
+  l.e[at] = on ? t * t * 0.21714724095162590 : 0.0; /* 1 / (2 ln 10) */
+}
+
+/* CalcLog10AbfUvlr (gene_snp_pair.cpp:297-356) of the subgroups in mk at two
+ * points of the grid.  With k = 1 / (v + phi) the reference's terms are
+ *   sum_s [log10(v k) / 2 + t^2 phi k / (2 ln 10)]
+ *   + log10(V / (V + o)) / 2 + T^2 o / (V + o) / (2 ln 10),
+ * 1/V = sum k, T^2 = (sum b k)^2 V; v k = 1 / (1 + phi / v), V / (V + o) =
+ * 1 / (1 + o sum k), and the logarithms are taken of the product once.  As
+ * in the reference the result is 0 when the average effect is 0 or its variance
+ * infinite or NaN. */
+__device__ __forceinline__ void p64_row(const P64Lds& l, int lane, uint64_t mk, const double (&p2)[2],
+                                        const double (&o2)[2], double (&out)[2]) {
+  double bn[2] = {0, 0}, bd[2] = {0, 0}, pr[2] = {1, 1}, ex[2] = {0, 0}, lx[2] = {0, 0};
+  for (uint64_t m = mk; m; m &= m - 1) {
+    const int at = (__ffsll((unsigned long long)m) - 1) * 64 + lane;
+    const double iv = l.iv[at], biv = l.biv[at], e = l.e[at];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const double r = dm::rcp_nr(fma(p2[u], iv, 1.0)), k = iv * r;
+      bn[u] = fma(biv, r, bn[u]);
+      bd[u] += k;
+      ex[u] = fma(e * p2[u], k, ex[u]);
+      pr[u] *= r;
+      if (pr[u] < 1e-250) {
+        lx[u] += log10(pr[u]);
+        pr[u] = 1.0;
+      }
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const double q = dm::rcp_nr(fma(o2[u], bd[u], 1.0));
+    const double v = 0.5 * (lx[u] + dm::log10_sum(pr[u] * q)) + fma(bn[u] * bn[u] * 0.21714724095162590 * o2[u], q, ex[u]);
+    out[u] = isnan(bd[u]) || bn[u] == 0.0 || bd[u] == 0.0 ? 0.0 : v;
+  }
+}
+
+/* log10_weighted_sum with equal weights (utils_math.cpp:100-131), one value
+ * after the other: the sum of 10^(v - m) against a reference m that follows
+ * the maximum within 16 decades; a NaN first value makes the result NaN, later
+ * ones are skipped. */
+struct P64Lws {
+  double m, s;
+  __device__ __forceinline__ void first(double x) {
+    m = x;
+    s = x == -INFINITY ? 0.0 : dm::exp10_sum(x - x); /* NaN and +inf: NaN */
+  }
+  __device__ __forceinline__ void add(double x) {
+    if (x > m + 16.0 || (m == -INFINITY && x > m)) {
+      s *= dm::exp10_sum(m - x);
+      m = x;
+    }
+    if (x > -INFINITY || (isnan(m) && !isnan(x))) s += dm::exp10_sum(x - m);
+  }
+  __device__ __forceinline__ double finish(int n) const {
+    const double r = m + dm::log10_sum(s / (double)n);
+    return fabs(r) <= 2.220446049250313e-16 ? 0.0 : r;
+  }
+};
 
 /* The consistent configuration over the large grid (gen, gen-fix, gen-maxh)
- * and the configurations over the small grid of pair p, FP64
+ * and the configurations over the small grid of 64 pairs, FP64
  * (CalcAbfsUvlrForConsistentConfiguration / ForSingletons /
  * ForEachConfiguration, gene_snp_pair.cpp:364-550); gen-sin and all follow in
- * bma_kernel. */
-__device__ __forceinline__ void plain_pair_abfs(const AssocParams& kp, int S, int64_t NP, int64_t p,
-                                                const double* st_b, const double* st_se, const double* st_t,
-                                                const uint8_t* has) {
+ * bma_kernel.  A wave takes every P64_WAVES-th of the three types and the
+ * configurations. */
+__device__ __forceinline__ void p64_pair_abfs(const AssocParams& kp, const P64Lds& l, int S, int64_t NP, int64_t p,
+                                              bool valid, int lane, int wv) {
   const double* phiL = kp.grid;
   const double* omaL = phiL + kp.GL;
   const double* phiS = phiL + 2 * kp.GL;
   const double* omaS = phiS + kp.GS;
   const uint64_t all = (S >= 64) ? ~0ull : ((1ull << S) - 1ull);
-  double buf[PLAIN_GMAX];
-  for (int type = 0; type < 3; ++type) {
-    for (int gi = 0; gi < kp.GL; ++gi) {
-      double p2 = type == 0 ? phiL[gi] : (type == 1 ? 0.0 : phiL[gi] + omaL[gi]);
-      double o2 = type == 0 ? omaL[gi] : (type == 1 ? phiL[gi] + omaL[gi] : 0.0);
-      buf[gi] = abf_plain(all, S, st_b, st_se, st_t, has, p2, o2);
-      if (kp.raw) {
-        const int64_t ro = raw_index(type * kp.GL + gi, p, NP, 3 * (int64_t)kp.GL + (int64_t)kp.n_cfg * kp.GS,
-                                     kp.raw_tiled);
-        if (kp.raw_f64)
-          ((double*)kp.raw)[ro] = buf[gi];
+  const int64_t n_raw = 3 * (int64_t)kp.GL + (int64_t)kp.n_cfg * kp.GS;
+  for (int task = wv; task < 3 + kp.n_cfg; task += P64_WAVES) {
+    const int n = task < 3 ? kp.GL : kp.GS;
+    const uint64_t mk = task < 3 ? all : kp.masks[task - 3];
+    const int64_t row0 = task < 3 ? (int64_t)task * kp.GL : 3 * (int64_t)kp.GL + (int64_t)(task - 3) * kp.GS;
+    P64Lws a = {0.0, 0.0};
+    for (int g0 = 0; g0 < n; g0 += 2) {
+      double p2[2], o2[2], v[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int gi = min(g0 + u, n - 1);
+        if (task < 3) {
+          const double ph = phiL[gi], om = omaL[gi];
+          p2[u] = task == 0 ? ph : (task == 1 ? 0.0 : ph + om);
+          o2[u] = task == 0 ? om : (task == 1 ? ph + om : 0.0);
+        } else {
+          p2[u] = phiS[gi];
+          o2[u] = omaS[gi];
+        }
+      }
+      p64_row(l, lane, mk, p2, o2, v);
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        if (g0 + u >= n) break;
+        if (kp.raw && valid) {
+          const int64_t ro = raw_index(row0 + g0 + u, p, NP, n_raw, kp.raw_tiled);
+          if (kp.raw_f64)
+            ((double*)kp.raw)[ro] = v[u];
+          else
+            ((float*)kp.raw)[ro] = (float)v[u];
+        }
+        if (g0 + u == 0)
+          a.first(v[u]);
         else
-          ((float*)kp.raw)[ro] = (float)buf[gi];
+          a.add(v[u]);
       }
     }
-    kp.w[(int64_t)type * NP + p] = l10ws_plain(buf, kp.GL);
-  }
-  for (int cfg = 0; cfg < kp.n_cfg; ++cfg) {
-    const uint64_t mk = kp.masks[cfg];
-    bool any = false;
-    for (int s = 0; s < S; ++s) any |= ((mk >> s) & 1ull) && has[s];
-    for (int gi = 0; gi < kp.GS; ++gi) {
-      buf[gi] = any ? abf_plain(mk, S, st_b, st_se, st_t, has, phiS[gi], omaS[gi]) : 0.0;
-      if (kp.raw) {
-        const int64_t ro = raw_index(3 * kp.GL + cfg * kp.GS + gi, p, NP,
-                                     3 * (int64_t)kp.GL + (int64_t)kp.n_cfg * kp.GS, kp.raw_tiled);
-        if (kp.raw_f64)
-          ((double*)kp.raw)[ro] = buf[gi];
-        else
-          ((float*)kp.raw)[ro] = (float)buf[gi];
-      }
-    }
-    kp.w[(int64_t)(3 + cfg) * NP + p] = l10ws_plain(buf, kp.GS);
+    if (valid) kp.w[(int64_t)task * NP + p] = a.finish(n);
   }
 }
 
+/* Summary statistics of one (pair, subgroup) from its sums
+ * (FitSingleGeneWithSingleSnp, utils_math.cpp:166-209): written out and left in
+ * LDS for the rows. */
+template <int KU>
+__device__ __forceinline__ void p64_stats(const eqbf_chunk& c, const AssocParams& kp, const P64Lds& l, const PrepRec& r,
+                                          bool has, double sxx, double sxy, const double (&a)[KU], int s, int S,
+                                          int64_t NP, int64_t p, bool valid, int lane) {
+  double st[3] = {NAN, NAN, NAN}, o5[5] = {NAN, NAN, NAN, NAN, NAN};
+  if (has && !(r.flags & PREP_TOO_FEW)) {
+    double proj = 0;
+#pragma unroll
+    for (int q = 0; q < KU; ++q) proj += a[q] * a[q];
+    const double xx = sxx - proj;
+    const int n = r.n, P = r.q + 2;
+    if (xx > 1e-12 * sxx) {
+      const double beta = sxy / xx;
+      const double rss = r.yy - sxy * beta;
+      const int rank = r.rank + 1;
+      const double se = sqrt(rss / (double)(n - P) / xx);
+      const double sig = sqrt(rss / (double)(n - rank));
+      o5[0] = 1.0 - rss / r.tss;
+      o5[1] = sig;
+      o5[2] = beta;
+      o5[3] = se;
+      if (kp.sstats) o5[4] = 2.0 * dm::t_lower_neg(fabs(beta / se), (double)(n - rank));
+      /* StandardizeSstatsAndCorrectSmallSampleSize (gene_snp_pair.cpp:256-290) */
+      double bhat = beta / sig, sebhat = se / sig, t = bhat / sebhat;
+      if (!isnan(t)) {
+        const double nu = (double)n - 2 - r.q;
+        t = dm::gauss_pinv(dm::t_lower_neg(fabs(bhat / sebhat), nu));
+        if (fabs(t) > 1e-8) {
+          const double sig2 = fabs(beta) / (fabs(t) * sebhat);
+          bhat = beta / sig2;
+          sebhat = fabs(bhat / t);
+        } else {
+          bhat = 0;
+          sebhat = INFINITY;
+        }
+        st[0] = bhat;
+        st[1] = sebhat;
+        st[2] = t;
+      }
+    } else {
+      o5[0] = 1.0 - r.yy / r.tss;
+      o5[1] = sqrt(r.yy / (double)(n - r.rank));
+    }
+  }
+  p64_put(l, s * 64 + lane, has, st[0], st[1], st[2]);
+  if (!valid) return;
+  kp.n_out[(int64_t)s * NP + p] = has ? r.n : 0;
+  if (kp.sstats)
+    for (int k = 0; k < 5; ++k) kp.sstats[((int64_t)k * S + s) * NP + p] = o5[k];
+  if (kp.stdsstats)
+    for (int k = 0; k < 3; ++k) kp.stdsstats[((int64_t)k * S + s) * NP + p] = st[k];
+}
+
 /* g >= 0: pairs of gene g (the plain path, one launch per gene); g < 0:
- * every pair of the chunk in one launch, thread = pair, its gene found by
- * binary search of pair_offset (EQBF_PREC_FP64_BATCHED).  Each pair's
- * arithmetic is the same either way. */
-__global__ void __launch_bounds__(64) assoc_plain_kernel(const eqbf_chunk c, const AssocParams kp, int g) {
+ * every pair of the chunk in one launch, the gene of a pair found by binary
+ * search of pair_offset (EQBF_PREC_FP64_BATCHED).  Each pair's arithmetic is
+ * the same either way.  KU: columns of the basis.  With four subgroups or
+ * fewer the waves also share out the members of a subgroup (parts), whose sums
+ * meet in LDS. */
+template <int KU>
+__global__ void __launch_bounds__(64 * P64_WAVES) __attribute__((amdgpu_waves_per_eu(KU <= 4 ? 4 : 2, 8)))
+assoc_plain_kernel(const eqbf_chunk c, const AssocParams kp, int g) {
+  extern __shared__ __align__(16) double p64_smem[];
   const int S = c.n_subgroups, N = c.n_samples;
   const int64_t NP = c.n_pairs;
-  int64_t p;
-  if (g >= 0) {
-    p = c.pair_offset[g] + blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (p >= c.pair_offset[g + 1]) return;
-  } else {
-    p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (p >= NP) return;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const P64Lds l = p64_lds(p64_smem, S);
+  double* sums = p64_smem + (p64_lds_bytes(S) + 7) / 8; /* [parts][S][2 + KU][64] */
+  const int64_t lo_p = g >= 0 ? c.pair_offset[g] : 0, hi_p = g >= 0 ? c.pair_offset[g + 1] : NP;
+  const int64_t pp = lo_p + blockIdx.x * (int64_t)64 + lane;
+  const bool valid = pp < hi_p;
+  const int64_t p = valid ? pp : hi_p - 1;
+  if (g < 0) {
     int lo = 0, hi = c.n_genes; /* pair_offset[lo] <= p < pair_offset[hi] */
     while (hi - lo > 1) {
       const int mid = (lo + hi) >> 1;
@@ -1197,95 +1306,95 @@ __global__ void __launch_bounds__(64) assoc_plain_kernel(const eqbf_chunk c, con
     g = lo;
   }
   const int64_t snp = c.pair_snp[p];
-  const int KC = kp.KU + 1;
-  double st_b[PLAIN_SMAX], st_se[PLAIN_SMAX], st_t[PLAIN_SMAX];
-  uint8_t has[PLAIN_SMAX];
-  for (int s = 0; s < S; ++s) {
+  constexpr int KC = KU + 1, U = 4;
+  const int parts = S <= 4 ? P64_WAVES / S : 1;
+  for (int item = wv; item < S * parts; item += P64_WAVES) {
+    const int s = item / parts, part = item - s * parts;
     const PrepRec r = kp.rec[(int64_t)g * S + s];
-    has[s] = r.n > 0 && c.snp_in_sbgrp[snp * S + s];
-    st_b[s] = st_se[s] = st_t[s] = NAN;
-    double o5[5] = {NAN, NAN, NAN, NAN, NAN};
-    if (has[s] && !(r.flags & PREP_TOO_FEW)) {
+    const bool has = r.n > 0 && c.snp_in_sbgrp[snp * S + s];
+    double sxx = 0, sxy = 0, a[KU];
+#pragma unroll
+    for (int q = 0; q < KU; ++q) a[q] = 0;
+    if (has && !(r.flags & PREP_TOO_FEW)) {
       const int32_t* idx = kp.idx + ((int64_t)g * S + s) * N;
-      double sxx = 0, sxy = 0, a[17];
-      for (int q = 0; q < kp.KU; ++q) a[q] = 0;
       const int set = c.geno_set_of_sbgrp[s];
-      for (int k = 0; k < r.n; ++k) {
-        const int i = idx[k];
-        const double x = geno_load(c, set, i, snp);
-        const double* b = kp.B + (((int64_t)g * N + i) * S + s) * KC;
-        sxx += x * x;
-        sxy += x * b[0];
-        for (int q = 0; q < kp.KU; ++q) a[q] += x * b[1 + q];
-      }
-      double proj = 0;
-      for (int q = 0; q < kp.KU; ++q) proj += a[q] * a[q];
-      const double xx = sxx - proj;
-      const int n = r.n, P = r.q + 2;
-      if (xx > 1e-12 * sxx) {
-        const double beta = sxy / xx;
-        const double rss = r.yy - sxy * beta;
-        const int rank = r.rank + 1;
-        const double se = sqrt(rss / (double)(n - P) / xx);
-        const double sig = sqrt(rss / (double)(n - rank));
-        o5[0] = 1.0 - rss / r.tss;
-        o5[1] = sig;
-        o5[2] = beta;
-        o5[3] = se;
-        o5[4] = 2.0 * dm::t_lower_neg(fabs(beta / se), (double)(n - rank));
-        /* StandardizeSstatsAndCorrectSmallSampleSize (gene_snp_pair.cpp:256-290) */
-        double bhat = beta / sig, sebhat = se / sig, t = bhat / sebhat;
-        if (!isnan(t)) {
-          double nu = (double)n - 2 - r.q;
-          t = dm::gauss_pinv(dm::t_lower_neg(fabs(bhat / sebhat), nu));
-          if (fabs(t) > 1e-8) {
-            double sig2 = fabs(beta) / (fabs(t) * sebhat);
-            bhat = beta / sig2;
-            sebhat = fabs(bhat / t);
-          } else {
-            bhat = 0;
-            sebhat = INFINITY;
-          }
-          st_b[s] = bhat;
-          st_se[s] = sebhat;
-          st_t[s] = t;
+      const int k1 = (int)((int64_t)r.n * (part + 1) / parts);
+      for (int k = (int)((int64_t)r.n * part / parts); k < k1; k += U) {
+        int i[U];
+        double x[U], b[U][KC];
+#pragma unroll
+        for (int u = 0; u < U; ++u) i[u] = idx[min(k + u, k1 - 1)];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          x[u] = geno_load(c, set, i[u], snp);
+          const double* bp = kp.B + (((int64_t)g * N + i[u]) * S + s) * KC;
+#pragma unroll
+          for (int q = 0; q < KC; ++q) b[u][q] = bp[q];
         }
-      } else {
-        o5[0] = 1.0 - r.yy / r.tss;
-        o5[1] = sqrt(r.yy / (double)(n - r.rank));
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          if (k + u < k1) {
+            sxx += x[u] * x[u];
+            sxy += x[u] * b[u][0];
+#pragma unroll
+            for (int q = 0; q < KU; ++q) a[q] += x[u] * b[u][1 + q];
+          }
+        }
       }
     }
-    kp.n_out[(int64_t)s * NP + p] = has[s] ? r.n : 0;
-    if (kp.sstats)
-      for (int k = 0; k < 5; ++k) kp.sstats[((int64_t)k * S + s) * NP + p] = o5[k];
-    if (kp.stdsstats) {
-      kp.stdsstats[((int64_t)0 * S + s) * NP + p] = st_b[s];
-      kp.stdsstats[((int64_t)1 * S + s) * NP + p] = st_se[s];
-      kp.stdsstats[((int64_t)2 * S + s) * NP + p] = st_t[s];
+    if (parts == 1) {
+      p64_stats<KU>(c, kp, l, r, has, sxx, sxy, a, s, S, NP, p, valid, lane);
+    } else {
+      double* o = sums + ((size_t)(part * S + s) * (2 + KU)) * 64 + lane;
+      o[0] = sxx;
+      o[64] = sxy;
+#pragma unroll
+      for (int q = 0; q < KU; ++q) o[(2 + q) * 64] = a[q];
     }
   }
-  if (!kp.join) return;
-  plain_pair_abfs(kp, S, NP, p, st_b, st_se, st_t, has);
+  __syncthreads();
+  if (parts > 1) {
+    for (int s = wv; s < S; s += P64_WAVES) {
+      double sxx = 0, sxy = 0, a[KU];
+#pragma unroll
+      for (int q = 0; q < KU; ++q) a[q] = 0;
+      for (int part = 0; part < parts; ++part) {
+        const double* o = sums + ((size_t)(part * S + s) * (2 + KU)) * 64 + lane;
+        sxx += o[0];
+        sxy += o[64];
+#pragma unroll
+        for (int q = 0; q < KU; ++q) a[q] += o[(2 + q) * 64];
+      }
+      const PrepRec r = kp.rec[(int64_t)g * S + s];
+      p64_stats<KU>(c, kp, l, r, r.n > 0 && c.snp_in_sbgrp[snp * S + s], sxx, sxy, a, s, S, NP, p, valid, lane);
+    }
+    __syncthreads();
+  }
+  if (kp.join) p64_pair_abfs(kp, l, S, NP, p, valid, lane, wv);
 }
 
 /* --inss: summary statistics given per (pair, subgroup) instead of computed
  * (GeneSnpPair::SetSstats, gene_snp_pair.cpp:241-254), standardised with
  * nu = n - 2 since no covariate count is known for them (:273, the map entry
- * defaults to 0), then the Bayes factors as on the plain path; one thread per
- * pair, FP64.  n <= 0: no result in that subgroup (HasResults, :61-68). */
-__global__ void __launch_bounds__(64) inss_abf_kernel(const eqbf_sstats_in in, const AssocParams kp) {
+ * defaults to 0), then the Bayes factors as on the FP64 path.  n <= 0: no
+ * result in that subgroup (HasResults, :61-68).  Bound by the FP64
+ * instructions: one logarithm and one exponential per row.  60,001 pairs of 5
+ * subgroups, --bfs all: 0.26 ms (2.6 ms with a thread per pair). */
+__global__ void __launch_bounds__(64 * P64_WAVES) __attribute__((amdgpu_waves_per_eu(4, 8))) inss_abf_kernel(const eqbf_sstats_in in, const AssocParams kp) {
+  extern __shared__ __align__(16) double p64_smem[];
   const int S = in.n_subgroups;
   const int64_t NP = in.n_pairs;
-  const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (p >= NP) return;
-  double st_b[PLAIN_SMAX], st_se[PLAIN_SMAX], st_t[PLAIN_SMAX];
-  uint8_t has[PLAIN_SMAX];
-  for (int s = 0; s < S; ++s) {
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t pp = blockIdx.x * (int64_t)64 + lane;
+  const bool valid = pp < NP;
+  const int64_t p = valid ? pp : NP - 1;
+  const P64Lds l = p64_lds(p64_smem, S);
+  for (int s = wv; s < S; s += P64_WAVES) {
     const int64_t e = (int64_t)s * NP + p;
     const int64_t n = in.n[e];
-    has[s] = n > 0;
-    st_b[s] = st_se[s] = st_t[s] = NAN;
-    if (has[s]) {
+    const bool has = n > 0;
+    double b = NAN, se = NAN, z = NAN;
+    if (has) {
       /* StandardizeSstatsAndCorrectSmallSampleSize (:256-290) */
       const double beta = in.betahat[e];
       double bhat = beta / in.sigmahat[e], sebhat = in.sebetahat[e] / in.sigmahat[e], t = bhat / sebhat;
@@ -1300,19 +1409,41 @@ __global__ void __launch_bounds__(64) inss_abf_kernel(const eqbf_sstats_in in, c
           bhat = 0;
           sebhat = INFINITY;
         }
-        st_b[s] = bhat;
-        st_se[s] = sebhat;
-        st_t[s] = t;
+        b = bhat;
+        se = sebhat;
+        z = t;
       }
     }
-    if (kp.n_out) kp.n_out[e] = has[s] ? (int32_t)(n < 2147483647 ? n : 2147483647) : 0;
+    p64_put(l, s * 64 + lane, has, b, se, z);
+    if (!valid) continue;
+    if (kp.n_out) kp.n_out[e] = has ? (int32_t)(n < 2147483647 ? n : 2147483647) : 0;
     if (kp.stdsstats) {
-      kp.stdsstats[e] = st_b[s];
-      kp.stdsstats[(int64_t)S * NP + e] = st_se[s];
-      kp.stdsstats[(int64_t)2 * S * NP + e] = st_t[s];
+      kp.stdsstats[e] = b;
+      kp.stdsstats[(int64_t)S * NP + e] = se;
+      kp.stdsstats[(int64_t)2 * S * NP + e] = z;
     }
   }
-  plain_pair_abfs(kp, S, NP, p, st_b, st_se, st_t, has);
+  __syncthreads();
+  p64_pair_abfs(kp, l, S, NP, p, valid, lane, wv);
+}
+
+/* LDS: the rows' statistics, and the partial sums where waves share a subgroup */
+template <int KU>
+void launch_plain(const eqbf_chunk& c, const AssocParams& kp, int64_t n_pairs, int g, hipStream_t st) {
+  const int S = c.n_subgroups;
+  const size_t parts = S <= 4 ? P64_WAVES / S : 0;
+  const size_t lds = (p64_lds_bytes(S) + 7) / 8 * 8 + parts * S * (2 + KU) * 64 * sizeof(double);
+  hipLaunchKernelGGL(assoc_plain_kernel<KU>, dim3((unsigned)((n_pairs + 63) / 64)), dim3(64 * P64_WAVES), lds, st, c, kp,
+                     g);
+}
+void dispatch_plain(int KU, const eqbf_chunk& c, const AssocParams& kp, int64_t n_pairs, int g, hipStream_t st) {
+  switch (KU) {
+    case 1: return launch_plain<1>(c, kp, n_pairs, g, st);
+    case 4: return launch_plain<4>(c, kp, n_pairs, g, st);
+    case 8: return launch_plain<8>(c, kp, n_pairs, g, st);
+    case 16: return launch_plain<16>(c, kp, n_pairs, g, st);
+    default: return launch_plain<17>(c, kp, n_pairs, g, st);
+  }
 }
 
 template <int NWV, int SPW, int KU>
@@ -1337,24 +1468,38 @@ int dispatch_mixed(int S, const eqbf_chunk& c, const AssocParams& kp, int grid, 
 }  // namespace
 
 /* ---- orchestration ------------------------------------------------------------- */
-int launch_bma(eqbf_ctx* ctx, double* w, int64_t NP, int S, int bfs, hipStream_t st) {
+int ctx_cfg_tables(eqbf_ctx* ctx, int bfs, int S, const uint64_t** masks, const double** inv_choose, hipStream_t st) {
   const int64_t n_cfg = eqbf_n_configs(bfs, S);
   if (n_cfg < 0) return ctx_fail(ctx, EQBF_ERR_UNSUPPORTED, "--bfs all with %d subgroups", S);
   const int64_t nm = std::max<int64_t>(n_cfg, 1);
-  uint64_t* d_masks = (uint64_t*)ctx_buf(ctx, "bma_tab", (size_t)nm * sizeof(uint64_t) + 65 * sizeof(double));
-  if (!d_masks) return ctx_fail(ctx, EQBF_ERR_HIP, "allocating the BMA tables failed");
-  double* d_inv_choose = (double*)(d_masks + nm);
-  std::vector<uint64_t> hm(nm, 0);
-  if (n_cfg > 0) eqbf_config_masks(bfs, S, hm.data());
-  std::vector<double> ic(65, 0.0);
-  for (int k = 1; k <= S; ++k) {
-    double ch = 1;
-    for (int i = 1; i <= k; ++i) ch = ch * (S - k + i) / i;
-    ic[k] = 1.0 / ch;
+  uint64_t*& d = ctx->cfg_tables[{bfs, S}];
+  if (!d) {
+    uint64_t* b = (uint64_t*)ctx_buf(ctx, "cfg_tables/" + std::to_string(bfs) + "/" + std::to_string(S),
+                                     (size_t)(nm + 65) * sizeof(uint64_t));
+    if (!b) return EQBF_ERR_HIP; /* ctx_buf has set the message */
+    std::vector<uint64_t> h(nm + 65, 0);
+    if (n_cfg > 0) eqbf_config_masks(bfs, S, h.data());
+    for (int k = 1; k <= S; ++k) {
+      double ch = 1;
+      for (int i = 1; i <= k; ++i) ch = ch * (S - k + i) / i;
+      const double ic = 1.0 / ch;
+      memcpy(&h[nm + k], &ic, sizeof ic);
+    }
+    EQBF_HIP(ctx, hipMemcpyAsync(b, h.data(), h.size() * sizeof(uint64_t), hipMemcpyHostToDevice, st));
+    EQBF_HIP(ctx, hipStreamSynchronize(st)); /* h goes out of scope; other streams may use the tables at once */
+    d = b;
   }
-  EQBF_HIP(ctx, hipMemcpyAsync(d_masks, hm.data(), nm * sizeof(uint64_t), hipMemcpyHostToDevice, st));
-  EQBF_HIP(ctx, hipMemcpyAsync(d_inv_choose, ic.data(), 65 * sizeof(double), hipMemcpyHostToDevice, st));
-  EQBF_HIP(ctx, hipStreamSynchronize(st)); /* host vectors go out of scope */
+  *masks = d;
+  *inv_choose = (const double*)(d + nm);
+  return EQBF_OK;
+}
+
+int launch_bma(eqbf_ctx* ctx, double* w, int64_t NP, int S, int bfs, hipStream_t st) {
+  const int64_t n_cfg = eqbf_n_configs(bfs, S);
+  const uint64_t* d_masks;
+  const double* d_inv_choose;
+  const int rc = ctx_cfg_tables(ctx, bfs, S, &d_masks, &d_inv_choose, st);
+  if (rc) return rc;
   {
     ProfScope ps(ctx, "bma_kernel", st);
     hipLaunchKernelGGL(bma_kernel, dim3((unsigned)((NP + 255) / 256)), dim3(256), 0, st, w, NP, S, (int)n_cfg,
@@ -1494,7 +1639,7 @@ int assoc_uvlr_run(eqbf_ctx* ctx, const eqbf_chunk* cp, const eqbf_assoc_opts* o
     if (S > PLAIN_SMAX) return ctx_fail(ctx, EQBF_ERR_UNSUPPORTED, "plain path supports at most 64 subgroups");
     if (o->precision == EQBF_PREC_FP64_BATCHED) {
       ProfScope ps(ctx, "assoc_plain_kernel", st);
-      hipLaunchKernelGGL(assoc_plain_kernel, dim3((unsigned)((c.n_pairs + 63) / 64)), dim3(64), 0, st, c, kp, -1);
+      dispatch_plain(KU, c, kp, c.n_pairs, -1, st);
     } else {
       std::vector<int64_t> off(G + 1);
       EQBF_HIP(ctx, hipMemcpyAsync(off.data(), c.pair_offset, (G + 1) * sizeof(int64_t), hipMemcpyDeviceToHost, st));
@@ -1503,7 +1648,7 @@ int assoc_uvlr_run(eqbf_ctx* ctx, const eqbf_chunk* cp, const eqbf_assoc_opts* o
         int64_t np = off[g + 1] - off[g];
         if (np <= 0) continue;
         ProfScope ps(ctx, "assoc_plain_kernel", st);
-        hipLaunchKernelGGL(assoc_plain_kernel, dim3((unsigned)((np + 63) / 64)), dim3(64), 0, st, c, kp, g);
+        dispatch_plain(KU, c, kp, np, g, st);
       }
     }
     EQBF_HIP(ctx, hipGetLastError());
@@ -1587,23 +1732,10 @@ int abf_from_sstats_run(eqbf_ctx* ctx, const eqbf_sstats_in* in, int bfs, int ra
   if (!out->w_abf) return ctx_fail(ctx, EQBF_ERR_ARG, "w_abf is required");
   if (NP == 0) return EQBF_OK;
   if (!in->n || !in->sigmahat || !in->betahat || !in->sebetahat) return ctx_fail(ctx, EQBF_ERR_ARG, "null input");
-  const int64_t nm = std::max<int64_t>(n_cfg, 1);
-  uint64_t* d_masks = (uint64_t*)ctx_buf(ctx, "inss_tab", (size_t)nm * sizeof(uint64_t) + 65 * sizeof(double));
-  if (!d_masks) return EQBF_ERR_HIP; /* ctx_buf has set the message */
-  double* d_inv_choose = (double*)(d_masks + nm);
-  {
-    std::vector<uint64_t> hm(nm, 0);
-    if (n_cfg > 0) eqbf_config_masks(bfs, S, hm.data());
-    std::vector<double> ic(65, 0.0);
-    for (int k = 1; k <= S; ++k) {
-      double ch = 1;
-      for (int i = 1; i <= k; ++i) ch = ch * (S - k + i) / i;
-      ic[k] = 1.0 / ch;
-    }
-    EQBF_HIP(ctx, hipMemcpyAsync(d_masks, hm.data(), nm * sizeof(uint64_t), hipMemcpyHostToDevice, st));
-    EQBF_HIP(ctx, hipMemcpyAsync(d_inv_choose, ic.data(), 65 * sizeof(double), hipMemcpyHostToDevice, st));
-    EQBF_HIP(ctx, hipStreamSynchronize(st)); /* host vectors go out of scope */
-  }
+  const uint64_t* d_masks;
+  const double* d_inv_choose;
+  const int rc = ctx_cfg_tables(ctx, bfs, S, &d_masks, &d_inv_choose, st);
+  if (rc) return rc;
   AssocParams kp;
   memset(&kp, 0, sizeof kp);
   kp.grid = (const double*)ctx->d_grid.ptr;
@@ -1622,7 +1754,8 @@ int abf_from_sstats_run(eqbf_ctx* ctx, const eqbf_sstats_in* in, int bfs, int ra
   kp.raw_tiled = raw_dtype == EQBF_F32_TILED;
   {
     ProfScope ps(ctx, "inss_abf_kernel", st);
-    hipLaunchKernelGGL(inss_abf_kernel, dim3((unsigned)((NP + 63) / 64)), dim3(64), 0, st, *in, kp);
+    hipLaunchKernelGGL(inss_abf_kernel, dim3((unsigned)((NP + 63) / 64)), dim3(64 * P64_WAVES), p64_lds_bytes(S), st,
+                       *in, kp);
   }
   EQBF_HIP(ctx, hipGetLastError());
   {

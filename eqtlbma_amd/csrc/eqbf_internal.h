@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <cstring>
 #include <cstdio>
 #include <map>
 #include <string>
@@ -60,6 +61,9 @@ struct eqbf_ctx {
     float ms = 0.f;
   };
   std::map<std::string, TuneChoice> tuned;
+  /* configuration masks and 1 / C(S, k) per (--bfs, S), in buffers of their
+   * own (ctx_cfg_tables) */
+  std::map<std::pair<int, int>, uint64_t*> cfg_tables;
   /* live kernel timing (eqbf_profile) */
   bool prof_on = false;
   struct ProfEntry {
@@ -297,8 +301,52 @@ __device__ __forceinline__ double exp10_core(double x) {
   return __builtin_amdgcn_ldexp(fma(q, f, 1.0), __double2loint(t));
 }
 
+/* 1 / x within an ulp for normal x whose reciprocal is normal */
+__device__ __forceinline__ double rcp_nr(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(fma(-x, r, 1.0), r, r);
+  return fma(fma(-x, r, 1.0), r, r);
+}
+
 /* 10^x for any x <= 308, -inf and NaN included: the terms of a log10 sum */
 __device__ __forceinline__ double exp10_sum(double x) { return exp10_core(x < -400.0 ? -400.0 : x); }
+
+/* log10 x, within an ulp.  x = 2^e m with m in [sqrt 1/2, sqrt 2), f = m - 1,
+ * s = f / (2 + f): ln m = f - (f^2/2 - s (f^2/2 + s^2 T(s^2))), T the interpolant
+ * of (2 atanh(s)/s - 2)/s^2 at seven Chebyshev nodes (4.7e-18 relative in ln m);
+ * ln m is kept in two parts, and e log10 2 with a leading part that is exact.
+ * About a third of the math library's instructions, which this leaves to
+ * zero, denormals, infinities, negative values and NaN. */
+__device__ __host__ __forceinline__ double log10_sum(double x) {
+  uint64_t u;
+  memcpy(&u, &x, 8);
+  const int32_t hx = (int32_t)(u >> 32);
+  if (__builtin_expect((uint32_t)(hx - 0x00100000) >= 0x7fe00000u, 0)) return log10(x);
+  const int32_t k = (hx - 0x3fe6a09e) >> 20; /* m >= sqrt 1/2 */
+  u -= (uint64_t)(uint32_t)(k << 20) << 32;
+  double m;
+  memcpy(&m, &u, 8);
+  const double f = m - 1.0, d = m + 1.0, e = (double)k;
+#ifdef __HIP_DEVICE_COMPILE__
+  double r = __builtin_amdgcn_rcp(d);
+  r = fma(fma(-d, r, 1.0), r, r);
+  r = fma(fma(-d, r, 1.0), r, r);
+#else
+  const double r = 1.0 / d;
+#endif
+  double s = f * r;
+  s = fma(fma(-s, d, f), r, s);
+  const double z = s * s, h = 0.5 * f * f;
+  double t = fma(0x1.2b584aae78a57p-3, z, 0x1.39fe606542ddep-3);
+  t = fma(t, z, 0x1.7462b4ab2ef6bp-3);
+  t = fma(t, z, 0x1.c71c62e5800a1p-3);
+  t = fma(t, z, 0x1.2492492df148dp-2);
+  t = fma(t, z, 0x1.99999999952e2p-2);
+  t = fma(t, z, 0x1.5555555555558p-1);
+  const double hi = f - h, lo = fma(s, fma(z, t, h), (f - hi) - h);
+  const double small = fma(hi, 0x1.95355baaafad3p-57, fma(lo, 0x1.bcb7b1526e50ep-2, e * 0x1.f79fef311f12bp-34));
+  return fma(e, 0x1.34413508p-2, fma(hi, 0x1.bcb7b1526e50ep-2, small));
+}
 
 }  // namespace dm
 
@@ -416,6 +464,9 @@ int avg_grid_run(eqbf_ctx* ctx, const double* raw, int64_t n_rows, int L, const 
 int abf_from_sstats_run(eqbf_ctx* ctx, const eqbf_sstats_in* in, int bfs, int raw_dtype, eqbf_assoc_out* out,
                         hipStream_t st);
 /* gen-sin and all rows of out->w_abf from the grid-averaged rows. */
+/* Configuration masks and inverse binomials of (bfs, S) on the device:
+ * uploaded, and waited for, by the first call that needs them. */
+int ctx_cfg_tables(eqbf_ctx* ctx, int bfs, int S, const uint64_t** masks, const double** inv_choose, hipStream_t st);
 int launch_bma(eqbf_ctx* ctx, double* w, int64_t n_pairs, int S, int bfs, hipStream_t st);
 int perm_stats_run(eqbf_ctx* ctx, const eqbf_chunk* c, const eqbf_perm_opts* po, const int32_t* tables_dev,
                    int32_t n_tables, const int32_t* gene_table, int64_t nperm, double* stats_dev, hipStream_t st);

@@ -233,3 +233,18 @@ def test_raw_tiled_layout(eng, orc, mode):
         b = eng.assoc_uvlr(hc, "join", "all", precision=mode, raw_tiled=True)
         assert np.array_equal(a.raw, b.raw, equal_nan=True)
         assert np.array_equal(a.w, b.w, equal_nan=True) and np.array_equal(a.n, b.n)
+
+
+@pytest.mark.parametrize("S,Q", [(1, 0), (2, 16), (4, 7), (5, 0), (8, 3), (9, 0), (44, 3), (64, 1)])
+def test_fp64_path_subgroups_and_covariates(eng, orc, S, Q):
+    """The FP64 path's split over waves (members of few subgroups, subgroups,
+    rows), each basis width, pairs that do not fill a workgroup; one launch
+    for the chunk gives the bits of one launch per gene."""
+    hc = synth.batched(seed=7 * S + Q, S=S, N_all=90, n_genes=3, p_mean=45, p_lo=10, p_hi=90, ns_lo=50, ns_hi=85,
+                       Q=Q, nan_frac=0.02, absent_frac=0.1 if S > 1 else 0.0)
+    bfs = "all" if S <= 5 else "sin"
+    gpu, _ref = _run(eng, orc, hc, bfs, GL25, GS10, "plain", tag="fp64 S=%d Q=%d" % (S, Q))
+    one = eng.assoc_uvlr(hc, analysis="join", bfs=bfs, precision="fp64_batched")
+    for a, b in ((gpu.n, one.n), (gpu.sstats, one.sstats), (gpu.stdsstats, one.stdsstats), (gpu.raw, one.raw),
+                 (gpu.w, one.w)):
+        assert np.array_equal(a, b, equal_nan=True)

@@ -122,3 +122,17 @@ def test_inss_empty_and_errors(eng):
     big = np.ones((65, 1))
     with pytest.raises(engine.EngineError, match="at most 64 subgroups"):
         eng.abf_from_sstats(big.astype(np.int64), big, big, big, "sin")
+
+
+@pytest.mark.parametrize("S,bfs,NP", [(64, "sin", 65), (9, "all", 1), (12, "gen", 127)])
+def test_inss_many_subgroups_and_tiny_errors(eng, orc, S, bfs, NP):
+    """Sizes off the workgroups' 64 pairs, and standard errors so small that
+    the product of the subgroups' ratios leaves the range of doubles."""
+    rng = np.random.default_rng(S)
+    n = rng.integers(50, 400, size=(S, NP))
+    sig = np.ones((S, NP))
+    se = 10.0 ** rng.uniform(-8, -1, size=(S, NP))
+    beta = se * rng.normal(size=(S, NP))
+    got = eng.abf_from_sstats(n, sig, beta, se, bfs)
+    std, raw, w = orc.abf_from_sstats(n, sig, beta, se, bfs, GL, GS)
+    _check(got, std, raw, w, np.ones(NP, bool))
