@@ -199,3 +199,30 @@ def test_perfect_fit_falls_back_to_general_path(eng, orc):
     keep = np.ones_like(ref, dtype=bool)
     keep[0, 4] = False
     _check(gpu[keep], ref[keep], "join")
+
+
+@pytest.mark.parametrize("S,N,P,nperm,wide", [
+    (1, 5, 1, 1, False),       # one wave with a tile, seven without; one permutation
+    (2, 63, 31, 15, False),    # one sample short of a step; a partial tile pair
+    (3, 64, 33, 16, False),    # whole steps; a second pair of one SNP
+    (4, 65, 300, 17, False),   # a second step of one sample; more tiles than waves
+    (5, 512, 70, 33, False),   # the most steps whose fragments and queues fit at S = 5
+    (6, 300, 40, 20, False),
+    (3, 513, 40, 20, False),   # one step more than the fused kernel holds
+    (3, 64, 40, 20, True),     # a genotype too large for its 32-bit digit pairs
+])
+def test_max_over_all_configurations_at_tile_edges(eng, orc, S, N, P, nperm, wide):
+    # the statistic is the exact one of the SNP with the maximum whichever
+    # kernel takes it, so the tolerance is that of the z and FP32 sums
+    hc = synth.plain(seed=41 + S, S=S, N=N, n_genes=2, snps_per_gene=P, frac_egenes=0.5)
+    if P > 31:
+        hc.genotypes[0, :, hc.pair_snp[hc.pair_offset[1] + 30]] = 2.0  # not estimable
+    if wide:
+        hc.genotypes[0, :, hc.pair_snp[hc.pair_offset[1] + 3]] *= 20.0
+    tables = engine.Rng(5).tables(hc.N, 2, nperm)
+    gene_table = np.array([0, 1], np.int32)
+    _say("[gpu] fused maximum S=%d N=%d P=%d nperm=%d wide=%d" % (S, N, P, nperm, wide))
+    gpu, prof = _run(eng, hc, tables, gene_table, "join", "all", True)
+    if N > 5:  # with few samples a perfect fit may move a gene to the general path
+        assert "pf_gemm_kernel" in prof and "perm_gather_kernel" not in prof
+    _check(gpu, _oracle(orc, hc, tables, gene_table, "join", "all", True), "join")
