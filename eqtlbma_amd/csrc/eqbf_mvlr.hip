@@ -1336,8 +1336,20 @@ struct HybTile {
   int32_t g, n;
 };
 
+/* A batch: second subgroups s2 .. s2 + nb - 1 of s1 (nb = 0: none), its groups of
+ * columns (ngm against the genotypes, then those against their squares) and base
+ * rows.  A column: its base row and the two presence words that it is masked with. */
+struct HybBatch {
+  int32_t s1, s2, nb, Q1, ngm, ng, nrow, pad;
+};
+struct HybColumn {
+  uint8_t row, wa, wb, pad;
+};
+
 struct HybPair {
   const HybTile* tiles;
+  const HybBatch* batches;
+  const HybColumn* columns; /* [batch][16 HYB_NG] */
   const uint64_t* pres;  /* [G][S][W] presence bits from the chunk's levels  */
   const uint64_t* presp; /* the same from the pairwise levels (may be pres) */
   const double* cp;
@@ -1351,20 +1363,17 @@ struct HybPair {
   double* sstats;
   int* flag;
   double fiterr;
-  int NSET, RSZ;
+  int NSET, RSZ, n_tiles, n_batch;
 };
 
 template <int Q1M>
-__device__ inline double hyb_quad(const double* __restrict__ Ai, const double (&u)[Q1M], const double (&v)[Q1M],
-                                  int Q1) {
+__device__ inline double hyb_quad(const double* __restrict__ Ai, const double (&u)[Q1M], const double (&v)[Q1M]) {
   double s = 0.0;
 #pragma unroll
   for (int a = 0; a < Q1M; ++a) {
-    if (a >= Q1) break;
     double r = 0.0;
 #pragma unroll
-    for (int b = 0; b < Q1M; ++b)
-      if (b < Q1) r += Ai[a * Q1M + b] * v[b];
+    for (int b = 0; b < Q1M; ++b) r += Ai[a * Q1M + b] * v[b];
     s += u[a] * r;
   }
   return s;
@@ -1384,258 +1393,341 @@ __global__ void __launch_bounds__(64) hyb_pres_kernel(const eqbf_chunk c, const 
   }
 }
 
-/* one lane per pair; the 64 pairs of a block belong to one gene.  The
- * individuals go by chunks of 64: the block stages the chunk's covariates
- * and levels in LDS (every lane reads them by broadcast), the presence bits
- * come as one uniform word a chunk, and each lane loads its genotypes eight
- * individuals at a time so that the loads overlap.  SPLIT: the pairwise
- * sets have presence bits of their own (hp.presp != hp.pres), so each
- * subgroup's first pass keeps its per-subgroup and pairwise sums apart. */
-template <int Q1M, class GT, bool SPLIT>
-__global__ void __launch_bounds__(64) hyb_pair_kernel(const eqbf_chunk c, const HybPair hp) {
-  __shared__ double st[(2 * (Q1M - 1) + 2) * 64];
+/* The sums of the pairs of a tile (64 pairs of one gene) for a first subgroup s1
+ * and nb second subgroups, as one FP64 matrix product of the tile's genotypes
+ * with columns over the individuals: covariates and levels with zeros where the
+ * sum's set has no member.  Columns: u1; u0 and x'y (with the first batch of
+ * s1); per second subgroup u12, x'y1, x'y2, u2; then, against the squared
+ * genotypes, the columns of ones of every set.
+ *
+ * Four waves: wave w takes the pairs 32 (w & 1) to + 31 and every second group of
+ * 16 columns, so that a genotype operand serves up to three groups and a column
+ * operand two tiles of 16 pairs.  The columns are not stored anywhere: a lane
+ * reads its base row (covariate, level or ones) from LDS and masks it with its
+ * set's presence word.  Rows are padded (HX_LD, HB_LD) so that the 16 rows x 2
+ * steps of a half wave fall into different banks.  The sums pass through LDS
+ * to the layout of one lane per pair for the closed forms.
+ *
+ * 48,000 pairs, 9 subgroups of 150, 3 covariates: 0.38 ms, of which the products
+ * at the FP64 matrix rate are 0.14; the rest is staging and the closed forms, which
+ * three workgroups per CU overlap only in part.  (One lane per pair with the sums
+ * of two second subgroups in registers had 750 waves for 1,024 SIMDs, read the
+ * genotypes S (S + 1) / 4 times and an LDS word per product: 2.35 ms.)  Past 8
+ * covariates the closed forms' registers allow two workgroups. */
+typedef double v4d __attribute__((ext_vector_type(4)));
+
+constexpr int HX_LD = 80, HB_LD = 66, HO_LD = 65;
+constexpr int HYB_NG = 6; /* groups of 16 columns a workgroup has at most */
+
+/* groups of a batch of nb second subgroups */
+int hyb_main_groups(int Q1, bool first, int nb) { return (Q1 + (first ? Q1 + 1 : 0) + nb * (2 * Q1 + 2) + 15) / 16; }
+int hyb_sq_groups(int nb) { return (2 + 2 * nb + 15) / 16; }
+
+/* Base rows: ones, covariates of s1 (own, pairwise), levels of s1 (own, pairwise),
+ * pairwise levels of the second subgroups.  Presence words: s1 by its own levels,
+ * s1, the second subgroups (by the pairwise levels), none, all. */
+HybColumn hyb_column(const HybBatch& t, int col) {
+  const int Q1 = t.Q1, Q = Q1 - 1, none = 2 + t.nb, all = 3 + t.nb;
+  const bool first = t.s2 == t.s1 + 1;
+  auto make = [](int row, int wa, int wb) { return HybColumn{(uint8_t)row, (uint8_t)wa, (uint8_t)wb, 0}; };
+  if (col >= 16 * t.ngm) {
+    const int k = col - 16 * t.ngm, b = (k - 2) / 2;
+    if (k < 2) return make(0, k, all);
+    if (b >= t.nb) return make(0, none, all);
+    return (k & 1) ? make(0, 2 + b, all) : make(0, 1, 2 + b);
+  }
+  int k = col;
+  if (k < Q1) return make(k ? Q + k : 0, 1, all);
+  k -= Q1;
+  if (first) {
+    if (k <= Q1) return make(k == Q1 ? 2 * Q + 1 : k, 0, all);
+    k -= Q1 + 1;
+  }
+  const int b = k / (2 * Q1 + 2), r = k % (2 * Q1 + 2);
+  if (b >= t.nb) return make(0, none, all);
+  if (r < Q1) return make(r ? Q + r : 0, 1, 2 + b);
+  if (r < Q1 + 2) return make(r == Q1 ? 2 * Q + 2 : 2 * Q + 3 + b, 1, 2 + b);
+  return make(r > Q1 + 2 ? Q + r - Q1 - 2 : 0, 2 + b, all);
+}
+
+/* gene of each pair, -1 where the gene or the SNP is missing from a subgroup:
+ * gene.cpp:314-321 skips such a pair, which has no sample size and no statistics */
+__global__ void __launch_bounds__(64) hyb_skip_kernel(const eqbf_chunk c, const HybPair hp) {
   const HybTile tl = hp.tiles[blockIdx.x];
-  const int g = tl.g, lane = threadIdx.x;
-  const bool act = lane < tl.n;
-  const int64_t p = tl.p0 + (act ? lane : 0);
-  const int64_t NP = c.n_pairs;
-  const int S = c.n_subgroups, N = c.n_samples, QM = c.n_covars_max;
-  const int W = (N + 63) >> 6;
-  const int64_t snp = c.pair_snp[p];
-  bool gene_ok = true, ok = act;
-  for (int s = 0; s < S; ++s) {
-    gene_ok &= c.gene_in_sbgrp[(int64_t)g * S + s] != 0;
-    ok &= c.snp_in_sbgrp[snp * S + s] != 0;
-  }
-  ok &= gene_ok;
-  if (gene_ok) {
-    const uint64_t* pres = hp.pres + (int64_t)g * S * W;
-    const uint64_t* presp = hp.presp + (int64_t)g * S * W;
-    const int npr = S * (S - 1) / 2;
-    const int RSZ = hp.RSZ;
-    const double* R = hp.rec + (int64_t)g * hp.NSET * RSZ;
-    const double f = hp.fiterr;
-    int pi = 0;
-    for (int s1 = 0; s1 < S; ++s1) {
-      const int Q1 = min(max(c.covar_count[s1], 0), QM) + 1, Q = Q1 - 1;
-      const double* cov0 = c.covars + (int64_t)s1 * QM * N;
-      const double* covp = hp.cp + (int64_t)s1 * QM * N;
-      const double* y = c.explevels + ((int64_t)g * S + s1) * N;
-      const GT* xb = (const GT*)c.genotypes + (int64_t)c.geno_set_of_sbgrp[s1] * c.geno_set_stride + snp;
-      const int64_t ld = c.geno_ld;
-      double u0[Q1M], u1[Q1M], sxx = 0.0, sxxp = 0.0, sxy = 0.0;
-#pragma unroll
-      for (int a = 0; a < Q1M; ++a) u0[a] = u1[a] = 0.0;
-      for (int c0 = 0; c0 < N; c0 += 64) {
-        const int n = min(64, N - c0);
-        __syncthreads();
-        if (lane < n) {
-          for (int q = 0; q < Q; ++q) {
-            st[q * 64 + lane] = cov0[(int64_t)q * N + c0 + lane];
-            st[(Q + q) * 64 + lane] = covp[(int64_t)q * N + c0 + lane];
-          }
-          st[2 * Q * 64 + lane] = y[c0 + lane];
-        }
-        __syncthreads();
-        const uint64_t m = pres[(int64_t)s1 * W + (c0 >> 6)];
-        const uint64_t mp = SPLIT ? presp[(int64_t)s1 * W + (c0 >> 6)] : m;
-        for (int j0 = 0; j0 < n; j0 += 8) {
-          double xv[8];
-#pragma unroll
-          for (int k = 0; k < 8; ++k) xv[k] = (ok && j0 + k < n) ? (double)xb[(int64_t)(c0 + j0 + k) * ld] : 0.0;
-#pragma unroll
-          for (int k = 0; k < 8; ++k) {
-            const int j = j0 + k;
-            const bool in0 = (m >> j) & 1ull, inp = (mp >> j) & 1ull;
-            if (j >= n || !(in0 || inp)) continue;
-            const double x = xv[k];
-            if (!SPLIT) { /* one set: the per-subgroup and pairwise sums together */
-              sxx += x * x;
-              sxy += x * st[2 * Q * 64 + j];
-              u0[0] += x;
-              u1[0] += x;
-#pragma unroll
-              for (int a = 1; a < Q1M; ++a)
-                if (a < Q1) {
-                  u0[a] += st[(a - 1) * 64 + j] * x;
-                  u1[a] += st[(Q + a - 1) * 64 + j] * x;
-                }
-              continue;
-            }
-            if (in0) {
-              sxx += x * x;
-              sxy += x * st[2 * Q * 64 + j];
-              u0[0] += x;
-#pragma unroll
-              for (int a = 1; a < Q1M; ++a)
-                if (a < Q1) u0[a] += st[(a - 1) * 64 + j] * x;
-            }
-            if (inp) {
-              sxxp += x * x;
-              u1[0] += x;
-#pragma unroll
-              for (int a = 1; a < Q1M; ++a)
-                if (a < Q1) u1[a] += st[(Q + a - 1) * 64 + j] * x;
-            }
-          }
-        }
-      }
-      const double* R0 = R + (int64_t)s1 * RSZ;
-      const double* R1 = R + (int64_t)(S + s1) * RSZ;
-      const double k0 = sxx - hyb_quad<Q1M>(R0, u0, u0, Q1);
-      double xty = sxy;
-#pragma unroll
-      for (int a = 0; a < Q1M; ++a)
-        if (a < Q1) xty -= u0[a] * R0[2 * Q1M * Q1M + a];
-      const double rss0 = R0[2 * Q1M * Q1M + 2 * Q1M], n0 = R0[2 * Q1M * Q1M + 2 * Q1M + 1];
-      const double rss1 = rss0 - xty * xty / k0;
-      const double sg = f * rss1 / n0 + (1.0 - f) * rss0 / n0;
-      if (ok) {
-        hp.b[(int64_t)s1 * NP + p] = xty / k0;
-        hp.Sig[(int64_t)(s1 * S + s1) * NP + p] = sg;
-        hp.Vg[(int64_t)(s1 * S + s1) * NP + p] = sg / k0;
-      }
-      /* w1 = A1^-1 u1, k1: the genotype column of M1^-1 is (-w1, 1) / k1 */
-      double w1[Q1M];
-#pragma unroll
-      for (int a = 0; a < Q1M; ++a) {
-        double r = 0.0;
-#pragma unroll
-        for (int b2 = 0; b2 < Q1M; ++b2)
-          if (a < Q1 && b2 < Q1) r += R1[a * Q1M + b2] * u1[b2];
-        w1[a] = r;
-      }
-      double k1 = SPLIT ? sxxp : sxx;
-#pragma unroll
-      for (int a = 0; a < Q1M; ++a)
-        if (a < Q1) k1 -= u1[a] * w1[a];
-      const double* yp1 = hp.yp + ((int64_t)g * S + s1) * N;
-      /* PW second subgroups per pass over the individuals (the genotypes
-       * are read once for them); a missing second one repeats the first
-       * and is not written */
-      constexpr int PW = Q1M <= 8 ? 2 : 1;
-      for (int s2 = s1 + 1; s2 < S; s2 += PW) {
-        const int nb = min(PW, S - s2);
-        const double* yp2[PW];
-        int sb[PW];
-#pragma unroll
-        for (int b = 0; b < PW; ++b) {
-          sb[b] = s2 + min(b, nb - 1);
-          yp2[b] = hp.yp + ((int64_t)g * S + sb[b]) * N;
-        }
-        double u12[PW][Q1M], u2[PW][Q1M], sxx12[PW], sxx2[PW], sy1[PW], sy2[PW];
-#pragma unroll
-        for (int b = 0; b < PW; ++b) {
-          sxx12[b] = sxx2[b] = sy1[b] = sy2[b] = 0.0;
-#pragma unroll
-          for (int a = 0; a < Q1M; ++a) u12[b][a] = u2[b][a] = 0.0;
-        }
-        for (int c0 = 0; c0 < N; c0 += 64) {
-          const int n = min(64, N - c0);
-          __syncthreads();
-          if (lane < n) {
-            for (int q = 0; q < Q; ++q) st[q * 64 + lane] = covp[(int64_t)q * N + c0 + lane];
-            st[Q * 64 + lane] = yp1[c0 + lane];
-#pragma unroll
-            for (int b = 0; b < PW; ++b) st[(Q + 1 + b) * 64 + lane] = yp2[b][c0 + lane];
-          }
-          __syncthreads();
-          const uint64_t m1 = presp[(int64_t)s1 * W + (c0 >> 6)];
-          uint64_t m2[PW], any = 0ull;
-#pragma unroll
-          for (int b = 0; b < PW; ++b) {
-            m2[b] = presp[(int64_t)sb[b] * W + (c0 >> 6)];
-            any |= m2[b];
-          }
-          for (int j0 = 0; j0 < n; j0 += 8) {
-            double xv[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) xv[k] = (ok && j0 + k < n) ? (double)xb[(int64_t)(c0 + j0 + k) * ld] : 0.0;
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-              const int j = j0 + k;
-              if (j >= n || !((any >> j) & 1ull)) continue;
-              const double x = xv[k];
-              double cv[Q1M];
-              cv[0] = 1.0;
-#pragma unroll
-              for (int a = 1; a < Q1M; ++a) cv[a] = (a < Q1) ? st[(a - 1) * 64 + j] : 0.0;
-              const bool in1 = (m1 >> j) & 1ull;
-#pragma unroll
-              for (int b = 0; b < PW; ++b) {
-                if (!((m2[b] >> j) & 1ull)) continue;
-                sxx2[b] += x * x;
-#pragma unroll
-                for (int a = 0; a < Q1M; ++a) u2[b][a] += cv[a] * x;
-                if (in1) {
-                  sxx12[b] += x * x;
-                  sy1[b] += x * st[Q * 64 + j];
-                  sy2[b] += x * st[(Q + 1 + b) * 64 + j];
-#pragma unroll
-                  for (int a = 0; a < Q1M; ++a) u12[b][a] += cv[a] * x;
-                }
-              }
-            }
-          }
-        }
-#pragma unroll
-        for (int b = 0; b < PW; ++b) {
-          if (b >= nb) break;
-          const int s2b = s2 + b, pib = pi + b;
-          const double* R2 = R + (int64_t)(2 * S + pib) * RSZ;
-          const double* R3 = R + (int64_t)(2 * S + npr + pib) * RSZ;
-          const double n12 = R2[2 * Q1M * Q1M + 2 * Q1M + 1];
-          if (ok && !(n12 > 0.0)) atomicOr(hp.flag, FLAG_HYB_NO_COMMON);
-          const double k12 = sxx12[b] - hyb_quad<Q1M>(R2, u12[b], u12[b], Q1);
-          double xty1 = sy1[b], xty2 = sy2[b];
-#pragma unroll
-          for (int a = 0; a < Q1M; ++a)
-            if (a < Q1) {
-              xty1 -= u12[b][a] * R2[2 * Q1M * Q1M + a];
-              xty2 -= u12[b][a] * R2[2 * Q1M * Q1M + Q1M + a];
-            }
-          const double s12 = R2[2 * Q1M * Q1M + 2 * Q1M] / n12 - f * xty1 * xty2 / (k12 * n12);
-          double w2[Q1M];
-#pragma unroll
-          for (int a = 0; a < Q1M; ++a) {
-            double r = 0.0;
-#pragma unroll
-            for (int b2 = 0; b2 < Q1M; ++b2)
-              if (a < Q1 && b2 < Q1) r += R3[a * Q1M + b2] * u2[b][b2];
-            w2[a] = r;
-          }
-          double k2 = sxx2[b], wu = 0.0;
-#pragma unroll
-          for (int a = 0; a < Q1M; ++a)
-            if (a < Q1) {
-              k2 -= u2[b][a] * w2[a];
-              wu += w1[a] * u12[b][a] + u12[b][a] * w2[a];
-            }
-          const double aw = hyb_quad<Q1M>(R2 + Q1M * Q1M, w1, w2, Q1);
-          const double a11 = (aw - wu + sxx12[b]) / (k1 * k2);
-          if (ok) {
-            hp.Sig[(int64_t)(s1 * S + s2b) * NP + p] = s12;
-            hp.Sig[(int64_t)(s2b * S + s1) * NP + p] = s12;
-            hp.Vg[(int64_t)(s1 * S + s2b) * NP + p] = s12 * a11;
-            hp.Vg[(int64_t)(s2b * S + s1) * NP + p] = s12 * a11;
-          }
-        }
-        pi += nb;
-      }
-    }
-  }
-  if (!act) return;
-  if (ok) {
-    hp.pgene[p] = g;
-    return;
-  }
-  /* gene.cpp:314-321 skips the pair: no sample size, no statistics */
+  const int lane = threadIdx.x, S = c.n_subgroups;
+  if (lane >= tl.n) return;
+  const int64_t p = tl.p0 + lane, NP = c.n_pairs, snp = c.pair_snp[p];
+  bool ok = true;
+  for (int s = 0; s < S; ++s)
+    ok &= c.gene_in_sbgrp[(int64_t)tl.g * S + s] != 0 && c.snp_in_sbgrp[snp * S + s] != 0;
+  hp.pgene[p] = ok ? tl.g : -1;
+  if (ok) return;
   for (int s = 0; s < S; ++s) {
     hp.n_out[(int64_t)s * NP + p] = 0;
     if (hp.sstats)
       for (int k = 0; k < 5; ++k) hp.sstats[((int64_t)k * S + s) * NP + p] = NAN;
   }
-  hp.pgene[p] = -1;
+}
+
+template <int Q1M, class GT>
+__global__ void __launch_bounds__(256, Q1M > 8 ? 2 : 3) hyb_pair_kernel(const eqbf_chunk c, const HybPair hp) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ uint64_t words[2 + 15 + 2];
+  __shared__ unsigned long long badm;
+  GT* const Xs = (GT*)smem;                                       /* [64][HX_LD] */
+  double* const base = (double*)(smem + 64 * HX_LD * sizeof(GT)); /* [rows][HB_LD] */
+  double* const sums = (double*)smem;                             /* [columns][HO_LD], after them */
+  const int n_items = hp.n_tiles * hp.n_batch, per = (n_items + 7) / 8;
+  /* the batches of a tile follow one another on one XCD */
+  const int item = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per || item >= n_items) return;
+  const HybBatch bt = hp.batches[item % hp.n_batch];
+  const HybTile tl = hp.tiles[item / hp.n_batch];
+  const int g = tl.g, s1 = bt.s1, nb = bt.nb;
+  const bool first = bt.s2 == s1 + 1;
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool act = lane < tl.n;
+  const int64_t p = tl.p0 + (act ? lane : 0);
+  const int64_t NP = c.n_pairs;
+  const int S = c.n_subgroups, N = c.n_samples, QM = c.n_covars_max;
+  const int W = (N + 63) >> 6;
+  const bool ok = hp.pgene[p] >= 0 && act;
+  const int64_t snp = c.pair_snp[p];
+  const int Q1 = bt.Q1, Q = Q1 - 1, ngm = bt.ngm, ng = bt.ng, nrow = bt.nrow;
+  const double* cov0 = c.covars + (int64_t)s1 * QM * N;
+  const double* covp = hp.cp + (int64_t)s1 * QM * N;
+  const double* y0 = c.explevels + ((int64_t)g * S + s1) * N;
+  const double* yp1 = hp.yp + ((int64_t)g * S + s1) * N;
+  const double* yp2 = hp.yp + ((int64_t)g * S + bt.s2) * N;
+  const GT* xb = (const GT*)c.genotypes + (int64_t)c.geno_set_of_sbgrp[s1] * c.geno_set_stride + snp;
+  const int64_t ld = c.geno_ld;
+  auto base_row = [&](int row) {
+    const double* r = cov0 + (int64_t)max(row - 1, 0) * N;
+    r = row > Q ? covp + (int64_t)(row - Q - 1) * N : r;
+    r = row == 2 * Q + 1 ? y0 : r;
+    r = row == 2 * Q + 2 ? yp1 : r;
+    r = row > 2 * Q + 2 ? yp2 + (int64_t)(row - 2 * Q - 3) * N : r;
+    return row == 0 ? y0 : r; /* read, not used */
+  };
+  auto word_at = [&](int k, int w) -> uint64_t {
+    if (k >= 2 + nb) return k == 2 + nb ? 0ull : ~0ull;
+    if (k == 0) return hp.pres[((int64_t)g * S + s1) * W + w];
+    return hp.presp[((int64_t)g * S + (k == 1 ? s1 : bt.s2 + k - 2)) * W + w];
+  };
+  const int half = wv & 1, kl = lane >> 4, pl = lane & 15;
+  v4d acc[HYB_NG / 2][2];
+  const HybColumn* const cols = hp.columns + (int64_t)(item % hp.n_batch) * (16 * HYB_NG);
+  int row[HYB_NG / 2], wa[HYB_NG / 2], wb[HYB_NG / 2];
+#pragma unroll
+  for (int j = 0; j < HYB_NG / 2; ++j) {
+    acc[j][0] = acc[j][1] = v4d{0.0, 0.0, 0.0, 0.0};
+    const HybColumn cl = cols[min((wv >> 1) + 2 * j, ng - 1) * 16 + pl];
+    row[j] = cl.row * HB_LD;
+    wa[j] = cl.wa;
+    wb[j] = cl.wb;
+  }
+  if (tid == 0) badm = 0ull;
+  /* a chunk of 64 individuals, read while the one before is worked on: 16 of
+   * them of the lane's pair, the lane's of every fourth base row, and a presence
+   * word (past N the last individual once more: no set has it) */
+  constexpr int BR = (2 * Q1M + 1 + 15 + 3) / 4;
+  GT xv[16];
+  double bv[BR];
+  uint64_t wd = 0ull;
+  auto load = [&](int c0) {
+#pragma unroll
+    for (int k = 0; k < 16; ++k) xv[k] = xb[(int64_t)min(c0 + 16 * wv + k, N - 1) * ld];
+#pragma unroll
+    for (int k = 0; k < BR; ++k)
+      if (wv + 4 * k < nrow) bv[k] = base_row(wv + 4 * k)[min(c0 + lane, N - 1)];
+    if (tid < 4 + nb) wd = word_at(tid, c0 >> 6);
+  };
+  bool bad = false; /* a genotype that is not finite: masked columns don't keep it out */
+  load(0);
+  for (int c0 = 0; c0 < N; c0 += 64) {
+    const int n = min(64, N - c0);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      Xs[(16 * wv + k) * HX_LD + lane] = xv[k];
+      bad |= !__builtin_isfinite(xv[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < BR; ++k)
+      if (wv + 4 * k < nrow)
+        base[(wv + 4 * k) * HB_LD + lane] = wv + 4 * k == 0 ? 1.0 : bv[k];
+    if (tid < 4 + nb) words[tid] = wd;
+    __syncthreads();
+    if (c0 + 64 < N) load(c0 + 64);
+    uint64_t m[HYB_NG / 2];
+#pragma unroll
+    for (int j = 0; j < HYB_NG / 2; ++j) m[j] = (words[wa[j]] & words[wb[j]]) >> kl;
+    const GT* xr = Xs + kl * HX_LD + half * 32 + pl;
+    const double* br = base + kl;
+    /* four steps of J groups at a time, without a branch between their reads; SQ:
+     * the last group's columns meet the squares (a wave has one at most) */
+    auto steps = [&](auto J, auto SQ) {
+      for (int k0 = 0; k0 < n; k0 += 16) {
+        GT x0[4], x1[4];
+        double v[4][J.value];
+        int w[J.value];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          x0[k] = xr[(k0 + 4 * k) * HX_LD];
+          x1[k] = xr[(k0 + 4 * k) * HX_LD + 16];
+#pragma unroll
+          for (int j = 0; j < J.value; ++j) v[k][j] = br[row[j] + k0 + 4 * k];
+        }
+#pragma unroll
+        for (int j = 0; j < J.value; ++j) {
+          w[j] = (int)m[j];
+          m[j] >>= 16;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const double b0 = (double)x0[k], b1 = (double)x1[k];
+#pragma unroll
+          for (int j = 0; j < J.value; ++j) {
+            const int keep = __builtin_amdgcn_sbfe(w[j], 4 * k, 1);
+            const double av = __hiloint2double(__double2hiint(v[k][j]) & keep, __double2loint(v[k][j]) & keep);
+            const bool sq = SQ.value && j == J.value - 1;
+            acc[j][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, sq ? b0 * b0 : b0, acc[j][0], 0, 0, 0);
+            acc[j][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, sq ? b1 * b1 : b1, acc[j][1], 0, 0, 0);
+          }
+        }
+      }
+    };
+    const int nj = (ng - (wv >> 1) + 1) >> 1; /* groups of this wave */
+    using std::integral_constant;
+    if ((wv >> 1) + 2 * (nj - 1) >= ngm) {
+      if (nj == 1) steps(integral_constant<int, 1>(), std::true_type());
+      if (nj == 2) steps(integral_constant<int, 2>(), std::true_type());
+      if (nj == 3) steps(integral_constant<int, 3>(), std::true_type());
+    } else {
+      if (nj == 1) steps(integral_constant<int, 1>(), std::false_type());
+      if (nj == 2) steps(integral_constant<int, 2>(), std::false_type());
+      if (nj == 3) steps(integral_constant<int, 3>(), std::false_type());
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < HYB_NG / 2; ++j) {
+    const int gr = (wv >> 1) + 2 * j;
+    if (gr < ng) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          sums[(gr * 16 + kl + 4 * r) * HO_LD + half * 32 + 16 * u + pl] = acc[j][u][r];
+    }
+  }
+  if (__any(bad)) {
+    const uint64_t bal = __ballot(bad);
+    if (lane == 0) atomicOr(&badm, (unsigned long long)bal);
+  }
+  __syncthreads();
+  if (badm != 0ull) { /* such pairs: the members of each set only, one by one */
+    if ((badm >> lane) & 1ull)
+      for (int col = wv; col < ng * 16; col += 4) {
+        const HybColumn cl = cols[col];
+        double a = 0.0;
+        for (int i = 0; i < N; ++i)
+          if (((word_at(cl.wa, i >> 6) & word_at(cl.wb, i >> 6)) >> (i & 63)) & 1ull) {
+            const double x = (double)xb[(int64_t)i * ld];
+            a += (cl.row == 0 ? 1.0 : base_row(cl.row)[i]) * (col >= 16 * ngm ? x * x : x);
+          }
+        sums[col * HO_LD + lane] = a;
+      }
+    __syncthreads();
+  }
+  /* closed forms, one lane per pair; wave w takes every fourth second subgroup */
+  const int npr = S * (S - 1) / 2, RSZ = hp.RSZ;
+  const double* R = hp.rec + (int64_t)g * hp.NSET * RSZ;
+  const double f = hp.fiterr;
+  auto col_at = [&](int col) { return sums[col * HO_LD + lane]; };
+  /* records are zero past Q1, and so is what goes with them: no branches */
+  auto take = [&](int col, double (&u)[Q1M]) {
+#pragma unroll
+    for (int a = 0; a < Q1M; ++a) {
+      const double v = col_at(col + min(a, Q1 - 1));
+      u[a] = a < Q1 ? v : 0.0;
+    }
+  };
+  auto mul = [&](const double* __restrict__ Ai, const double (&u)[Q1M], double (&w)[Q1M]) {
+#pragma unroll
+    for (int a = 0; a < Q1M; ++a) {
+      double r = 0.0;
+#pragma unroll
+      for (int b = 0; b < Q1M; ++b) r += Ai[a * Q1M + b] * u[b];
+      w[a] = r;
+    }
+  };
+  const int sq = 16 * ngm;
+  /* w1 = A1^-1 u1, k1: the genotype column of M1^-1 is (-w1, 1) / k1 */
+  double w1[Q1M], k1 = col_at(sq + 1);
+  {
+    double u1[Q1M];
+    take(0, u1);
+    mul(R + (int64_t)(S + s1) * RSZ, u1, w1);
+#pragma unroll
+    for (int a = 0; a < Q1M; ++a)
+      k1 -= u1[a] * w1[a];
+  }
+  if (first && wv == 3) {
+    const double* R0 = R + (int64_t)s1 * RSZ;
+    double u0[Q1M];
+    take(Q1, u0);
+    const double k0 = col_at(sq) - hyb_quad<Q1M>(R0, u0, u0);
+    double xty = col_at(2 * Q1);
+#pragma unroll
+    for (int a = 0; a < Q1M; ++a)
+      xty -= u0[a] * R0[2 * Q1M * Q1M + a];
+    const double rss0 = R0[2 * Q1M * Q1M + 2 * Q1M], n0 = R0[2 * Q1M * Q1M + 2 * Q1M + 1];
+    const double rss1 = rss0 - xty * xty / k0;
+    const double sg = f * rss1 / n0 + (1.0 - f) * rss0 / n0;
+    if (ok) {
+      hp.b[(int64_t)s1 * NP + p] = xty / k0;
+      hp.Sig[(int64_t)(s1 * S + s1) * NP + p] = sg;
+      hp.Vg[(int64_t)(s1 * S + s1) * NP + p] = sg / k0;
+    }
+  }
+  const int col0 = Q1 + (first ? Q1 + 1 : 0);
+  for (int b = wv; b < nb; b += 4) {
+    const int s2 = bt.s2 + b, pi = s1 * S - s1 * (s1 + 1) / 2 + s2 - s1 - 1;
+    const double* R2 = R + (int64_t)(2 * S + pi) * RSZ;
+    const double* R3 = R + (int64_t)(2 * S + npr + pi) * RSZ;
+    const double n12 = R2[2 * Q1M * Q1M + 2 * Q1M + 1];
+    if (ok && !(n12 > 0.0)) atomicOr(hp.flag, FLAG_HYB_NO_COMMON);
+    const int cb = col0 + b * (2 * Q1 + 2);
+    double u12[Q1M];
+    take(cb, u12);
+    const double sxx12 = col_at(sq + 2 + 2 * b);
+    const double k12 = sxx12 - hyb_quad<Q1M>(R2, u12, u12);
+    double xty1 = col_at(cb + Q1), xty2 = col_at(cb + Q1 + 1);
+#pragma unroll
+    for (int a = 0; a < Q1M; ++a) {
+      xty1 -= u12[a] * R2[2 * Q1M * Q1M + a];
+      xty2 -= u12[a] * R2[2 * Q1M * Q1M + Q1M + a];
+    }
+    const double s12 = R2[2 * Q1M * Q1M + 2 * Q1M] / n12 - f * xty1 * xty2 / (k12 * n12);
+    double u2[Q1M], w2[Q1M];
+    take(cb + Q1 + 2, u2);
+    mul(R3, u2, w2);
+    double k2 = col_at(sq + 3 + 2 * b), wu = 0.0;
+#pragma unroll
+    for (int a = 0; a < Q1M; ++a) {
+      k2 -= u2[a] * w2[a];
+      wu += w1[a] * u12[a] + u12[a] * w2[a];
+    }
+    const double aw = hyb_quad<Q1M>(R2 + Q1M * Q1M, w1, w2);
+    const double a11 = (aw - wu + sxx12) / (k1 * k2);
+    if (ok) {
+      hp.Sig[(int64_t)(s1 * S + s2) * NP + p] = s12;
+      hp.Sig[(int64_t)(s2 * S + s1) * NP + p] = s12;
+      hp.Vg[(int64_t)(s1 * S + s2) * NP + p] = s12 * a11;
+      hp.Vg[(int64_t)(s2 * S + s1) * NP + p] = s12 * a11;
+    }
+  }
 }
 
 /* per (pair, configuration): Vg^-1, Vg^-1 t, t = gamma o sqrt(diag Sigma),
@@ -1731,14 +1823,44 @@ int hybrid_run_sm(eqbf_ctx* ctx, const eqbf_chunk& c, const eqbf_hybrid_opts* o,
   const int RSZ = 2 * Q1M * Q1M + 2 * Q1M + 2;
   /* tiles of at most 64 pairs of one gene */
   std::vector<int64_t> off(G + 1);
+  std::vector<int32_t> q1(S);
   EQBF_HIP(ctx, hipMemcpyAsync(off.data(), c.pair_offset, (G + 1) * sizeof(int64_t), hipMemcpyDeviceToHost, st));
+  EQBF_HIP(ctx, hipMemcpyAsync(q1.data(), c.covar_count, S * sizeof(int32_t), hipMemcpyDeviceToHost, st));
   EQBF_HIP(ctx, hipStreamSynchronize(st));
   std::vector<HybTile> tiles;
   for (int g = 0; g < G; ++g)
     for (int64_t p0 = off[g]; p0 < off[g + 1]; p0 += 64)
       tiles.push_back(HybTile{p0, g, (int32_t)std::min<int64_t>(64, off[g + 1] - p0)});
   if (tiles.empty()) return EQBF_OK;
-  HybTile* dtiles = (HybTile*)ctx_buf(ctx, "hyb_tiles", tiles.size() * sizeof(HybTile));
+  /* batches of second subgroups: as many as a workgroup's groups of columns
+   * hold, of even size */
+  std::vector<HybBatch> batches;
+  std::vector<HybColumn> columns;
+  size_t lds = 0;
+  for (int s1 = 0; s1 < S; ++s1) {
+    const int Q1 = std::min(std::max(q1[s1], 0), c.n_covars_max) + 1, n2 = S - 1 - s1;
+    int nb_max = 15;
+    while (hyb_main_groups(Q1, true, nb_max) + hyb_sq_groups(nb_max) > HYB_NG) --nb_max;
+    const int k = std::max(1, (n2 + nb_max - 1) / nb_max);
+    for (int b = 0; b < k; ++b) {
+      const int lo = s1 + 1 + n2 * b / k, nb = s1 + 1 + n2 * (b + 1) / k - lo;
+      const int ngm = hyb_main_groups(Q1, b == 0, nb);
+      batches.push_back(HybBatch{s1, lo, nb, Q1, ngm, ngm + hyb_sq_groups(nb), 2 * Q1 + 1 + nb, 0});
+      const HybBatch& t = batches.back();
+      for (int col = 0; col < 16 * HYB_NG; ++col)
+        columns.push_back(col < 16 * t.ng ? hyb_column(t, col) : HybColumn{});
+      const size_t in = 64 * HX_LD * (c.geno_dtype == EQBF_F32 ? 4 : 8) + (size_t)t.nrow * HB_LD * 8;
+      lds = std::max(lds, std::max(in, (size_t)16 * t.ng * HO_LD * 8));
+    }
+  }
+  const size_t tb = tiles.size() * sizeof(HybTile), btb = batches.size() * sizeof(HybBatch);
+  std::vector<unsigned char> lists(tb + btb + columns.size() * sizeof(HybColumn));
+  memcpy(lists.data(), tiles.data(), tb);
+  memcpy(lists.data() + tb, batches.data(), btb);
+  memcpy(lists.data() + tb + btb, columns.data(), lists.size() - tb - btb);
+  if (tiles.size() * batches.size() > (size_t)INT32_MAX - 8)
+    return ctx_fail(ctx, EQBF_ERR_UNSUPPORTED, "too many pairs in a chunk for --error hybrid");
+  HybTile* dtiles = (HybTile*)ctx_buf(ctx, "hyb_tiles", lists.size());
   double* rec = (double*)ctx_buf(ctx, "hyb_rec", (size_t)G * NSET * RSZ * sizeof(double));
   double* bb = (double*)ctx_buf(ctx, "hyb_b", (size_t)S * NP * sizeof(double));
   double* sig = (double*)ctx_buf(ctx, "hyb_sig", (size_t)S * S * NP * sizeof(double));
@@ -1750,7 +1872,7 @@ int hybrid_run_sm(eqbf_ctx* ctx, const eqbf_chunk& c, const eqbf_hybrid_opts* o,
   uint64_t* dmask = (uint64_t*)ctx_buf(ctx, "mv_masks", hm.size() * sizeof(uint64_t));
   if (!dtiles || !rec || !bb || !sig || !vg || !pgene || !dmask)
     return ctx_fail(ctx, EQBF_ERR_HIP, "allocating hybrid buffers failed");
-  EQBF_HIP(ctx, hipMemcpyAsync(dtiles, tiles.data(), tiles.size() * sizeof(HybTile), hipMemcpyHostToDevice, st));
+  EQBF_HIP(ctx, hipMemcpyAsync(dtiles, lists.data(), lists.size(), hipMemcpyHostToDevice, st));
   EQBF_HIP(ctx, hipMemcpyAsync(dmask, hm.data(), hm.size() * sizeof(uint64_t), hipMemcpyHostToDevice, st));
   EQBF_HIP(ctx, hipStreamSynchronize(st)); /* the host vectors go out of scope */
   HybGene hg;
@@ -1773,6 +1895,10 @@ int hybrid_run_sm(eqbf_ctx* ctx, const eqbf_chunk& c, const eqbf_hybrid_opts* o,
   if (split) hipLaunchKernelGGL(hyb_pres_kernel, dim3(G, S), dim3(64), 0, st, c, hg.yp, presp, W);
   HybPair hp;
   hp.tiles = dtiles;
+  hp.batches = (const HybBatch*)(dtiles + tiles.size());
+  hp.columns = (const HybColumn*)(hp.batches + batches.size());
+  hp.n_tiles = (int)tiles.size();
+  hp.n_batch = (int)batches.size();
   hp.pres = pres;
   hp.presp = presp;
   hp.cp = hg.cp;
@@ -1788,17 +1914,14 @@ int hybrid_run_sm(eqbf_ctx* ctx, const eqbf_chunk& c, const eqbf_hybrid_opts* o,
   hp.fiterr = o->fiterr;
   hp.NSET = NSET;
   hp.RSZ = RSZ;
+  hipLaunchKernelGGL(hyb_skip_kernel, dim3((unsigned)tiles.size()), dim3(64), 0, st, c, hp);
   {
     ProfScope ps(ctx, "hyb_pair_kernel", st);
-    const dim3 grid((unsigned)tiles.size());
-    if (c.geno_dtype == EQBF_F32 && split)
-      hipLaunchKernelGGL((hyb_pair_kernel<Q1M, float, true>), grid, dim3(64), 0, st, c, hp);
-    else if (c.geno_dtype == EQBF_F32)
-      hipLaunchKernelGGL((hyb_pair_kernel<Q1M, float, false>), grid, dim3(64), 0, st, c, hp);
-    else if (split)
-      hipLaunchKernelGGL((hyb_pair_kernel<Q1M, double, true>), grid, dim3(64), 0, st, c, hp);
+    const dim3 grid((unsigned)((tiles.size() * batches.size() + 7) / 8 * 8));
+    if (c.geno_dtype == EQBF_F32)
+      hipLaunchKernelGGL((hyb_pair_kernel<Q1M, float>), grid, dim3(256), lds, st, c, hp);
     else
-      hipLaunchKernelGGL((hyb_pair_kernel<Q1M, double, false>), grid, dim3(64), 0, st, c, hp);
+      hipLaunchKernelGGL((hyb_pair_kernel<Q1M, double>), grid, dim3(256), lds, st, c, hp);
   }
   EQBF_HIP(ctx, hipGetLastError());
   return mv_rows_run<SM>(ctx, c, o->bfs, out, st, [&](int64_t c0, int nb, double* par, int PSZ, int64_t pair_blocks) {

@@ -114,3 +114,24 @@ def test_hybrid_no_common_individual_is_an_error(eng):
     _say("[gpu] hybrid subgroups without a common individual")
     with pytest.raises(engine.EngineError, match="no individuals in common"):
         eng.assoc_hybrid(hc, "gen", 0.5)
+
+
+@pytest.mark.parametrize("S,N,P,Q,n_genes", [
+    (1, 64, 64, 0, 1),    # no second subgroup; one whole chunk of individuals, one whole tile
+    (2, 65, 65, 3, 2),    # a second chunk and a second tile of one
+    (9, 129, 3, 3, 1),    # two batches for the first subgroup
+    (16, 63, 2, 0, 1),    # the most second subgroups of a batch
+    (4, 127, 2, 16, 1),   # the most covariates: one second subgroup a batch
+    (7, 70, 33, 7, 1),    # the middle size of the covariate blocks
+])
+def test_hybrid_tile_and_batch_edges(eng, orc, S, N, P, Q, n_genes):
+    # an individual without levels has a NaN genotype: no set holds it, so it may
+    # reach no sum of any pair
+    hc = synth.hybrid(seed=300 + S, S=S, N=N, P=P, Q=Q, n_genes=n_genes, miss=0.05)
+    hc.explevels[0, :, N - 1] = np.nan
+    ref = orc.assoc_hybrid(hc, "gen", 0.5, GL, GS)
+    hc.genotypes[0, N - 1, hc.pair_snp[0]] = np.nan
+    _say("[gpu] hybrid edges S=%d N=%d P=%d Q=%d" % (S, N, P, Q))
+    gpu = eng.assoc_hybrid(hc, "gen", 0.5)
+    _close(gpu.raw, ref.raw, "raw")
+    _close(gpu.w, ref.w, "w")
