@@ -24,9 +24,9 @@
  * M^-1 eVb comes from one solve instead of an explicit inverse.
  *
  * Kernels (one chunk):
- *   mvlr_prep_kernel   one wave per gene: common members, basis of
+ *   mvlr_prep_kernel   one workgroup per gene: common members, basis of
  *                      [1, covariates], y~_s, Y~'Y~, Sigma0 and Sigma0^-1
- *   mvlr_sums_kernel   one thread per pair: k and b (FP64 sums over members)
+ *   mvlr_sums_kernel   one wave per 16 pairs: k and b (FP64 sums over members)
  *   mvlr_cfg_kernel    one thread per (pair, configuration): Sigma, Sigma^-1,
  *                      Sigma^-1 t, t, eVb (structure-of-arrays, coalesced)
  *   mvlr_grid_kernel   one thread per (pair, raw row): M, LU, log10 ABF
@@ -121,7 +121,7 @@ __device__ inline void lu_apply(const double (&A)[SM][SM], const int (&piv)[SM],
 
 __global__ void mv_zero_kernel(int* p) { *p = 0; }
 
-/* ---- per-gene preparation: one wave per gene ------------------------------------ */
+/* ---- per-gene preparation ------------------------------------------ */
 struct MvPrep {
   MvRec* mrec;
   int32_t* midx; /* [G][N] member sample indices            */
@@ -134,9 +134,16 @@ struct MvPrep {
   int KU;
 };
 
+/* Eight waves: the first finds the members and the basis, then they share the
+ * subgroups and the entries of Y~'Y~.  Bound by the chain of wave sums; 60 genes, 9
+ * subgroups of 150, 3 covariates: 76 us (119 us with one wave). */
+constexpr int MV_PREP_WAVES = 8;
+
 template <int SM>
-__global__ void __launch_bounds__(64) mvlr_prep_kernel(const eqbf_chunk c, const MvPrep pp) {
-  const int S = c.n_subgroups, N = c.n_samples, g = blockIdx.x, lane = threadIdx.x;
+__global__ void __launch_bounds__(64 * MV_PREP_WAVES) mvlr_prep_kernel(const eqbf_chunk c, const MvPrep pp) {
+  __shared__ uint32_t s_kept;
+  const int S = c.n_subgroups, N = c.n_samples, g = blockIdx.x;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int KU = pp.KU;
   MvRec r;
   r.n = 0;
@@ -146,7 +153,7 @@ __global__ void __launch_bounds__(64) mvlr_prep_kernel(const eqbf_chunk c, const
   for (int s = 0; s < S; ++s)
     if (!c.gene_in_sbgrp[(int64_t)g * S + s]) r.flags = MV_SKIP;
   if (r.flags != MV_OK) {
-    if (lane == 0) pp.mrec[g] = r;
+    if (threadIdx.x == 0) pp.mrec[g] = r;
     return;
   }
   /* members of subgroup 0 (expression level not NaN, genotyped); every other
@@ -166,7 +173,7 @@ __global__ void __launch_bounds__(64) mvlr_prep_kernel(const eqbf_chunk c, const
     }
     mismatch |= __ballot(diff) != 0ull;
     const uint64_t bal = __ballot(m0);
-    if (m0) idx[n + __popcll(bal & ((1ull << lane) - 1ull))] = i;
+    if (m0 && wv == 0) idx[n + __popcll(bal & ((1ull << lane) - 1ull))] = i;
     n += __popcll(bal);
   }
   __syncthreads();
@@ -177,7 +184,7 @@ __global__ void __launch_bounds__(64) mvlr_prep_kernel(const eqbf_chunk c, const
   else if (n < Q + 3) /* no residual degree of freedom for the F statistic */
     r.flags = MV_FEW;
   if (r.flags != MV_OK) {
-    if (lane == 0) pp.mrec[g] = r;
+    if (threadIdx.x == 0) pp.mrec[g] = r;
     return;
   }
   if (Q > 0) { /* a member without covariates is a data error (gene_snp_pair.cpp:137-144) */
@@ -185,7 +192,7 @@ __global__ void __launch_bounds__(64) mvlr_prep_kernel(const eqbf_chunk c, const
     for (int k = lane; k < n; k += 64) miss |= !c.covar_in_sbgrp[idx[k]];
     if (__ballot(miss) != 0ull) {
       r.flags = MV_SKIP;
-      if (lane == 0) {
+      if (threadIdx.x == 0) {
         atomicOr(pp.flag, FLAG_MISSING_COVAR);
         pp.mrec[g] = r;
       }
@@ -197,7 +204,7 @@ __global__ void __launch_bounds__(64) mvlr_prep_kernel(const eqbf_chunk c, const
   /* orthonormal basis of [1, covariates] by two-pass modified Gram-Schmidt;
    * each lane only touches its own rows k = lane + 64 m */
   uint32_t kept = 0;
-  for (int j = 0; j <= Q; ++j) {
+  for (int j = 0; j <= Q && wv == 0; ++j) {
     double* cj = U + (int64_t)j * N;
     for (int k = lane; k < n; k += 64)
       cj[k] = (j == 0) ? 1.0 : c.covars[((int64_t)(j - 1)) * N + idx[k]];
@@ -224,9 +231,12 @@ __global__ void __launch_bounds__(64) mvlr_prep_kernel(const eqbf_chunk c, const
       ++r.rank;
     }
   }
-  for (int j = Q + 1; j < KU; ++j)
+  if (threadIdx.x == 0) s_kept = kept;
+  __syncthreads();
+  kept = s_kept;
+  for (int j = Q + 1 + wv; j < KU; j += MV_PREP_WAVES)
     for (int k = lane; k < n; k += 64) U[(int64_t)j * N + k] = 0.0;
-  for (int s = 0; s < S; ++s) {
+  for (int s = wv; s < S; s += MV_PREP_WAVES) {
     double* ys = Y + (int64_t)s * N;
     for (int k = lane; k < n; k += 64) ys[k] = c.explevels[((int64_t)g * S + s) * N + idx[k]];
     for (int pass = 0; pass < 2; ++pass)
@@ -239,9 +249,12 @@ __global__ void __launch_bounds__(64) mvlr_prep_kernel(const eqbf_chunk c, const
         for (int k = lane; k < n; k += 64) ys[k] -= d * cl[k];
       }
   }
+  __syncthreads();
   double* yty = pp.YtY + (int64_t)g * S * S;
+  int turn = 0;
   for (int a = 0; a < S; ++a)
     for (int b = a; b < S; ++b) {
+      if (turn++ % MV_PREP_WAVES != wv) continue;
       const double* ya = Y + (int64_t)a * N;
       const double* yb = Y + (int64_t)b * N;
       double d = 0;
@@ -252,7 +265,8 @@ __global__ void __launch_bounds__(64) mvlr_prep_kernel(const eqbf_chunk c, const
         yty[b * S + a] = d;
       }
     }
-  if (lane == 0) {
+  __syncthreads();
+  if (threadIdx.x == 0) {
     /* Sigma0 = Y'TY / (n + m - q - s - 1) = Y'TY / n, m = q + s + 1 */
     double A[SM][SM];
     int piv[SM];
@@ -303,65 +317,110 @@ __device__ inline int gene_of_pair(const int64_t* __restrict__ off, int G, int64
   return lo;
 }
 
-template <int SM>
+typedef double v4d __attribute__((ext_vector_type(4)));
+
+/* One wave per 16 pairs: the sums over the members are FP64 matrix products of
+ * their genotypes with the gene's levels and covariate basis (NG groups of 16
+ * columns, rows of A), both read as the operands want them, the genotypes once.
+ * Lane l holds pair l % 16, columns l / 16 + 4 r.  The pairs of a wave may belong to
+ * several genes: one product each, for its own pairs.
+ *
+ * Bound by the latency of its reads, four steps in flight.  48,000 pairs, 9
+ * subgroups of 150, 3 covariates: 44 us.  (A thread per pair, 750 waves, read the
+ * genotypes once per basis column: 437 us.) */
+template <int NG>
 __global__ void __launch_bounds__(256) mvlr_sums_kernel(const eqbf_chunk c, const MvSums ms) {
   const int64_t NP = c.n_pairs;
-  const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (p >= NP) return;
-  const int S = c.n_subgroups, N = c.n_samples;
+  const int lane = threadIdx.x & 63, kl = lane >> 4, pl = lane & 15;
+  const int64_t p0 = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / 64 * 16;
+  if (p0 >= NP) return;
+  const int64_t p = min(p0 + pl, NP - 1);
+  const bool act = p0 + pl < NP;
+  const int S = c.n_subgroups, N = c.n_samples, KU = ms.KU;
   const int g = gene_of_pair(c.pair_offset, c.n_genes, p);
   const int64_t snp = c.pair_snp[p];
   const MvRec r = ms.mrec[g];
   bool all_geno = true;
   for (int s = 0; s < S; ++s) all_geno &= c.snp_in_sbgrp[snp * S + s] != 0;
-  if (r.flags == MV_MISMATCH && all_geno) atomicOr(ms.flag, FLAG_MVLR_SAMPLES);
+  if (act && r.flags == MV_MISMATCH && all_geno) atomicOr(ms.flag, FLAG_MVLR_SAMPLES);
   const bool has = r.flags != MV_SKIP && r.flags != MV_MISMATCH && all_geno;
+  const bool fit = act && has && r.flags != MV_FEW;
   /* the reference records the sample size of each subgroup and NaN summary
    * statistics for --error mvlr (gene_snp_pair.cpp:154-158) */
-  for (int s = 0; s < S; ++s) {
-    ms.n_out[(int64_t)s * NP + p] = has ? r.n : 0;
-    if (ms.sstats)
-      for (int k = 0; k < 5; ++k) ms.sstats[((int64_t)k * S + s) * NP + p] = NAN;
-    if (ms.stdsstats)
-      for (int k = 0; k < 3; ++k) ms.stdsstats[((int64_t)k * S + s) * NP + p] = NAN;
-  }
-  if (!has || r.flags == MV_FEW) {
-    ms.pgene[p] = -1;
-    return;
-  }
-  const int n = r.n;
-  const int32_t* idx = ms.midx + (int64_t)g * N;
-  const double* U = ms.Ut + (int64_t)g * ms.KU * N;
-  const double* Y = ms.Yt + (int64_t)g * S * N;
+  if (act)
+    for (int s = kl; s < S; s += 4) {
+      ms.n_out[(int64_t)s * NP + p] = has ? r.n : 0;
+      if (ms.sstats)
+        for (int k = 0; k < 5; ++k) ms.sstats[((int64_t)k * S + s) * NP + p] = NAN;
+      if (ms.stdsstats)
+        for (int k = 0; k < 3; ++k) ms.stdsstats[((int64_t)k * S + s) * NP + p] = NAN;
+    }
+  if (act && kl == 0) ms.pgene[p] = fit ? g : -1;
   const int64_t gbase = (int64_t)c.geno_set_of_sbgrp[0] * c.geno_set_stride + snp;
   const bool f32 = c.geno_dtype == EQBF_F32;
-  double xx = 0, b[SM];
+  uint64_t left = __ballot(fit);
+  while (left) {
+    const int gw = __builtin_amdgcn_readlane(g, __builtin_ctzll(left));
+    const bool mine = fit && g == gw;
+    left &= ~__ballot(mine);
+    const int n = ms.mrec[gw].n;
+    const int32_t* idx = ms.midx + (int64_t)gw * N;
+    /* this lane's column of each group: levels, then the basis */
+    const double* col[NG];
+    bool on[NG];
+    v4d acc[NG];
 #pragma unroll
-  for (int s = 0; s < SM; ++s) b[s] = 0;
-  for (int k = 0; k < n; ++k) {
-    const int64_t off = gbase + (int64_t)idx[k] * c.geno_ld;
-    const double x = f32 ? (double)((const float*)c.genotypes)[off] : ((const double*)c.genotypes)[off];
-    xx += x * x;
-#pragma unroll
-    for (int s = 0; s < SM; ++s)
-      if (s < S) b[s] += x * Y[(int64_t)s * N + k];
-  }
-  double proj = 0;
-  for (int q = 0; q < ms.KU; ++q) {
-    const double* uq = U + (int64_t)q * N;
-    double a = 0;
-    for (int k = 0; k < n; ++k) {
-      const int64_t off = gbase + (int64_t)idx[k] * c.geno_ld;
-      const double x = f32 ? (double)((const float*)c.genotypes)[off] : ((const double*)c.genotypes)[off];
-      a += x * uq[k];
+    for (int j = 0; j < NG; ++j) {
+      const int m = 16 * j + pl;
+      on[j] = m < S + KU;
+      col[j] = m < S ? ms.Yt + ((int64_t)gw * S + m) * N : ms.Ut + ((int64_t)gw * KU + min(m - S, KU - 1)) * N;
+      acc[j] = v4d{0.0, 0.0, 0.0, 0.0};
     }
-    proj += a * a;
-  }
-  ms.kb[p] = xx - proj;
+    double xx = 0.0;
+    for (int k0 = 0; k0 < n; k0 += 16) {
+      int64_t at[4];
+      double x[4], v[4][NG];
 #pragma unroll
-  for (int s = 0; s < SM; ++s)
-    if (s < S) ms.kb[(int64_t)(1 + s) * NP + p] = b[s];
-  ms.pgene[p] = g;
+      for (int u = 0; u < 4; ++u) at[u] = gbase + (int64_t)idx[min(k0 + 4 * u + kl, n - 1)] * c.geno_ld;
+      if (f32) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[u] = (double)((const float*)c.genotypes)[at[u]];
+      } else {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[u] = ((const double*)c.genotypes)[at[u]];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int j = 0; j < NG; ++j) v[u][j] = col[j][min(k0 + 4 * u + kl, n - 1)];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const bool in = k0 + 4 * u + kl < n; /* past n the last member once more, with zeros */
+        xx += in ? x[u] * x[u] : 0.0;
+#pragma unroll
+        for (int j = 0; j < NG; ++j)
+          acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(in && on[j] ? v[u][j] : 0.0, x[u], acc[j], 0, 0, 0);
+      }
+    }
+    double proj = 0.0;
+#pragma unroll
+    for (int j = 0; j < NG; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int m = 16 * j + kl + 4 * q;
+        if (m < S) {
+          if (mine) ms.kb[(int64_t)(1 + m) * NP + p] = acc[j][q];
+        } else if (m < S + KU) {
+          proj += acc[j][q] * acc[j][q];
+        }
+      }
+#pragma unroll
+    for (int o = 16; o < 64; o <<= 1) {
+      xx += __shfl_xor(xx, o, 64);
+      proj += __shfl_xor(proj, o, 64);
+    }
+    if (mine && kl == 0) ms.kb[p] = xx - proj;
+  }
 }
 
 /* ---- per (pair, configuration): Sigma, Sigma^-1, Sigma^-1 t, t, eVb -------------- */
@@ -1065,7 +1124,7 @@ int mvlr_run_sm(eqbf_ctx* ctx, const eqbf_chunk& c, const eqbf_mvlr_opts* o, eqb
   {
     ProfScope ps(ctx, "mvlr_prep_kernel", st);
     with_exact_sm<SM>(c.n_subgroups, [&](auto e) {
-      hipLaunchKernelGGL(mvlr_prep_kernel<decltype(e)::value>, dim3(G), dim3(64), 0, st, c, pp);
+      hipLaunchKernelGGL(mvlr_prep_kernel<decltype(e)::value>, dim3(G), dim3(64 * MV_PREP_WAVES), 0, st, c, pp);
     });
   }
   MvSums ms;
@@ -1082,7 +1141,14 @@ int mvlr_run_sm(eqbf_ctx* ctx, const eqbf_chunk& c, const eqbf_mvlr_opts* o, eqb
   ms.KU = KU;
   {
     ProfScope ps(ctx, "mvlr_sums_kernel", st);
-    hipLaunchKernelGGL(mvlr_sums_kernel<SM>, dim3((unsigned)((NP + 255) / 256)), dim3(256), 0, st, c, ms);
+    const dim3 grid((unsigned)((NP + 63) / 64));
+    const int groups = (S + ms.KU + 15) / 16; /* S <= 16, KU <= 17 */
+    if (groups == 1)
+      hipLaunchKernelGGL(mvlr_sums_kernel<1>, grid, dim3(256), 0, st, c, ms);
+    else if (groups == 2)
+      hipLaunchKernelGGL(mvlr_sums_kernel<2>, grid, dim3(256), 0, st, c, ms);
+    else
+      hipLaunchKernelGGL(mvlr_sums_kernel<3>, grid, dim3(256), 0, st, c, ms);
   }
   EQBF_HIP(ctx, hipGetLastError());
   return mv_rows_run<SM>(ctx, c, o->bfs, out, st, [&](int64_t c0, int nb, double* par, int PSZ, int64_t pair_blocks) {
@@ -1414,8 +1480,6 @@ __global__ void __launch_bounds__(64) hyb_pres_kernel(const eqbf_chunk c, const 
  * of two second subgroups in registers had 750 waves for 1,024 SIMDs, read the
  * genotypes S (S + 1) / 4 times and an LDS word per product: 2.35 ms.)  Past 8
  * covariates the closed forms' registers allow two workgroups. */
-typedef double v4d __attribute__((ext_vector_type(4)));
-
 constexpr int HX_LD = 80, HB_LD = 66, HO_LD = 65;
 constexpr int HYB_NG = 6; /* groups of 16 columns a workgroup has at most */
 

@@ -79,3 +79,20 @@ def test_mvlr_rejects_different_samples(eng, orc):
     assert "same samples" in str(ei.value)
     with pytest.raises(RuntimeError):
         orc.assoc_mvlr(hc, "gen", 0.0, GL, GS)
+
+
+@pytest.mark.parametrize("S,N,P,Q,n_genes", [
+    (2, 64, 1, 0, 40),    # a gene per pair: many genes to a wave's 16 pairs
+    (9, 65, 17, 3, 3),    # genes end within a wave; one member past whole steps
+    (15, 67, 5, 1, 2),    # 17 columns: a second group of one
+    (16, 79, 33, 16, 2),  # 33 columns, three groups: the most subgroups and covariates
+    (10, 70, 64, 2, 1),   # the largest Hessenberg size, one whole wave of pairs
+])
+def test_mvlr_sums_and_rows_at_wave_edges(eng, orc, S, N, P, Q, n_genes):
+    hc = synth.mvlr(seed=400 + S, S=S, N=N, n_genes=n_genes, snps_per_gene=P, Q=Q)
+    if n_genes > 2:  # genes without a result between the others
+        hc.gene_in_sbgrp[1, 0] = 0
+        hc.explevels[1, 0, :] = np.nan
+    _say("[gpu] mvlr edges S=%d N=%d P=%d Q=%d" % (S, N, P, Q))
+    gpu = eng.assoc_mvlr(hc, "gen", 0.5)
+    _compare(gpu, orc.assoc_mvlr(hc, "gen", 0.5, GL, GS))
