@@ -779,14 +779,32 @@ __global__ void __launch_bounds__(64) mvlr_hess_kernel(const eqbf_chunk c, const
   out[(int64_t)(HS + 4 * SM) * NP] = et;
 }
 
-/* per (pair, group of rows): every grid point of the group from the
- * Hessenberg form (H staged in LDS, the carried vectors in registers) */
+/* a / x with r = rcp_nr(x): the quotient and its remainder's correction */
+__device__ __forceinline__ double div_by(double a, double x, double r) {
+  const double q = a * r;
+  return fma(fma(-q, x, a), r, q);
+}
+
+/* per (64 pairs, group of rows): every grid point of the group from the
+ * Hessenberg form, the points shared out among four waves.
+ *
+ * What is needed of M^-1 are the four products of (tt, vt) with M^-1 (ut, zt).  With
+ * M = L U, L^-1 (ut, zt) and (tt, vt) U^-1 both follow the elimination row by row,
+ * so that a lane holds two rows of the matrix and nothing is solved backwards; H and
+ * the carried vectors stay in LDS for the four waves.
+ *
+ * Bound by the vector unit, about 750 instructions a point (9 subgroups).  48,000
+ * pairs, 9 subgroups, 100 points: 0.28 ms.  (With U kept for the solves a wave took
+ * 344 registers, one to a SIMD, and an IEEE division for each quotient: 0.40 ms.) */
+constexpr int MV_ROW_WAVES = 4;
+
 template <int SM>
-__global__ void __launch_bounds__(64) mvlr_rows_kernel(const eqbf_chunk c, const MvGrid mg,
-                                                       const double* __restrict__ hess) {
+__global__ void __launch_bounds__(64 * MV_ROW_WAVES, 3) mvlr_rows_kernel(const eqbf_chunk c, const MvGrid mg,
+                                                                      const double* __restrict__ hess) {
   const int64_t NP = c.n_pairs;
-  const int64_t p = blockIdx.x * (int64_t)64 + threadIdx.x;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bool act = blockIdx.x * (int64_t)64 + lane < NP;
+  const int64_t p = act ? blockIdx.x * (int64_t)64 + lane : NP - 1;
   const int g = blockIdx.y;
   /* group g -> configuration (relative to the batch) and row type */
   int cfg, type;
@@ -798,8 +816,7 @@ __global__ void __launch_bounds__(64) mvlr_rows_kernel(const eqbf_chunk c, const
     type = 3;
   }
   constexpr int HS = HessIdx<SM>::size, E = HS + 4 * SM + 1;
-  __shared__ double Hs[HS][64];
-  if (p >= NP) return; /* no barrier below: each lane uses its own LDS column */
+  __shared__ double Hs[HS + 4 * SM][64]; /* H, ut, zt, tt, vt */
   const int PSZ = mg.PSZ, S = SM;
   const double* pr = mg.par + (int64_t)cfg * PSZ * NP + p;
   const bool ok = pr[(int64_t)(PSZ - 1) * NP] == 0.0;
@@ -809,10 +826,6 @@ __global__ void __launch_bounds__(64) mvlr_rows_kernel(const eqbf_chunk c, const
   const double* go = type == 3 ? mg.grid + 2 * mg.GL + mg.GS : mg.grid + mg.GL;
   const double ln10 = 2.302585092994045684;
   double* raw = mg.raw + row_base * NP + p;
-  if (!ok) {
-    for (int gi = 0; gi < n_rows; ++gi) raw[(int64_t)gi * NP] = NAN;
-    return;
-  }
   if (type == 1) { /* gen-fix: M = I + o2 k u t' */
     const double kk = pr[(int64_t)(S * S + 3 * S) * NP];
     double tu = 0.0, tz = 0.0, et = 0.0;
@@ -824,26 +837,20 @@ __global__ void __launch_bounds__(64) mvlr_rows_kernel(const eqbf_chunk c, const
       tz += t * z;
       et += z * t;
     }
-    for (int gi = 0; gi < n_rows; ++gi) {
+    for (int gi = wv; gi < n_rows; gi += MV_ROW_WAVES) {
       const double o2 = gp[gi] + go[gi];
       const double sig = 1.0 + o2 * kk * tu;
       const double quad = o2 * et * (tz / sig);
-      raw[(int64_t)gi * NP] = (0.5 * quad - 0.5 * log(fabs(sig))) / ln10;
+      if (act) raw[(int64_t)gi * NP] = ok ? (0.5 * quad - 0.5 * log(fabs(sig))) / ln10 : NAN;
     }
     return;
   }
   const double* hv = hess + (int64_t)cfg * E * NP + p;
-  for (int e = 0; e < HS; ++e) Hs[e][lane] = hv[(int64_t)e * NP];
-  double ut[SM], zt[SM], tt[SM], vt[SM];
-#pragma unroll
-  for (int i = 0; i < SM; ++i) {
-    ut[i] = hv[(int64_t)(HS + i) * NP];
-    zt[i] = hv[(int64_t)(HS + SM + i) * NP];
-    tt[i] = hv[(int64_t)(HS + 2 * SM + i) * NP];
-    vt[i] = hv[(int64_t)(HS + 3 * SM + i) * NP];
-  }
+#pragma unroll 8
+  for (int e = wv; e < HS + 4 * SM; e += MV_ROW_WAVES) Hs[e][lane] = hv[(int64_t)e * NP];
   const double et = hv[(int64_t)(HS + 4 * SM) * NP];
-  for (int gi = 0; gi < n_rows; ++gi) {
+  __syncthreads();
+  for (int gi = wv; gi < n_rows; gi += MV_ROW_WAVES) {
     double p2, o2;
     if (type == 2) { /* gen-maxh */
       p2 = gp[gi] + go[gi];
@@ -852,82 +859,70 @@ __global__ void __launch_bounds__(64) mvlr_rows_kernel(const eqbf_chunk c, const
       p2 = gp[gi];
       o2 = go[gi];
     }
-    double W[SM][SM], r1[SM], r2[SM];
+    auto entry = [&](int i, int j) { return (i == j ? 1.0 : 0.0) + p2 * Hs[HessIdx<SM>::at(i, j)][lane]; };
+    asm volatile("" ::: "memory"); /* H is read again for each point, not kept in registers */
+    double cur[SM], nxt[SM], a[SM], b[SM];
 #pragma unroll
     for (int i = 0; i < SM; ++i) {
-#pragma unroll
-      for (int j = (i == 0 ? 0 : i - 1); j < SM; ++j) W[i][j] = (i == j ? 1.0 : 0.0) + p2 * Hs[HessIdx<SM>::at(i, j)][lane];
-      r1[i] = ut[i];
-      r2[i] = zt[i];
+      cur[i] = entry(0, i);
+      a[i] = Hs[HS + 2 * SM + i][lane];
+      b[i] = Hs[HS + 3 * SM + i][lane];
     }
-    /* LU of the Hessenberg matrix, partial pivoting between rows j and j+1 */
+    double u = Hs[HS][lane], z = Hs[HS + SM][lane]; /* this row of L^-1 (ut, zt) */
+    double tu = 0.0, tz = 0.0, vu = 0.0, vz = 0.0;   /* t' M^-1 ut, ... */
     double mant = 1.0;
     int ex = 0;
+    /* LU of the Hessenberg matrix, partial pivoting between rows j and j+1 */
 #pragma unroll
-    for (int j = 0; j + 1 < SM; ++j) {
-      const bool sw = fabs(W[j + 1][j]) > fabs(W[j][j]);
+    for (int j = 0; j < SM; ++j) {
+      double un = 0.0, zn = 0.0;
+      if (j + 1 < SM) {
 #pragma unroll
-      for (int col = j; col < SM; ++col) {
-        const double a = W[j][col], b = W[j + 1][col];
-        W[j][col] = sw ? b : a;
-        W[j + 1][col] = sw ? a : b;
+        for (int col = j; col < SM; ++col) nxt[col] = entry(j + 1, col);
+        un = Hs[HS + j + 1][lane];
+        zn = Hs[HS + SM + j + 1][lane];
+        const bool sw = fabs(nxt[j]) > fabs(cur[j]);
+        auto order = [&](double& x, double& y) {
+          const double xs = sw ? y : x;
+          y = sw ? x : y;
+          x = xs;
+        };
+#pragma unroll
+        for (int col = j; col < SM; ++col) order(cur[col], nxt[col]);
+        order(u, un);
+        order(z, zn);
       }
-      {
-        const double a = r1[j], b = r1[j + 1];
-        r1[j] = sw ? b : a;
-        r1[j + 1] = sw ? a : b;
-        const double c2 = r2[j], d2 = r2[j + 1];
-        r2[j] = sw ? d2 : c2;
-        r2[j + 1] = sw ? c2 : d2;
-      }
-      const double piv = W[j][j];
-      const double f = W[j + 1][j] / piv;
-#pragma unroll
-      for (int col = j + 1; col < SM; ++col) W[j + 1][col] -= f * W[j][col];
-      r1[j + 1] -= f * r1[j];
-      r2[j + 1] -= f * r2[j];
+      const double piv = cur[j], rp = dm::rcp_nr(piv);
+      const double ya = div_by(a[j], piv, rp), yb = div_by(b[j], piv, rp);
+      tu += ya * u;
+      tz += ya * z;
+      vu += yb * u;
+      vz += yb * z;
       int e;
       mant = frexp(mant * piv, &e);
       ex += e;
-    }
-    {
-      int e;
-      mant = frexp(mant * W[SM - 1][SM - 1], &e);
-      ex += e;
+      if (j + 1 < SM) {
+        const double f = div_by(nxt[j], piv, rp);
+#pragma unroll
+        for (int col = j + 1; col < SM; ++col) {
+          a[col] -= ya * cur[col];
+          b[col] -= yb * cur[col];
+          cur[col] = nxt[col] - f * cur[col];
+        }
+        u = un - f * u;
+        z = zn - f * z;
+      }
     }
     double lnd = log(fabs(mant)) + (double)ex * 0.69314718055994530942;
-#pragma unroll
-    for (int i = SM - 1; i >= 0; --i) {
-      double a = r1[i], b = r2[i];
-#pragma unroll
-      for (int col = i + 1; col < SM; ++col) {
-        a -= W[i][col] * r1[col];
-        b -= W[i][col] * r2[col];
-      }
-      r1[i] = a / W[i][i];
-      r2[i] = b / W[i][i];
-    }
     if (o2 != 0.0) {
-      double tau = 0.0, tz = 0.0;
-#pragma unroll
-      for (int i = 0; i < SM; ++i) {
-        tau += tt[i] * r1[i];
-        tz += tt[i] * r2[i];
-      }
-      const double sig = 1.0 + o2 * tau;
+      const double sig = 1.0 + o2 * tu;
       const double coef = o2 * tz / sig;
-#pragma unroll
-      for (int i = 0; i < SM; ++i) r2[i] -= coef * r1[i];
+      tz -= coef * tu;
+      vz -= coef * vu;
       lnd += log(fabs(sig));
     }
-    double txd = 0.0, vxd = 0.0;
-#pragma unroll
-    for (int i = 0; i < SM; ++i) {
-      txd += tt[i] * r2[i];
-      vxd += vt[i] * r2[i];
-    }
-    const double quad = o2 * et * txd + p2 * vxd;
-    raw[(int64_t)gi * NP] = (0.5 * quad - 0.5 * lnd) / ln10;
+    const double quad = o2 * et * tz + p2 * vz;
+    if (act) raw[(int64_t)gi * NP] = ok ? (0.5 * quad - 0.5 * lnd) / ln10 : NAN;
   }
 }
 
@@ -1001,7 +996,8 @@ void launch_hess_rows(unsigned pair_blocks, unsigned nb, unsigned groups, hipStr
     hipLaunchKernelGGL(mvlr_hess_kernel<n>, dim3(pair_blocks, nb), dim3(64), 0, st, c, mg, hess);
   }
   ProfScope ps(ctx, "mvlr_rows_kernel", st);
-  hipLaunchKernelGGL(mvlr_rows_kernel<n>, dim3(pair_blocks, groups), dim3(64), 0, st, c, mg, (const double*)hess);
+  hipLaunchKernelGGL(mvlr_rows_kernel<n>, dim3(pair_blocks, groups), dim3(64 * MV_ROW_WAVES), 0, st, c, mg,
+                     (const double*)hess);
 }
 
 constexpr bool hess_ok(int S) { return S >= 2 && S <= 10; }
