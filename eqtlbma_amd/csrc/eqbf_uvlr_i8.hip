@@ -64,6 +64,7 @@ constexpr int I8_ROWS = 32;         /* SNP rows per pass (half a tile)          
 constexpr int I8_PLANE = I8_ROWS * 64; /* bytes of one digit plane: 32 rows x 64 samples */
 constexpr int I8_ABUF = 8 * I8_PLANE;  /* the eight planes of one step              */
 /* s_waitcnt vmcnt(n) lgkmcnt(0) (expcnt not waited for) */
+constexpr int I8_VMCNT0 = 0 | (7 << 4);
 constexpr int I8_VMCNT4 = 4 | (7 << 4);
 constexpr int I8_LGKM0 = 15 | (7 << 4) | (3 << 14); /* lgkmcnt(0) only */
 constexpr int I8_VMCNT8 = 8 | (7 << 4);
@@ -416,11 +417,11 @@ __global__ void __launch_bounds__(I8_NT) uvlr_sums_i8_kernel(const eqbf_chunk c,
      * of its SIMD still multiplies); one barrier per step.  The loop is
      * unrolled three times so that P, Q, R rotate without register copies
      * (a copy of a register a load is still writing waits for every load). */
-    auto step = [&](int ck, const xt (&P)[4], xt (&R)[4]) {
+    auto step = [&](int ck, const xt (&P)[4], xt (&R)[4], auto loads) {
       const bool more = ck + 1 < NCK;
       if (more) issue_b(ck + 1);
       __builtin_amdgcn_sched_barrier(0); /* keep the B copy ahead of the genotype loads */
-      load_x(ck + 3, R);
+      if constexpr (loads.value) load_x(ck + 3, R);
       __builtin_amdgcn_sched_barrier(0);
       const unsigned char* Bs = smem + (ck & 1) * CKB;
       const unsigned char* A = Abase + (ck & 1) * I8_ABUF;
@@ -467,19 +468,22 @@ __global__ void __launch_bounds__(I8_NT) uvlr_sums_i8_kernel(const eqbf_chunk c,
       /* the next step's B copy has landed (only the four genotype loads
        * issued after it may be in flight) and the digit writes are done;
        * every wave is done with the buffers of step ck */
-      i8_barrier<I8_VMCNT4>();
+      i8_barrier<loads.value ? I8_VMCNT4 : I8_VMCNT0>();
     };
     /* after step 0's conversion: xn = step 1, xl = step 2, xr free; whole
      * rounds of three steps in the loop (every path through its body leaves
-     * the same loads in flight), the remaining one or two after it */
+     * the same loads in flight), the remaining one or two after it.  Those load
+     * no genotypes: nothing would read them, so the compiler would drop the
+     * loads, and a wait that leaves the four newest in flight would then leave
+     * B copies in flight. */
     int ck = 0;
     for (; ck + 3 <= NCK; ck += 3) {
-      step(ck, xn, xr);
-      step(ck + 1, xl, xn);
-      step(ck + 2, xr, xl);
+      step(ck, xn, xr, std::true_type());
+      step(ck + 1, xl, xn, std::true_type());
+      step(ck + 2, xr, xl, std::true_type());
     }
-    if (ck < NCK) step(ck, xn, xr);
-    if (ck + 1 < NCK) step(ck + 1, xl, xn);
+    if (ck < NCK) step(ck, xn, xr, std::false_type());
+    if (ck + 1 < NCK) step(ck + 1, xl, xn, std::false_type());
 
     /* fold the weight classes (exact in FP64) and stage the sums in LDS:
      * E[row][col], col < CX: x'b; CX + s: x''x' over the members of s */

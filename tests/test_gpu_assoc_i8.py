@@ -141,3 +141,32 @@ def test_i8_persistent_half_tiles(eng, monkeypatch, n_all):
         err = float(np.max(np.abs(x[fin] - y[fin]), initial=0))
         _say("[gpu]   %s int8 vs FP64 product max abs diff %.2e" % (name, err))
         assert err <= 2e-5, name
+
+
+@pytest.mark.parametrize("N_all,genes,S", [(64, 2, 3), (65, 3, 5), (129, 3, 44), (300, 20, 44), (500, 40, 44)])
+def test_first_pass_of_a_context_equals_the_fp64_product(monkeypatch, N_all, genes, S):
+    # one to eight 64-sample steps, among them counts that leave one and two steps
+    # after the kernel's rounds of three.  The first pass reads memory that no
+    # cache holds, so that a step which does not wait for its coefficients shows.
+    from eqtlbma_amd.engine import Engine
+    hc = synth.batched(seed=90 + S, S=S, N_all=N_all, n_genes=genes, p_mean=150, p_lo=60, p_hi=300,
+                       ns_lo=N_all // 2, ns_hi=N_all - 1, Q=3)
+    _say("[gpu] first pass N=%d S=%d pairs=%d" % (N_all, S, hc.n_pairs))
+    out = []
+    for env in ("1", "0"):
+        monkeypatch.setenv("EQBF_I8_SUMS", env)
+        e = Engine(0)
+        e.set_grids(GL25, GS10)
+        out.append([e.assoc_uvlr(hc, analysis="join", bfs="sin", precision="mixed", want_sstats=False,
+                                 want_std=False) for _ in range(2)])
+        e.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a.n, b.n)
+        assert np.array_equal(np.isnan(a.w), np.isnan(b.w))
+        fin = np.isfinite(b.w)
+        # FP32 terms on both sides: three inputs and about five operations, each to
+        # 2^-24 of the log10 ABF, are 4.8e-7 of it a side (strong effects reach 100)
+        err = np.abs(a.w[fin] - b.w[fin])
+        k = int(np.argmax(err))
+        assert np.all(err <= 2e-5 + 1e-6 * np.abs(b.w[fin])), (float(err[k]), float(b.w[fin][k]))
+    assert np.array_equal(out[0][0].w, out[0][1].w, equal_nan=True)  # the sums are exact: no order to differ in
