@@ -75,9 +75,11 @@ constexpr int I8_VMCNT8 = 8 | (7 << 4);
  * every vector-memory operation (vmcnt(0)) before the next one, which
  * serialises the copy of the next step with the reads of this one.  The
  * instruction has no register output; its completion is awaited by the
- * explicit vmcnt of i8_barrier. */
+ * explicit vmcnt of i8_barrier.  A scalar write of M0 needs one wait state before
+ * a global load to LDS, which nobody inserts within an asm statement: without the
+ * s_nop a copy could go where the one before it went. */
 __device__ __forceinline__ void dma16(const void* src, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds_addr) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds_addr) : "memory", "m0");
 }
 
 /* Workgroup barrier after the given wait: LDS writes done (lgkmcnt(0)) and
