@@ -85,11 +85,6 @@ __device__ double block_sum(double v, double* red) {
   return t;
 }
 
-__global__ void zero_u64_kernel(uint64_t* p, int64_t n) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    p[i] = 0;
-}
-
 /* ---- prep: one workgroup per (gene, subgroup) ---------------------------------- */
 __global__ void __launch_bounds__(256) prep_kernel(const eqbf_chunk c, PrepRec* __restrict__ rec,
                                                    double* __restrict__ B, uint64_t* __restrict__ memb,
@@ -551,8 +546,8 @@ void launch_prep_reg(int blocks, hipStream_t st, const eqbf_chunk& c, PrepRec* r
 }
 
 /* ---- packed work list: tiles of up to 64 pairs of one gene ---------------------- */
-__global__ void __launch_bounds__(1024) tiles_kernel(const int64_t* __restrict__ pair_offset, int G,
-                                                     int4* __restrict__ tiles, int* __restrict__ n_tiles) {
+__device__ void tiles_list(const int64_t* __restrict__ pair_offset, int G, int4* __restrict__ tiles,
+                           int* __restrict__ n_tiles) { /* 1,024 threads */
   __shared__ int part[1024];
   __shared__ int carry;
   if (threadIdx.x == 0) carry = 0;
@@ -583,6 +578,34 @@ __global__ void __launch_bounds__(1024) tiles_kernel(const int64_t* __restrict__
     __syncthreads();
   }
   if (threadIdx.x == 0) *n_tiles = carry;
+}
+
+/* What a pass starts from, in one launch: workgroup 0 clears the flags and lists
+ * the tiles (mixed path), the others clear the membership words, the
+ * coefficients (the batched path multiplies over every sample: rows of
+ * non-members are zero) and the batched path's redo bits.  As five launches in a
+ * chain these were 20 us of the 59 us that one gene of 3 subgroups takes. */
+struct ClearArgs {
+  uint64_t *memb, *B;
+  uint32_t* redo;
+  int64_t n_memb, n_B, n_redo;
+  int* flag; /* 8 bytes */
+  const int64_t* pair_offset;
+  int4* tiles; /* null: none */
+  int* n_tiles;
+  int G;
+};
+
+__global__ void __launch_bounds__(1024) clear_kernel(const ClearArgs a) {
+  if (blockIdx.x == 0) {
+    if (threadIdx.x < 2) a.flag[threadIdx.x] = 0;
+    if (a.tiles) tiles_list(a.pair_offset, a.G, a.tiles, a.n_tiles);
+    return;
+  }
+  const int64_t first = (blockIdx.x - 1) * (int64_t)1024 + threadIdx.x, step = (gridDim.x - 1) * (int64_t)1024;
+  for (int64_t i = first; i < a.n_B; i += step) a.B[i] = 0;
+  for (int64_t i = first; i < a.n_memb; i += step) a.memb[i] = 0;
+  for (int64_t i = first; i < a.n_redo; i += step) a.redo[i] = 0;
 }
 
 /* ---- Bayes-factor phase helpers (FP32 terms, FP64 grid averages) ------------ */
@@ -1579,10 +1602,29 @@ int assoc_uvlr_run(eqbf_ctx* ctx, const eqbf_chunk* cp, const eqbf_assoc_opts* o
   if (rc) return rc;
 
   const bool fast = o->precision == EQBF_PREC_MIXED && uvlr_fast_eligible(c, KU);
-  hipLaunchKernelGGL(zero_u64_kernel, dim3(1024), dim3(256), 0, st, memb, (int64_t)G * N);
-  /* the batched path multiplies over every sample: rows of non-members are zero */
-  if (fast) hipLaunchKernelGGL(zero_u64_kernel, dim3(4096), dim3(256), 0, st, (uint64_t*)B, (int64_t)G * N * S * KC);
-  hipLaunchKernelGGL(zero_u64_kernel, dim3(1), dim3(64), 0, st, (uint64_t*)ctx->d_flag.ptr, (int64_t)1);
+  {
+    ClearArgs ca;
+    memset(&ca, 0, sizeof ca);
+    ca.memb = memb;
+    ca.n_memb = (int64_t)G * N;
+    ca.flag = (int*)ctx->d_flag.ptr;
+    ca.pair_offset = c.pair_offset;
+    ca.G = G;
+    if (!plain) {
+      ca.tiles = tiles;
+      ca.n_tiles = n_tiles;
+    }
+    if (fast) {
+      ca.B = (uint64_t*)B;
+      ca.n_B = (int64_t)G * N * S * KC;
+      ca.redo = uvlr_fast_redo(ctx, c, ca.n_redo);
+      if (!ca.redo) return EQBF_ERR_HIP; /* ctx_buf has set the message */
+    }
+    const int64_t n = ca.n_memb + ca.n_B + ca.n_redo;
+    ProfScope ps(ctx, "clear_kernel", st);
+    hipLaunchKernelGGL(clear_kernel, dim3(1 + (unsigned)std::min<int64_t>((n + 4095) / 4096, 2048)), dim3(1024), 0, st,
+                       ca);
+  }
   {
     ProfScope ps(ctx, "prep_kernel", st);
     const size_t plds = (size_t)N * (KC * sizeof(double) + sizeof(int));
@@ -1665,10 +1707,6 @@ int assoc_uvlr_run(eqbf_ctx* ctx, const eqbf_chunk* cp, const eqbf_assoc_opts* o
 
   /* mixed path */
   if (join && n_cfg > 60000) return ctx_fail(ctx, EQBF_ERR_UNSUPPORTED, "too many configurations");
-  {
-    ProfScope ps(ctx, "tiles_kernel", st);
-    hipLaunchKernelGGL(tiles_kernel, dim3(1), dim3(1024), 0, st, c.pair_offset, G, tiles, n_tiles);
-  }
   if (fast) {
     rc = uvlr_fast_run(ctx, c, o, out, st, rec, B, memb, idx, tiles, n_tiles, KU, d_masks, (int)n_cfg);
     if (rc) return rc;

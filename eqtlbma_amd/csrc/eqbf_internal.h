@@ -443,6 +443,8 @@ void launch_tiles(const int64_t* pair_offset, int G, int4* tiles, int* n_tiles, 
 void launch_zero_u64(uint64_t* p, int64_t n, hipStream_t st);
 /* batched mixed-precision uvlr path (one genotype set, matrix-core sums) */
 bool uvlr_fast_eligible(const eqbf_chunk& c, int KU);
+uint32_t* uvlr_fast_redo(eqbf_ctx* ctx, const eqbf_chunk& c, int64_t& words);
+/* the redo bits are clear on entry */
 int uvlr_fast_run(eqbf_ctx* ctx, const eqbf_chunk& c, const eqbf_assoc_opts* o, eqbf_assoc_out* out, hipStream_t st,
                   const PrepRec* rec, const double* B, const uint64_t* memb, const int32_t* idx, const int4* tiles,
                   const int* n_tiles, int KU, const uint64_t* d_masks, int n_cfg);

@@ -464,9 +464,6 @@ __device__ inline bool uvlr_bf_inputs_fast(const PrepRec& r, double xx, double s
  * non-member is not read (GeneSnpPair::FillStlContainers reads the members'
  * genotypes only, gene_snp_pair.cpp:79-170). */
 constexpr int NT_REPAIR = 256;
-__global__ void redo_zero_kernel(uint32_t* __restrict__ p, int64_t n) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) p[i] = 0u;
-}
 __device__ inline double repair_wave_sum(double v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
@@ -905,6 +902,12 @@ bool uvlr_fast_eligible(const eqbf_chunk& c, int KU) {
 }
 
 
+/* bits of (subgroup, pair) items that the sums kernel marks, and their words */
+uint32_t* uvlr_fast_redo(eqbf_ctx* ctx, const eqbf_chunk& c, int64_t& words) {
+  words = ((int64_t)c.n_subgroups * c.n_pairs + 31) / 32;
+  return (uint32_t*)ctx_buf(ctx, "sums_redo", (size_t)(words + 2) * sizeof(uint32_t));
+}
+
 int uvlr_fast_run(eqbf_ctx* ctx, const eqbf_chunk& c, const eqbf_assoc_opts* o, eqbf_assoc_out* out, hipStream_t st,
                   const PrepRec* rec, const double* B, const uint64_t* memb, const int32_t* idx, const int4* tiles,
                   const int* n_tiles, int KU, const uint64_t* d_masks, int n_cfg) {
@@ -955,11 +958,10 @@ int uvlr_fast_run(eqbf_ctx* ctx, const eqbf_chunk& c, const eqbf_assoc_opts* o, 
   const size_t max_tiles = (size_t)(NP / 64) + (size_t)G + 1;
   /* the sums go through sx2 to the statistics kernel; items the sums
    * kernel marks in the redo bitmap are recomputed in FP64 in between */
-  const int64_t redo_words = ((int64_t)S * NP + 31) / 32;
   sp.sx2 = (double*)ctx_buf(ctx, "sums_x2", (size_t)2 * S * std::max<int64_t>(NP, 1) * sizeof(double));
-  sp.redo = (uint32_t*)ctx_buf(ctx, "sums_redo", (size_t)(redo_words + 2) * sizeof(uint32_t));
+  int64_t redo_words;
+  sp.redo = uvlr_fast_redo(ctx, c, redo_words); /* cleared by the caller */
   if (!sp.sx2 || !sp.redo) return EQBF_ERR_HIP; /* ctx_buf has set the message */
-  hipLaunchKernelGGL(redo_zero_kernel, dim3(256), dim3(256), 0, st, sp.redo, redo_words);
   const size_t xsz = c.geno_dtype == EQBF_F32 ? 4 : 8;
   auto stage_bytes = [&](int kch) {
     return dma ? (size_t)kch * ((size_t)sp.CX * 8 + 64 * xsz + 8) : (size_t)8 * kch * (65 + CXPP);
