@@ -418,25 +418,15 @@ def perm_leg(args, torch, result):
             "kernels_ms_total": {k: v[0] for k, v in kern.items()},
             "kernels_launches": {k: v[1] for k, v in kern.items()},
             "egenes_p_below_0.01": int(np.sum(pv < 0.01))}
-    # roofline of the contraction: 2 N P S nperm int8 multiply-adds per gene counted once
+    # roofline of the contraction: 2 N P S nperm int8 multiply-adds per gene counted
+    # once.  Under --pbf all --maxbf the kernel also bounds and sums the statistics
+    # (the z values stay on the chip); pf_bma_kernel is then its thresholds
     if "pf_gemm_kernel" in kern:
         ops = 2.0 * N * NP * S * nperm
         gm = kern["pf_gemm_kernel"][0] / 1e3
         perm["roofline_gemm"] = {"bound": "mfma", "achieved": ops / gm / 1e12, "peak": 5000.0,
                                  "unit": "TOP/s (int8)", "frac": ops / gm / 1e12 / 5000.0, "kernel": "pf_gemm_kernel",
                                  "alg_ops": ops, "total_ms": gm * 1e3}
-    if "pf_bma_kernel" in kern:
-        # --maxbf: every z of every (SNP, subgroup, permutation) is read once to
-        # bound the SNP's statistic; only the SNPs whose bound reaches the
-        # running maximum are evaluated (310 exponentials each), so the floor
-        # is the read of the z buffer (FP32)
-        zbytes = float(NP) * S * nperm * 4
-        bm = kern["pf_bma_kernel"][0] / 1e3
-        terms = float(NP) * nperm * n_cfg * gS.shape[0]
-        perm["roofline_bma"] = {"bound": "hbm", "achieved": zbytes / bm / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                                "frac": zbytes / bm / 1e9 / HBM_PEAK_GBS, "kernel": "pf_bma_kernel",
-                                "alg_bytes": zbytes, "total_ms": bm * 1e3,
-                                "terms_if_every_snp_were_evaluated_per_s": terms / bm}
     log("perm: %d genes x %d permutations in %.2f s = %.1f genes/s; kernels %s" %
         (G, nperm, dt, value, {k: round(v[0], 1) for k, v in kern.items()}))
 
@@ -1060,11 +1050,11 @@ def hm_leg(args, torch, result):
     kern = {k: ((v[0] - before.get(k, (0.0, 0))[0]), (v[1] - before.get(k, (0, 0))[1]))
             for k, v in after.items() if v[1] > before.get(k, (0, 0))[1]}
     passes = kern.get("hm_pair_kernel", (0.0, 1))[1]
-    pk = kern.get("hm_pair_kernel", (float("nan"), 1))
+    pk = kern.get("hm_collapse_kernel", (float("nan"), 1))
     pair_ms = pk[0] / max(pk[1], 1)
-    # algorithmic bytes of one pair-kernel launch: the raw ABFs read once, the
-    # per-pair configuration, grid-point and SNP log10 sums written once
-    alg = NP * (K * L + K + L + 1) * 8.0
+    # algorithmic bytes of the one pass over the SNPs (hm_collapse_kernel, once a
+    # call): the raw ABFs read once; the EM passes run on one row per gene
+    alg = NP * K * L * 8.0
     res = {"metric": "EM iterations x SNP-gene pairs per second", "value": iters * NP / dt, "unit": "pairs/s",
            "seconds": dt, "iterations": int(iters), "passes": int(passes), "log10_lik": lik,
            "ms_per_pass": dt * 1e3 / max(passes, 1),
@@ -1072,10 +1062,10 @@ def hm_leg(args, torch, result):
                        "configurations x 10 grid points of FP64 raw log10 ABFs (%.1f GB) resident in HBM, "
                        "default start, %d iterations" % (G, NP, NP * K * L * 8 / 1e9, iters),
            "kernels_ms_per_pass": {k: v[0] / max(v[1], 1) for k, v in kern.items()},
-           "roofline": {"bound": "hbm", "kernel": "hm_pair_kernel", "alg_bytes_per_launch": alg,
+           "roofline": {"bound": "hbm", "kernel": "hm_collapse_kernel", "alg_bytes_per_launch": alg,
                         "achieved": alg / (pair_ms / 1e3) / 1e9, "peak": 8000.0, "unit": "GB/s",
                         "frac": alg / (pair_ms / 1e3) / 1e9 / 8000.0, "avg_launch_ms": pair_ms,
-                        "traffic": _load_traffic_hm("hm_pair_kernel", G)}}
+                        "traffic": _load_traffic_hm("hm_collapse_kernel", G)}}
     avg_leg(args, torch, result, eng, raw, off, off_d, K, L, 5, p.pi0, grid, cfg)
     if args.no_cpu_baseline:
         eng.close()
