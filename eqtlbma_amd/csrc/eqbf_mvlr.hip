@@ -134,14 +134,20 @@ struct MvPrep {
   int KU;
 };
 
-/* Eight waves: the first finds the members and the basis, then they share the
- * subgroups and the entries of Y~'Y~.  Bound by the chain of wave sums; 60 genes, 9
- * subgroups of 150, 3 covariates: 76 us (119 us with one wave). */
+/* Up to eight waves a gene: the first finds the members and the basis, then they
+ * share the subgroups and the entries of Y~'Y~.  Bound by the chain of wave sums; 60
+ * genes, 9 subgroups of 150, 3 covariates: 76 us (119 us with one wave).  The
+ * registers allow 2,048 waves at a time on the chip, and a wave that waits for the
+ * first one's part holds its own, so many genes take fewer waves each: 2,000 genes
+ * took 0.59 ms with eight, 0.20 ms with one. */
 constexpr int MV_PREP_WAVES = 8;
+
+inline int mv_prep_waves(int G) { return std::max(1, std::min(MV_PREP_WAVES, 2048 / std::max(G, 1))); }
 
 template <int SM>
 __global__ void __launch_bounds__(64 * MV_PREP_WAVES) mvlr_prep_kernel(const eqbf_chunk c, const MvPrep pp) {
   __shared__ uint32_t s_kept;
+  const int nwv = blockDim.x >> 6;
   const int S = c.n_subgroups, N = c.n_samples, g = blockIdx.x;
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int KU = pp.KU;
@@ -234,9 +240,9 @@ __global__ void __launch_bounds__(64 * MV_PREP_WAVES) mvlr_prep_kernel(const eqb
   if (threadIdx.x == 0) s_kept = kept;
   __syncthreads();
   kept = s_kept;
-  for (int j = Q + 1 + wv; j < KU; j += MV_PREP_WAVES)
+  for (int j = Q + 1 + wv; j < KU; j += nwv)
     for (int k = lane; k < n; k += 64) U[(int64_t)j * N + k] = 0.0;
-  for (int s = wv; s < S; s += MV_PREP_WAVES) {
+  for (int s = wv; s < S; s += nwv) {
     double* ys = Y + (int64_t)s * N;
     for (int k = lane; k < n; k += 64) ys[k] = c.explevels[((int64_t)g * S + s) * N + idx[k]];
     for (int pass = 0; pass < 2; ++pass)
@@ -254,7 +260,7 @@ __global__ void __launch_bounds__(64 * MV_PREP_WAVES) mvlr_prep_kernel(const eqb
   int turn = 0;
   for (int a = 0; a < S; ++a)
     for (int b = a; b < S; ++b) {
-      if (turn++ % MV_PREP_WAVES != wv) continue;
+      if (turn++ % nwv != wv) continue;
       const double* ya = Y + (int64_t)a * N;
       const double* yb = Y + (int64_t)b * N;
       double d = 0;
@@ -1120,7 +1126,7 @@ int mvlr_run_sm(eqbf_ctx* ctx, const eqbf_chunk& c, const eqbf_mvlr_opts* o, eqb
   {
     ProfScope ps(ctx, "mvlr_prep_kernel", st);
     with_exact_sm<SM>(c.n_subgroups, [&](auto e) {
-      hipLaunchKernelGGL(mvlr_prep_kernel<decltype(e)::value>, dim3(G), dim3(64 * MV_PREP_WAVES), 0, st, c, pp);
+      hipLaunchKernelGGL(mvlr_prep_kernel<decltype(e)::value>, dim3(G), dim3(64 * mv_prep_waves(G)), 0, st, c, pp);
     });
   }
   MvSums ms;

@@ -87,6 +87,8 @@ def test_mvlr_rejects_different_samples(eng, orc):
     (15, 67, 5, 1, 2),    # 17 columns: a second group of one
     (16, 79, 33, 16, 2),  # 33 columns, three groups: the most subgroups and covariates
     (10, 70, 64, 2, 1),   # the largest Hessenberg size, one whole wave of pairs
+    (3, 24, 1, 1, 400),   # five waves a gene in the preparation
+    (2, 20, 1, 0, 2100),  # one
 ])
 def test_mvlr_sums_and_rows_at_wave_edges(eng, orc, S, N, P, Q, n_genes):
     hc = synth.mvlr(seed=400 + S, S=S, N=N, n_genes=n_genes, snps_per_gene=P, Q=Q)
