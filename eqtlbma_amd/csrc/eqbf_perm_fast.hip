@@ -1472,7 +1472,12 @@ __global__ void __launch_bounds__(64 * PFX_WG) pf_max_kernel(const PfMaxArgs x) 
     for (int c = 0;; ++c) {
       float ze[S] = {};
       uint32_t e = 0u;
-      if (phase == 0 && __any(mask != 0)) {
+      /* Room in the queues: a turn puts at most 64 entries into queue 1, and only
+       * where 64 fit, so n1 <= PFQ; then one action, which is due whenever a queue
+       * has 64, takes 64 of them.  Queue 2 gets at most 64, and only while it has
+       * fewer than 64.  So n1 <= 128 and n2 < 128 whatever passes, and what a
+       * shift keeps is at most 64. */
+      if (phase == 0 && n1 <= PFQ - 64 && __any(mask != 0)) {
         const int k = __builtin_ctz(mask | 0x100u);
 #pragma unroll
         for (int s = 0; s < S; ++s) {

@@ -226,3 +226,35 @@ def test_max_over_all_configurations_at_tile_edges(eng, orc, S, N, P, nperm, wid
     if N > 5:  # with few samples a perfect fit may move a gene to the general path
         assert "pf_gemm_kernel" in prof and "perm_gather_kernel" not in prof
     _check(gpu, _oracle(orc, hc, tables, gene_table, "join", "all", True), "join")
+
+
+def _linked_chunk(S, block, changed, n_genes=2, N=100, P=100):
+    """Genes of P SNPs in linkage blocks: the SNPs of a block are one SNP with a
+    share of its calls drawn anew."""
+    hc = synth.plain(seed=90 + S, S=S, N=N, n_genes=n_genes, snps_per_gene=P, frac_egenes=0.0)
+    rng = np.random.default_rng(17)
+    for g in range(n_genes):
+        o = hc.pair_offset[g]
+        for b in range(0, P, block):
+            for j in range(b + 1, min(b + block, P)):
+                x = hc.genotypes[0, :, o + b].copy()
+                new = rng.random(N) < changed
+                x[new] = rng.integers(0, 3, int(new.sum()))
+                hc.genotypes[0, :, o + j] = x
+    return hc
+
+
+@pytest.mark.parametrize("S", [3, 5])
+@pytest.mark.parametrize("block", [32, 100])
+@pytest.mark.parametrize("changed", [0.0, 0.02, 0.1])
+def test_max_over_linked_snps(eng, orc, S, block, changed):
+    # where SNPs are linked most of them pass the bounds, so that the queues of
+    # candidates fill as fast as they can
+    hc = _linked_chunk(S, block, changed)
+    nperm = 200
+    tables = engine.Rng(5).tables(hc.N, 2, nperm)
+    gene_table = np.array([0, 1], np.int32)
+    _say("[gpu] maximum over linked SNPs S=%d block=%d changed=%g" % (S, block, changed))
+    gpu, prof = _run(eng, hc, tables, gene_table, "join", "all", True)
+    assert "perm_gather_kernel" not in prof
+    _check(gpu, _oracle(orc, hc, tables, gene_table, "join", "all", True), "join")
