@@ -1110,8 +1110,8 @@ __global__ void __launch_bounds__(64 * PF_WG) pf_bma_max_kernel(const PfBmaArgs 
  * since Z1^2 <= m Z2 in a configuration of m subgroups, and the sum over the
  * configurations of size m is then convex in the z_s^2, so largest where one of
  * them is T.  F is convex with a slope of at most 1 / (2 ln 2), so from the T at
- * which F reaches a level L below the running maximum M (pf_thr_kernel), M asks for
- * at least (M - L) 2 ln 2 more.  Second bound: pf_bound_sum.  Survivors pass
+ * which F reaches a level L below the running maximum M (pf_thr_kernel), or would
+ * reach it at that slope, M asks for at least (M - L) 2 ln 2 more.  Second bound: pf_bound_sum.  Survivors pass
  * through two queues per wave, 64 at a time, and what is left of all queues at the
  * end is shared out in full waves.  A z of 0 (its subgroup drops out of the
  * configurations) skips the bounds.  A wave starts with the exact value of its
@@ -1139,8 +1139,10 @@ size_t pf_max_lds(int S, int Npad) {
 }
 
 /* thr[bin][pair]: a lower bound of the T at which F reaches the bin's level, from
- * F at T = 0..63 (lane = T): the chords of a convex function lie above it.  One
- * wave per pair. */
+ * F at T = 0..63 (lane = T): the chords of a convex function lie above it.  Where
+ * F(0) is above the level, the T below 0 at which the steepest slope would reach
+ * it, so that a maximum M asks for T >= (M - F(0)) 2 ln 2 of such a SNP.  One wave
+ * per pair. */
 template <int S>
 __global__ void __launch_bounds__(256) pf_thr_kernel(const float* __restrict__ coef, int64_t nbp, int GS,
                                                      float* __restrict__ thr) {
@@ -1161,10 +1163,12 @@ __global__ void __launch_bounds__(256) pf_thr_kernel(const float* __restrict__ c
   for (int k = 0; k < PFX_BINS; ++k) {
     const float L = PFX_L0 + k - 0.0078125f; /* margin of the FP32 sums */
     const int n = __popcll(__ballot(F <= L)); /* F grows with T */
-    float t = -1.f;
+    float t;
     if (n >= 64) {
       t = 63.f;
-    } else if (n > 0) {
+    } else if (n == 0) {
+      t = (L - __shfl(F, 0, 64)) * 1.38629436f - 0.001f; /* 2 ln 2 */
+    } else {
       const float f0 = __shfl(F, n - 1, 64), f1 = __shfl(F, n, 64);
       t = (float)(n - 1) + (L - f0) / (f1 - f0) - 0.001f;
     }
@@ -1523,6 +1527,9 @@ __global__ void __launch_bounds__(64 * PFX_WG) pf_max_kernel(const PfMaxArgs x) 
       __syncthreads();
     }
   }
+  /* a maximum of nothing: the general path (the bounds keep the largest SNP, and
+   * the last barrier above is after every update) */
+  if (tid < 16 && (int64_t)pb * 16 + tid < a.nperm) fb |= mb[tid] == 0u;
   if (fb) atomicOr(&a.fallback[bi], 1);
   if (tid < 16 && (int64_t)pb * 16 + tid < a.nperm)
     x.pmax[(int64_t)x.bslot[bi] * a.NPP + (int64_t)pb * 16 + tid] = __uint_as_float(mb[tid]);

@@ -244,7 +244,7 @@ def _linked_chunk(S, block, changed, n_genes=2, N=100, P=100):
     return hc
 
 
-@pytest.mark.parametrize("S", [3, 5])
+@pytest.mark.parametrize("S", [1, 3, 5])
 @pytest.mark.parametrize("block", [32, 100])
 @pytest.mark.parametrize("changed", [0.0, 0.02, 0.1])
 def test_max_over_linked_snps(eng, orc, S, block, changed):
@@ -255,6 +255,21 @@ def test_max_over_linked_snps(eng, orc, S, block, changed):
     tables = engine.Rng(5).tables(hc.N, 2, nperm)
     gene_table = np.array([0, 1], np.int32)
     _say("[gpu] maximum over linked SNPs S=%d block=%d changed=%g" % (S, block, changed))
+    gpu, prof = _run(eng, hc, tables, gene_table, "join", "all", True)
+    assert "perm_gather_kernel" not in prof
+    _check(gpu, _oracle(orc, hc, tables, gene_table, "join", "all", True), "join")
+
+
+@pytest.mark.parametrize("S", [1, 2, 5])
+@pytest.mark.parametrize("P", [1, 2, 3, 5])
+def test_max_over_few_snps(eng, orc, S, P):
+    # a gene of few SNPs has maxima below the statistic of z = 0 times a few:
+    # the threshold of the first bound then lies below z = 0
+    hc = synth.plain(seed=60 + 7 * S + P, S=S, N=100, n_genes=4, snps_per_gene=P, frac_egenes=0.0)
+    nperm = 200
+    tables = engine.Rng(5).tables(hc.N, 4, nperm)
+    gene_table = np.arange(4, dtype=np.int32)
+    _say("[gpu] maximum over few SNPs S=%d P=%d" % (S, P))
     gpu, prof = _run(eng, hc, tables, gene_table, "join", "all", True)
     assert "perm_gather_kernel" not in prof
     _check(gpu, _oracle(orc, hc, tables, gene_table, "join", "all", True), "join")
