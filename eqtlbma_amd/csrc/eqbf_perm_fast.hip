@@ -51,6 +51,7 @@
  * is exact for every input.
  */
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -154,9 +155,13 @@ __device__ inline double block_max(double v, double* red) {
   return r;
 }
 
-/* One workgroup per (batch gene, subgroup). */
+/* One workgroup per (batch gene, subgroup).  Levels that are all equal (a gene
+ * that a subgroup does not express), or whose sum of squares leaves the normal
+ * numbers, have no R: such a gene goes to the general path (fallback, null where
+ * the caller looks after y'y = 0 itself). */
 __global__ void __launch_bounds__(256) pf_prep_y_kernel(const eqbf_chunk c, const int32_t* __restrict__ bgene,
-                                                        int Npad, uint32_t* __restrict__ W, YStat* __restrict__ ys) {
+                                                        int Npad, uint32_t* __restrict__ W, YStat* __restrict__ ys,
+                                                        int* __restrict__ fallback) {
   __shared__ double red[256];
   const int S = c.n_subgroups, N = c.n_samples;
   const int bi = blockIdx.x / S, s = blockIdx.x - bi * S;
@@ -197,7 +202,10 @@ __global__ void __launch_bounds__(256) pf_prep_y_kernel(const eqbf_chunk c, cons
     Wg[i] = word;
   }
   ts = block_sum(ts, red);
-  if (threadIdx.x == 0) ys[(int64_t)bi * S + s] = YStat{yy, ldexp(1.0, -ex), ts};
+  if (threadIdx.x == 0) {
+    ys[(int64_t)bi * S + s] = YStat{yy, ldexp(1.0, -ex), ts};
+    if (fallback && !(yy >= DBL_MIN && yy < INFINITY)) atomicOr(&fallback[bi], 1);
+  }
 }
 
 /* Genotypes of the batch pairs, SNP-major int8 [pair][Npad], and per pair
@@ -1795,7 +1803,8 @@ int perm_fast_run(eqbf_ctx* ctx, const eqbf_chunk* cp, const eqbf_perm_opts* po,
     hipLaunchKernelGGL(pf_clear_kernel, dim3((unsigned)std::min(256, (nb + 63) / 64)), dim3(64), 0, st, d_fb, nb);
     {
       ProfScope ps(ctx, "pf_prep_kernel", st);
-      hipLaunchKernelGGL(pf_prep_y_kernel, dim3(nb * S), dim3(256), 0, st, c, d_bgene, Npad, d_W, d_ys);
+      hipLaunchKernelGGL(pf_prep_y_kernel, dim3(nb * S), dim3(256), 0, st, c, d_bgene, Npad, d_W, d_ys,
+                         join ? d_fb : nullptr); /* sep: pf_gemm_kernel's own rule */
       hipLaunchKernelGGL((f32 ? pf_prep_x_kernel<float> : pf_prep_x_kernel<double>), dim3((unsigned)((nbp + 63) / 64)),
                          dim3(256), (size_t)64 * (Npad / 4 + 1) * sizeof(uint32_t), st, c, d_bpoff, d_goff, nb, Npad, d_G8,
                          d_ps, d_pf);

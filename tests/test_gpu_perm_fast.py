@@ -273,3 +273,19 @@ def test_max_over_few_snps(eng, orc, S, P):
     gpu, prof = _run(eng, hc, tables, gene_table, "join", "all", True)
     assert "perm_gather_kernel" not in prof
     _check(gpu, _oracle(orc, hc, tables, gene_table, "join", "all", True), "join")
+
+
+@pytest.mark.parametrize("pbf,use_max", [("all", True), ("all", False), ("gen", True), ("gen-sin", True)])
+@pytest.mark.parametrize("N", [60, 520])  # 520: the two kernels in the place of the fused one
+def test_constant_subgroup_takes_the_general_path(eng, orc, pbf, use_max, N):
+    # a subgroup where the gene is not expressed, all zeros: its residual sum of
+    # squares is 0 and no statistic of it has a closed form
+    hc = synth.plain(seed=23, S=3, N=N, n_genes=3, snps_per_gene=12, frac_egenes=0.34)
+    hc.explevels[1, 2] = 0.0
+    nperm = 24
+    tables = engine.Rng(5).tables(hc.N, 3, nperm)
+    gene_table = np.arange(3, dtype=np.int32)
+    _say("[gpu] constant subgroup pbf=%s max=%s N=%d" % (pbf, use_max, N))
+    gpu, prof = _run(eng, hc, tables, gene_table, "join", pbf, use_max)
+    assert "pf_prep_kernel" in prof and "perm_gather_kernel" in prof
+    _check(gpu, _oracle(orc, hc, tables, gene_table, "join", pbf, use_max), "join")
