@@ -1139,6 +1139,14 @@ constexpr int PFX_PAD = 32;   /* rows past the batch's last pair    */
 constexpr int PFX_BINS = 32;  /* levels L = PFX_L0 + bin            */
 constexpr float PFX_L0 = -2.f;
 
+/* SNPs from which a gene is worth the one kernel: its eight waves take 32 SNPs at
+ * a time, and those without a tile wait for the others.  Both kernels of a gene's
+ * share, one and two kernels, us for 1,000 permutations of (genes x SNPs): S = 1,
+ * N = 100: 1,034 / 336 (375 x 64), 408 / 368 (125 x 192), 360 / 426 (93 x 256); S =
+ * 3, N = 200: 2,009 / 1,013, 759 / 850, 654 / 928; S = 5, N = 300: 1,758 / 1,158
+ * (187 x 64), 1,206 / 1,024 (125 x 96), 927 / 1,066 (93 x 128). */
+constexpr int64_t pf_max_snps(int S) { return S <= 3 ? 224 : 128; }
+
 /* bytes of LDS: fragments, then the digit words (phase 1) or the queues */
 size_t pf_max_lds(int S, int Npad) {
   const size_t frag = (size_t)S * (Npad / 64) * 4 * 64 * 16;
@@ -1687,10 +1695,22 @@ int perm_fast_run(eqbf_ctx* ctx, const eqbf_chunk* cp, const eqbf_perm_opts* po,
     zeta_budget = std::max(zeta_budget, (size_t)256 << 20);
   }
   /* --pbf all --maxbf: in one kernel where its fragments fit the LDS and the
-   * genotypes of a tile its registers, else with the bounds on stored z values */
+   * genotypes of a tile its registers, else with the bounds on stored z values.
+   * Genes of few SNPs (pf_max_snps) take the latter too, last and in batches of
+   * their own, where no gene has more or where they are enough work: a batch costs
+   * 50 to 150 us in launches, which 2,048 workgroups (gene x 16 permutations) of
+   * the one kernel cost more than.  24 genes, 10,000 permutations, S = 5: six genes
+   * of 20 SNPs among 18 of 1,000, 5,580 us together, 4,755 apart; one among 23,
+   * 5,494 and 5,558; ten genes, 1,000 permutations, S = 3, one of 20 SNPs among 500,
+   * 325 and 479. */
   const bool prune = join && mode == PF_JOIN_ALL && po->use_max_bf && S <= 6 &&
                      (size_t)64 * GS * NCF * sizeof(float) <= 48 * 1024;
-  const bool fused = prune && !wide && nks <= PFX_NKS && pf_max_lds(S, Npad) <= (size_t)158 * 1024;
+  const bool fits = prune && !wide && nks <= PFX_NKS && pf_max_lds(S, Npad) <= (size_t)158 * 1024;
+  auto large = [&](int g) { return off[g + 1] - off[g] >= pf_max_snps(S); };
+  const int64_t n_large = std::count_if(genes.begin(), genes.end(), large), n_small = (int64_t)genes.size() - n_large;
+  const bool apart = n_large == 0 || n_small * npb16 > 2048;
+  auto in_one = [&](int g) { return fits && (!apart || large(g)); };
+  if (fits && apart) std::stable_partition(genes.begin(), genes.end(), in_one);
   const int s_lo = (!join && po->sep_sbgrp >= 0) ? po->sep_sbgrp : 0;
   const int s_hi = (!join && po->sep_sbgrp >= 0) ? po->sep_sbgrp + 1 : S;
 
@@ -1714,6 +1734,7 @@ int perm_fast_run(eqbf_ctx* ctx, const eqbf_chunk* cp, const eqbf_perm_opts* po,
   std::vector<int> fb_all;
   size_t gi = 0;
   while (gi < genes.size()) {
+    const bool fused = in_one(genes[gi]);
     /* gather the batch */
     std::vector<int32_t> bgene, btable, bslot;
     std::vector<int64_t> bpoff(1, 0), goff;
@@ -1721,6 +1742,7 @@ int perm_fast_run(eqbf_ctx* ctx, const eqbf_chunk* cp, const eqbf_perm_opts* po,
     int nslots = 0;
     while (gi < genes.size()) {
       const int g = genes[gi];
+      if (in_one(g) != fused) break;
       const int64_t np = off[g + 1] - off[g];
       const size_t zb = join && !fused ? (size_t)np * S * NPP * sizeof(float) : 0;
       if (!bgene.empty() && (zbytes + zb > zeta_budget || bgene.size() >= 4096 || bpoff.back() + np > ((int64_t)1 << 23) ||

@@ -208,6 +208,14 @@ def test_perfect_fit_falls_back_to_general_path(eng, orc):
     (4, 65, 300, 17, False),   # a second step of one sample; more tiles than waves
     (5, 512, 70, 33, False),   # the most steps whose fragments and queues fit at S = 5
     (6, 300, 40, 20, False),
+    (1, 100, 223, 17, False),  # the last size of the two kernels and the first of the one
+    (1, 100, 224, 17, False),
+    (3, 64, 255, 33, False),   # eight tile pairs, one SNP less, one more
+    (2, 63, 256, 16, False),
+    (3, 64, 257, 17, False),
+    (5, 320, 127, 20, False),  # the line at four subgroups and more
+    (5, 320, 128, 20, False),
+    (6, 300, 161, 15, False),
     (3, 513, 40, 20, False),   # one step more than the fused kernel holds
     (3, 64, 40, 20, True),     # a genotype too large for its 32-bit digit pairs
 ])
@@ -228,7 +236,7 @@ def test_max_over_all_configurations_at_tile_edges(eng, orc, S, N, P, nperm, wid
     _check(gpu, _oracle(orc, hc, tables, gene_table, "join", "all", True), "join")
 
 
-def _linked_chunk(S, block, changed, n_genes=2, N=100, P=100):
+def _linked_chunk(S, block, changed, n_genes=2, N=100, P=300):
     """Genes of P SNPs in linkage blocks: the SNPs of a block are one SNP with a
     share of its calls drawn anew."""
     hc = synth.plain(seed=90 + S, S=S, N=N, n_genes=n_genes, snps_per_gene=P, frac_egenes=0.0)
@@ -245,13 +253,14 @@ def _linked_chunk(S, block, changed, n_genes=2, N=100, P=100):
 
 
 @pytest.mark.parametrize("S", [1, 3, 5])
-@pytest.mark.parametrize("block", [32, 100])
+@pytest.mark.parametrize("block", [32, 300])
 @pytest.mark.parametrize("changed", [0.0, 0.02, 0.1])
 def test_max_over_linked_snps(eng, orc, S, block, changed):
     # where SNPs are linked most of them pass the bounds, so that the queues of
-    # candidates fill as fast as they can
+    # candidates fill as fast as they can; identical ones are one SNP, whose maxima
+    # may lie below its statistic of z = 0
     hc = _linked_chunk(S, block, changed)
-    nperm = 200
+    nperm = 100
     tables = engine.Rng(5).tables(hc.N, 2, nperm)
     gene_table = np.array([0, 1], np.int32)
     _say("[gpu] maximum over linked SNPs S=%d block=%d changed=%g" % (S, block, changed))
@@ -263,8 +272,7 @@ def test_max_over_linked_snps(eng, orc, S, block, changed):
 @pytest.mark.parametrize("S", [1, 2, 5])
 @pytest.mark.parametrize("P", [1, 2, 3, 5])
 def test_max_over_few_snps(eng, orc, S, P):
-    # a gene of few SNPs has maxima below the statistic of z = 0 times a few:
-    # the threshold of the first bound then lies below z = 0
+    # a gene of few SNPs has maxima around and below the statistic of z = 0
     hc = synth.plain(seed=60 + 7 * S + P, S=S, N=100, n_genes=4, snps_per_gene=P, frac_egenes=0.0)
     nperm = 200
     tables = engine.Rng(5).tables(hc.N, 4, nperm)
@@ -276,16 +284,34 @@ def test_max_over_few_snps(eng, orc, S, P):
 
 
 @pytest.mark.parametrize("pbf,use_max", [("all", True), ("all", False), ("gen", True), ("gen-sin", True)])
-@pytest.mark.parametrize("N", [60, 520])  # 520: the two kernels in the place of the fused one
-def test_constant_subgroup_takes_the_general_path(eng, orc, pbf, use_max, N):
+@pytest.mark.parametrize("P", [12, 240])  # with the maximum of "all": two kernels, one kernel
+def test_constant_subgroup_takes_the_general_path(eng, orc, pbf, use_max, P):
     # a subgroup where the gene is not expressed, all zeros: its residual sum of
     # squares is 0 and no statistic of it has a closed form
-    hc = synth.plain(seed=23, S=3, N=N, n_genes=3, snps_per_gene=12, frac_egenes=0.34)
+    hc = synth.plain(seed=23, S=3, N=60, n_genes=3, snps_per_gene=P, frac_egenes=0.34)
     hc.explevels[1, 2] = 0.0
     nperm = 24
     tables = engine.Rng(5).tables(hc.N, 3, nperm)
     gene_table = np.arange(3, dtype=np.int32)
-    _say("[gpu] constant subgroup pbf=%s max=%s N=%d" % (pbf, use_max, N))
+    _say("[gpu] constant subgroup pbf=%s max=%s P=%d" % (pbf, use_max, P))
     gpu, prof = _run(eng, hc, tables, gene_table, "join", pbf, use_max)
     assert "pf_prep_kernel" in prof and "perm_gather_kernel" in prof
     _check(gpu, _oracle(orc, hc, tables, gene_table, "join", pbf, use_max), "join")
+
+
+@pytest.mark.parametrize("n_small,nperm", [(3, 50), (42, 800)])  # with the large genes, apart from them
+def test_genes_of_few_and_of_many_snps_in_one_chunk(eng, orc, n_small, nperm):
+    # apart, the genes are taken in another order than the chunk's, in two batches
+    sizes = [(3, 1, 4)[k % 3] for k in range(n_small)] + [40]
+    sizes[1:1], sizes[3:3] = [230], [224]
+    hc = synth.plain(seed=71, S=2, N=60, n_genes=len(sizes), snps_per_gene=230, frac_egenes=0.34)
+    hc.pair_snp = np.concatenate([np.arange(g * 230, g * 230 + n) for g, n in enumerate(sizes)]).astype(np.int32)
+    hc.pair_offset = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int64)
+    tables = engine.Rng(5).tables(hc.N, len(sizes) - 1, nperm)
+    gene_table = np.arange(len(sizes), dtype=np.int32) - 1
+    gene_table[0], gene_table[2] = 1, -1
+    _say("[gpu] %d genes of few SNPs, 2 of many" % n_small)
+    gpu, prof = _run(eng, hc, tables, gene_table, "join", "all", True)
+    assert "perm_gather_kernel" not in prof
+    assert np.all(np.isnan(gpu[2]))
+    _check(gpu, _oracle(orc, hc, tables, gene_table, "join", "all", True), "join")
