@@ -419,13 +419,14 @@ def perm_leg(args, torch, result):
             "kernels_launches": {k: v[1] for k, v in kern.items()},
             "egenes_p_below_0.01": int(np.sum(pv < 0.01))}
     # roofline of the contraction: 2 N P S nperm int8 multiply-adds per gene counted
-    # once.  Under --pbf all --maxbf the kernel also bounds and sums the statistics
-    # (the z values stay on the chip); pf_bma_kernel is then its thresholds
-    if "pf_gemm_kernel" in kern:
+    # once.  pf_max_kernel (--pbf all --maxbf) also bounds and sums the statistics:
+    # the z values stay on the chip
+    name = next((k for k in ("pf_max_kernel", "pf_gemm_kernel") if k in kern), None)
+    if name:
         ops = 2.0 * N * NP * S * nperm
-        gm = kern["pf_gemm_kernel"][0] / 1e3
+        gm = kern[name][0] / 1e3
         perm["roofline_gemm"] = {"bound": "mfma", "achieved": ops / gm / 1e12, "peak": 5000.0,
-                                 "unit": "TOP/s (int8)", "frac": ops / gm / 1e12 / 5000.0, "kernel": "pf_gemm_kernel",
+                                 "unit": "TOP/s (int8)", "frac": ops / gm / 1e12 / 5000.0, "kernel": name,
                                  "alg_ops": ops, "total_ms": gm * 1e3}
     log("perm: %d genes x %d permutations in %.2f s = %.1f genes/s; kernels %s" %
         (G, nperm, dt, value, {k: round(v[0], 1) for k, v in kern.items()}))

@@ -1551,15 +1551,13 @@ __global__ void __launch_bounds__(64 * PFX_WG) pf_max_kernel(const PfMaxArgs x) 
     x.pmax[(int64_t)x.bslot[bi] * a.NPP + (int64_t)pb * 16 + tid] = __uint_as_float(mb[tid]);
 }
 
-/* profiled under the names of the two kernels that the one takes the place of:
- * the thresholds with the Bayes factors, the rest with the contraction */
 template <int S>
 void launch_pf_max_s(eqbf_ctx* ctx, hipStream_t st, const PfMaxArgs& x, float* thr, size_t lds) {
   {
-    ProfScope ps(ctx, "pf_bma_kernel", st);
+    ProfScope ps(ctx, "pf_thr_kernel", st);
     hipLaunchKernelGGL(pf_thr_kernel<S>, dim3((unsigned)((x.nbp + 3) / 4)), dim3(256), 0, st, x.coef, x.nbp, x.GS, thr);
   }
-  ProfScope ps(ctx, "pf_gemm_kernel", st);
+  ProfScope ps(ctx, "pf_max_kernel", st);
   hipLaunchKernelGGL(pf_max_kernel<S>, dim3((unsigned)((x.g.n_items + 7) / 8 * 8)), dim3(64 * PFX_WG), lds, st, x);
 }
 void launch_pf_max(eqbf_ctx* ctx, int S, hipStream_t st, const PfMaxArgs& x, float* thr, size_t lds) {

@@ -206,7 +206,7 @@ def test_perfect_fit_falls_back_to_general_path(eng, orc):
     (2, 63, 31, 15, False),    # one sample short of a step; a partial tile pair
     (3, 64, 33, 16, False),    # whole steps; a second pair of one SNP
     (4, 65, 300, 17, False),   # a second step of one sample; more tiles than waves
-    (5, 512, 70, 33, False),   # the most steps whose fragments and queues fit at S = 5
+    (5, 512, 70, 33, False),
     (6, 300, 40, 20, False),
     (1, 100, 223, 17, False),  # the last size of the two kernels and the first of the one
     (1, 100, 224, 17, False),
@@ -214,10 +214,15 @@ def test_perfect_fit_falls_back_to_general_path(eng, orc):
     (2, 63, 256, 16, False),
     (3, 64, 257, 17, False),
     (5, 320, 127, 20, False),  # the line at four subgroups and more
-    (5, 320, 128, 20, False),
-    (6, 300, 161, 15, False),
-    (3, 513, 40, 20, False),   # one step more than the fused kernel holds
+    (5, 320, 128, 20, False),  # the most samples that fit at each number of subgroups
+    (6, 256, 161, 15, False),
+    (4, 448, 130, 18, False),
+    (3, 512, 230, 20, False),
+    (3, 513, 230, 20, False),  # one step more than the fused kernel holds
+    (4, 449, 130, 18, False),  # fragments that do not fit
+    (3, 513, 40, 20, False),
     (3, 64, 40, 20, True),     # a genotype too large for its 32-bit digit pairs
+    (3, 64, 230, 20, True),
 ])
 def test_max_over_all_configurations_at_tile_edges(eng, orc, S, N, P, nperm, wide):
     # the statistic is the exact one of the SNP with the maximum whichever
@@ -232,7 +237,9 @@ def test_max_over_all_configurations_at_tile_edges(eng, orc, S, N, P, nperm, wid
     _say("[gpu] fused maximum S=%d N=%d P=%d nperm=%d wide=%d" % (S, N, P, nperm, wide))
     gpu, prof = _run(eng, hc, tables, gene_table, "join", "all", True)
     if N > 5:  # with few samples a perfect fit may move a gene to the general path
-        assert "pf_gemm_kernel" in prof and "perm_gather_kernel" not in prof
+        fits = N <= {4: 448, 5: 320, 6: 256}.get(S, 512)
+        one = not wide and fits and P >= (224 if S <= 3 else 128)
+        assert ("pf_max_kernel" if one else "pf_gemm_kernel") in prof and "perm_gather_kernel" not in prof
     _check(gpu, _oracle(orc, hc, tables, gene_table, "join", "all", True), "join")
 
 
@@ -265,7 +272,7 @@ def test_max_over_linked_snps(eng, orc, S, block, changed):
     gene_table = np.array([0, 1], np.int32)
     _say("[gpu] maximum over linked SNPs S=%d block=%d changed=%g" % (S, block, changed))
     gpu, prof = _run(eng, hc, tables, gene_table, "join", "all", True)
-    assert "perm_gather_kernel" not in prof
+    assert "pf_max_kernel" in prof and "perm_gather_kernel" not in prof
     _check(gpu, _oracle(orc, hc, tables, gene_table, "join", "all", True), "join")
 
 
@@ -279,7 +286,7 @@ def test_max_over_few_snps(eng, orc, S, P):
     gene_table = np.arange(4, dtype=np.int32)
     _say("[gpu] maximum over few SNPs S=%d P=%d" % (S, P))
     gpu, prof = _run(eng, hc, tables, gene_table, "join", "all", True)
-    assert "perm_gather_kernel" not in prof
+    assert "pf_gemm_kernel" in prof and "perm_gather_kernel" not in prof
     _check(gpu, _oracle(orc, hc, tables, gene_table, "join", "all", True), "join")
 
 
@@ -295,7 +302,8 @@ def test_constant_subgroup_takes_the_general_path(eng, orc, pbf, use_max, P):
     gene_table = np.arange(3, dtype=np.int32)
     _say("[gpu] constant subgroup pbf=%s max=%s P=%d" % (pbf, use_max, P))
     gpu, prof = _run(eng, hc, tables, gene_table, "join", pbf, use_max)
-    assert "pf_prep_kernel" in prof and "perm_gather_kernel" in prof
+    one = pbf == "all" and use_max and P >= 224
+    assert ("pf_max_kernel" if one else "pf_gemm_kernel") in prof and "perm_gather_kernel" in prof
     _check(gpu, _oracle(orc, hc, tables, gene_table, "join", pbf, use_max), "join")
 
 
@@ -312,6 +320,7 @@ def test_genes_of_few_and_of_many_snps_in_one_chunk(eng, orc, n_small, nperm):
     gene_table[0], gene_table[2] = 1, -1
     _say("[gpu] %d genes of few SNPs, 2 of many" % n_small)
     gpu, prof = _run(eng, hc, tables, gene_table, "join", "all", True)
-    assert "perm_gather_kernel" not in prof
+    assert "pf_max_kernel" in prof and "perm_gather_kernel" not in prof
+    assert ("pf_gemm_kernel" in prof) == (n_small == 42)
     assert np.all(np.isnan(gpu[2]))
     _check(gpu, _oracle(orc, hc, tables, gene_table, "join", "all", True), "join")
