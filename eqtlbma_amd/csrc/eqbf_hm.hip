@@ -766,13 +766,20 @@ struct HmRun {
     return EQBF_OK;
   }
 
-  /* Configs model: each gene's SNPs summed into one row (hm_collapse_kernel).
-   * Worth its one read where a gene has two SNPs or more on average: an EM is
-   * at least three passes. */
+  /* Configs model: each gene's SNPs summed into one row (hm_collapse_kernel),
+   * where the passes over the SNPs cost more than the 25 to 60 us of its kernels
+   * and of the flags' way to the host: 2e6 raw ABFs with four SNPs a gene or more,
+   * or long genes (a gene is one workgroup's serial work in a pass), longer ones
+   * where a row has few values.  Whole EM of three iterations, us, summed and not:
+   * 70 values a row, 1,024 genes of 8 SNPs 238 / 196, of 32 228 / 256; 16,384 of 4
+   * 684 / 658, of 8 709 / 771; 16 genes of 32 202 / 182, of 64 200 / 189, of 128
+   * 199 / 205; 310 values, one gene of 32 200 / 193, of 64 200 / 202; 5 values, one
+   * gene of 128 193 / 202, 256 of 128 415 / 254.  Twelve iterations move the lines
+   * to a third of those lengths. */
   int collapse() {
     const int64_t NP = snps.NP, G = h.G;
-    if (types || NP < 2 * G) return EQBF_OK;
     const int KL = h.K * h.L;
+    if (types || (NP < (KL >= 64 ? 64 : 200) * G && (NP < 4 * G || NP * KL < 2000000))) return EQBF_OK;
     /* columns a workgroup covers, and the whole waves that hold its row groups */
     const int ny = (KL + HM_COLL_NT - 1) / HM_COLL_NT, cols = (KL + ny - 1) / ny;
     const int nt = (std::max(1, HM_COLL_NT / cols) * cols + 63) / 64 * 64;

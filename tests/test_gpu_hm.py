@@ -210,3 +210,30 @@ def test_hm_gene_sums_vs_oracle(eng, orc, K, L, G, pmax, odd):
             raw[off[g]:off[g + 1]] += np.linspace(-200, 60, off[g + 1] - off[g])[:, None, None]
     prm = orc.HmParams(0.5, np.full(L, 1 / L), cfg=np.full(K, 1 / K))
     _em_both(eng, orc, raw, off, prm, thresh=1e-3, maxit=6)
+
+
+@pytest.mark.parametrize("K,L,G,P,odd,summed", [
+    (7, 10, 20, 63, None, False), (7, 10, 20, 64, None, True),     # the line of long genes
+    (1, 5, 20, 199, None, False), (1, 5, 20, 200, "rising", True),  # ... where a row has few values
+    (31, 10, 1612, 4, None, False), (31, 10, 1613, 4, None, True),  # 2e6 raw ABFs
+    (31, 10, 2200, 3, None, False),
+    (31, 10, 30, 90, "nan", True), (3, 5, 12, 300, "inf", True), (40, 20, 6, 70, None, True),
+])
+def test_hm_line_of_the_gene_sums(eng, orc, K, L, G, P, odd, summed):
+    """Both sides of the lines from which a gene's SNPs are summed once, by the
+    kernels that ran."""
+    raw, off = _case(83 + K, G, K, L, pmin=P, pmax=P)
+    if odd == "nan":
+        raw[off[3] + 1, 1, 2] = np.nan
+        raw[off[9], K - 1, 1] = np.nan
+    elif odd == "inf":
+        raw[off[2], 1, 1] = -np.inf
+    elif odd == "rising":
+        raw += np.tile(np.linspace(-200, 60, P), G)[:, None, None]
+    prm = orc.HmParams(0.5, np.full(L, 1 / L), cfg=np.full(K, 1 / K))
+    eng.profile(True)
+    before = eng.profile_read().get("hm_collapse_kernel", (0.0, 0))[1]
+    _em_both(eng, orc, raw, off, prm, thresh=1e-3, maxit=6)
+    ran = eng.profile_read().get("hm_collapse_kernel", (0.0, 0))[1] > before
+    eng.profile(False)
+    assert ran == summed
