@@ -367,7 +367,11 @@ __device__ __forceinline__ float pf_zeta_slow(const float* __restrict__ zt, cons
  *
  * Bound by the epilogue, about 30 instructions per (SNP, permutation): the
  * digits recombined and R formed in FP64, z = R P(R^2) in FP32.  (A table of
- * z(atanh R) in LDS behind a series for atanh took 170.) */
+ * z(atanh R) in LDS behind a series for atanh took 170.)  Four waves a SIMD: left
+ * to itself the compiler takes 160 registers for the two tiles, and with three
+ * waves a call on 300 genes of 5 SNPs and 1,000 permutations, S = 5, N = 300, took
+ * 1.07 ms under sep, 0.87 with four; 24 genes of 1,000, 5,000 permutations 1.89 and
+ * 1.60, under gen 4.88 and 4.61. */
 struct PfGemmArgs {
   const int8_t* G8;
   const uint32_t* W;
@@ -452,7 +456,7 @@ __device__ __forceinline__ double pf_fold_narrow(const v4i (&acc)[4], int r) {
 }
 
 template <int MODE>
-__global__ void __launch_bounds__(256) pf_gemm_kernel(const PfGemmArgs a) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) pf_gemm_kernel(const PfGemmArgs a) {
   extern __shared__ __align__(16) unsigned char sm[];
   uint32_t* Ws = (uint32_t*)sm;
   v4i* Bf = (v4i*)(sm + (size_t)a.Npad * 4);
