@@ -1144,12 +1144,13 @@ constexpr int PFX_BINS = 32;  /* levels L = PFX_L0 + bin            */
 constexpr float PFX_L0 = -2.f;
 
 /* SNPs from which a gene is worth the one kernel: its eight waves take 32 SNPs at
- * a time, and those without a tile wait for the others.  Both kernels of a gene's
- * share, one and two kernels, us for 1,000 permutations of (genes x SNPs): S = 1,
- * N = 100: 1,034 / 336 (375 x 64), 408 / 368 (125 x 192), 360 / 426 (93 x 256); S =
- * 3, N = 200: 2,009 / 1,013, 759 / 850, 654 / 928; S = 5, N = 300: 1,758 / 1,158
- * (187 x 64), 1,206 / 1,024 (125 x 96), 927 / 1,066 (93 x 128). */
-constexpr int64_t pf_max_snps(int S) { return S <= 3 ? 224 : 128; }
+ * a time, and those without a tile wait for the others.  All kernels of both kinds,
+ * one and two, us for 1,000 permutations of (genes x SNPs): S = 1, N = 100: 1,034 /
+ * 312 (375 x 64), 408 / 349 (125 x 192), 360 / 411 (93 x 256); S = 3, N = 200:
+ * 2,004 / 914, 751 / 791, 654 / 880; S = 5, N = 300: 1,738 / 1,045 (187 x 64),
+ * 1,196 / 926 (125 x 96), 914 / 976 (93 x 128); S = 6, N = 150: 1,375 / 1,268 (93 x
+ * 128), 1,054 / 1,250 (62 x 192). */
+constexpr int64_t pf_max_snps(int S) { return S <= 3 ? 224 : S <= 5 ? 128 : 160; }
 
 /* bytes of LDS: fragments, then the digit words (phase 1) or the queues */
 size_t pf_max_lds(int S, int Npad) {

@@ -216,6 +216,7 @@ def test_perfect_fit_falls_back_to_general_path(eng, orc):
     (5, 320, 127, 20, False),  # the line at four subgroups and more
     (5, 320, 128, 20, False),  # the most samples that fit at each number of subgroups
     (6, 256, 161, 15, False),
+    (6, 256, 159, 15, False),
     (4, 448, 130, 18, False),
     (3, 512, 230, 20, False),
     (3, 513, 230, 20, False),  # one step more than the fused kernel holds
@@ -238,7 +239,7 @@ def test_max_over_all_configurations_at_tile_edges(eng, orc, S, N, P, nperm, wid
     gpu, prof = _run(eng, hc, tables, gene_table, "join", "all", True)
     if N > 5:  # with few samples a perfect fit may move a gene to the general path
         fits = N <= {4: 448, 5: 320, 6: 256}.get(S, 512)
-        one = not wide and fits and P >= (224 if S <= 3 else 128)
+        one = not wide and fits and P >= (224 if S <= 3 else 128 if S <= 5 else 160)
         assert ("pf_max_kernel" if one else "pf_gemm_kernel") in prof and "perm_gather_kernel" not in prof
     _check(gpu, _oracle(orc, hc, tables, gene_table, "join", "all", True), "join")
 
