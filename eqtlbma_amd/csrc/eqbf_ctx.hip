@@ -38,6 +38,17 @@ void* ctx_buf(eqbf_ctx* ctx, const std::string& name, size_t bytes) {
   return b.ptr;
 }
 
+void ctx_drop(eqbf_ctx* ctx, std::initializer_list<const char*> names) {
+  (void)hipDeviceSynchronize(); /* any stream may use them */
+  for (const char* n : names) {
+    auto it = ctx->bufs.find(n);
+    if (it == ctx->bufs.end()) continue;
+    if (it->second.ptr) (void)hipFree(it->second.ptr);
+    ctx->bufs.erase(it);
+    ++ctx->buf_epoch;
+  }
+}
+
 extern "C" int eqbf_create(eqbf_ctx** out, int device) {
   if (!out) return EQBF_ERR_ARG;
   *out = nullptr;

@@ -748,6 +748,16 @@ struct HmRun {
   int NC;
   std::vector<double> hpar, hred;
 
+  /* Gives the gene sums up: where their scratch does not fit, the passes run over
+   * the SNPs in the memory that those need alone. */
+  int no_sums() {
+    sums = HmRows();
+    ctx_drop(ctx, {"hm_part", "hm_one", "hm_off1", "hm_flag", "hm_rows1", "hms_cfg", "hms_grd", "hms_snp"});
+    (void)hipGetLastError(); /* the failed allocation's */
+    ctx->err.clear();
+    return EQBF_OK;
+  }
+
   /* makes the passes run over `r`; its per-row buffers on first use */
   int use(HmRows& r, const char* prefix) {
     if (!r.cfg) {
@@ -757,7 +767,10 @@ struct HmRun {
       r.grd = (double*)ctx_buf(ctx, p + "grd", n * h.L * sizeof(double));
       r.num = types ? (double*)ctx_buf(ctx, p + "num", n * h.K * h.S * sizeof(double)) : nullptr;
       r.snp = (double*)ctx_buf(ctx, p + "snp", n * sizeof(double));
-      if (!r.cfg || !r.grd || (types && !r.num) || !r.snp) return EQBF_ERR_HIP;
+      if (!r.cfg || !r.grd || (types && !r.num) || !r.snp) {
+        r.cfg = nullptr; /* none of them is used */
+        return EQBF_ERR_HIP;
+      }
     }
     h.raw = r.raw;
     h.off = r.off;
@@ -794,7 +807,7 @@ struct HmRun {
     double* one = (double*)ctx_buf(ctx, "hm_one", (size_t)G * KL * sizeof(double));
     int64_t* off1 = (int64_t*)ctx_buf(ctx, "hm_off1", (size_t)(G + 1) * sizeof(int64_t));
     int* flag = (int*)ctx_buf(ctx, "hm_flag", (size_t)G * sizeof(int));
-    if (!part || !one || !off1 || !flag) return EQBF_ERR_HIP;
+    if (!part || !one || !off1 || !flag) return no_sums();
     {
       ProfScope ps(ctx, "hm_collapse_kernel", st);
       hipLaunchKernelGGL(hm_collapse_kernel, dim3((unsigned)nb, (unsigned)ny), dim3(nt), 0, st, snps.raw, snps.off, NP,
@@ -820,7 +833,7 @@ struct HmRun {
       return EQBF_OK;
     }
     double* rows = (double*)ctx_buf(ctx, "hm_rows1", (size_t)std::max<int64_t>(h1[G], 1) * KL * sizeof(double));
-    if (!rows) return EQBF_ERR_HIP;
+    if (!rows) return no_sums();
     EQBF_HIP(ctx, hipMemcpyAsync(off1, h1.data(), (G + 1) * sizeof(int64_t), hipMemcpyHostToDevice, st));
     hipLaunchKernelGGL(hm_collapse_copy_kernel, dim3((unsigned)G), dim3(HM_NT), 0, st, snps.raw, snps.off, one, flag,
                        off1, KL, rows);
@@ -851,7 +864,11 @@ struct HmRun {
       if (d > 0) lo_d = std::min(lo_d, d);
     }
     h.range = bad ? -1.0 : 290.0 + std::log10(lo_g) + std::log10(lo_d);
-    int rc = use(!bad && sums.raw ? sums : snps, !bad && sums.raw ? "hms_" : "hm_");
+    int rc = !bad && sums.raw ? use(sums, "hms_") : use(snps, "hm_");
+    if (rc && sums.raw) {
+      no_sums();
+      rc = use(snps, "hm_");
+    }
     if (rc) return rc;
     EQBF_HIP(ctx, hipMemcpyAsync((void*)h.par, hpar.data(), hpar.size() * sizeof(double), hipMemcpyHostToDevice, st));
     return EQBF_OK;

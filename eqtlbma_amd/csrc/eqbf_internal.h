@@ -10,6 +10,7 @@
 #include <cstdint>
 #include <cstring>
 #include <cstdio>
+#include <initializer_list>
 #include <map>
 #include <string>
 #include <vector>
@@ -102,6 +103,8 @@ int ctx_fail(eqbf_ctx* ctx, int code, const char* fmt, ...);
 
 /* Returns a device buffer of at least `bytes` (contents undefined). */
 void* ctx_buf(eqbf_ctx* ctx, const std::string& name, size_t bytes);
+/* Gives back the buffers of these names. */
+void ctx_drop(eqbf_ctx* ctx, std::initializer_list<const char*> names);
 /* Ensures t-tail tables for nu in [1, nu_max] exist on the device. */
 int ctx_ensure_tz(eqbf_ctx* ctx, int nu_max, hipStream_t st);
 double* ctx_tz_table(eqbf_ctx* ctx);
@@ -439,8 +442,6 @@ int assoc_uvlr_run(eqbf_ctx* ctx, const eqbf_chunk* c, const eqbf_assoc_opts* o,
  * per device by eqbf_create). */
 int assoc_noalloc_setup(eqbf_ctx* ctx);
 /* packed work list of 64-pair tiles of every gene (one block scan) */
-void launch_tiles(const int64_t* pair_offset, int G, int4* tiles, int* n_tiles, hipStream_t st);
-void launch_zero_u64(uint64_t* p, int64_t n, hipStream_t st);
 /* batched mixed-precision uvlr path (one genotype set, matrix-core sums) */
 bool uvlr_fast_eligible(const eqbf_chunk& c, int KU);
 uint32_t* uvlr_fast_redo(eqbf_ctx* ctx, const eqbf_chunk& c, int64_t& words);
