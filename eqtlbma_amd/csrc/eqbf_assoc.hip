@@ -27,10 +27,9 @@
  *     64-pair tiles of every gene of the chunk, XCD-aware; FP64 sums and
  *     residual sums of squares; t-tail by tabulated cubic Hermite in FP64;
  *     Bayes-factor terms in FP32; grid averages with FP64 accumulation.
- *   plain (EQBF_PREC_FP64_PLAIN): one launch per gene, one thread per pair,
- *     every quantity in FP64 with the reference's loop structure;
- *     EQBF_PREC_FP64_BATCHED runs the same per-pair code for every gene of
- *     the call in one launch.
+ *   plain (EQBF_PREC_FP64_PLAIN): one launch per gene, eight waves per 64
+ *     pairs, every quantity in FP64; EQBF_PREC_FP64_BATCHED runs the same
+ *     per-pair code for every gene of the call in one launch.
  */
 #include <algorithm>
 #include <cstring>

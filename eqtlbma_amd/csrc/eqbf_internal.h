@@ -314,7 +314,8 @@ __device__ __forceinline__ double rcp_nr(double x) {
 /* 10^x for any x <= 308, -inf and NaN included: the terms of a log10 sum */
 __device__ __forceinline__ double exp10_sum(double x) { return exp10_core(x < -400.0 ? -400.0 : x); }
 
-/* log10 x, within an ulp.  x = 2^e m with m in [sqrt 1/2, sqrt 2), f = m - 1,
+/* log10 x, within an ulp, by the reduction of fdlibm's logarithm (Sun, 1993) with
+ * coefficients of its own.  x = 2^e m with m in [sqrt 1/2, sqrt 2), f = m - 1,
  * s = f / (2 + f): ln m = f - (f^2/2 - s (f^2/2 + s^2 T(s^2))), T the interpolant
  * of (2 atanh(s)/s - 2)/s^2 at seven Chebyshev nodes (4.7e-18 relative in ln m);
  * ln m is kept in two parts, and e log10 2 with a leading part that is exact.

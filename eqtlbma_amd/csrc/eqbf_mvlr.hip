@@ -29,7 +29,9 @@
  *   mvlr_sums_kernel   one wave per 16 pairs: k and b (FP64 sums over members)
  *   mvlr_cfg_kernel    one thread per (pair, configuration): Sigma, Sigma^-1,
  *                      Sigma^-1 t, t, eVb (structure-of-arrays, coalesced)
- *   mvlr_grid_kernel   one thread per (pair, raw row): M, LU, log10 ABF
+ *   mvlr_hess_kernel, mvlr_rows_kernel  2 to 10 subgroups: a Hessenberg form per
+ *                      (pair, configuration), then log10 ABFs by elimination
+ *   mvlr_grid_kernel   the others, one thread per (pair, raw row): M, LU, log10 ABF
  *   mvlr_wavg_kernel   one thread per (pair, weighted row): grid average
  *                      (utils::log10_weighted_sum)
  * followed by the BMA kernel of the univariate path (gen-sin, all).
@@ -135,8 +137,8 @@ struct MvPrep {
 };
 
 /* Up to eight waves a gene: the first finds the members and the basis, then they
- * share the subgroups and the entries of Y~'Y~.  Bound by the chain of wave sums; 60
- * genes, 9 subgroups of 150, 3 covariates: 76 us (119 us with one wave).  The
+ * share the subgroups and the entries of Y~'Y~.  Bound by the chain of wave sums; 120
+ * genes, 9 subgroups of 150, no covariates: 77 us (119 us with one wave).  The
  * registers allow 2,048 waves at a time on the chip, and a wave that waits for the
  * first one's part holds its own, so many genes take fewer waves each: 2,000 genes
  * took 0.59 ms with eight, 0.20 ms with one. */
@@ -331,8 +333,8 @@ typedef double v4d __attribute__((ext_vector_type(4)));
  * Lane l holds pair l % 16, columns l / 16 + 4 r.  The pairs of a wave may belong to
  * several genes: one product each, for its own pairs.
  *
- * Bound by the latency of its reads, four steps in flight.  48,000 pairs, 9
- * subgroups of 150, 3 covariates: 44 us.  (A thread per pair, 750 waves, read the
+ * Bound by the latency of its reads, four steps in flight.  96,000 pairs, 9
+ * subgroups of 150, no covariates: 44 us.  (A thread per pair, 1,500 waves, read the
  * genotypes once per basis column: 437 us.) */
 template <int NG>
 __global__ void __launch_bounds__(256) mvlr_sums_kernel(const eqbf_chunk c, const MvSums ms) {
@@ -799,7 +801,7 @@ __device__ __forceinline__ double div_by(double a, double x, double r) {
  * so that a lane holds two rows of the matrix and nothing is solved backwards; H and
  * the carried vectors stay in LDS for the four waves.
  *
- * Bound by the vector unit, about 750 instructions a point (9 subgroups).  48,000
+ * Bound by the vector unit, about 750 instructions a point (9 subgroups).  96,000
  * pairs, 9 subgroups, 100 points: 0.28 ms.  (With U kept for the solves a wave took
  * 344 registers, one to a SIMD, and an IEEE division for each quotient: 0.40 ms.) */
 constexpr int MV_ROW_WAVES = 4;

@@ -246,7 +246,7 @@ int eqbf_assoc_hybrid_device(eqbf_ctx* ctx, const eqbf_chunk* chunk_dev, const e
  * arrays [S][n_pairs]; n <= 0 means no result in that subgroup (HasResults,
  * gene_snp_pair.cpp:61-68).  The small-sample correction uses nu = n - 2: no
  * covariate count is known for given statistics (:273).  n <= 2 (nu <= 0)
- * gives a NaN z.  FP64 throughout, one thread per pair.  Outputs as in
+ * gives a NaN z.  FP64 throughout.  Outputs as in
  * eqbf_assoc_uvlr: n (optional, int32), stdsstats (optional), raw_abf (FP64
  * or FP32 as raw_dtype, optional), w_abf (required); sstats is not written.
  * At most 64 subgroups and grids of at most 128 points. */
