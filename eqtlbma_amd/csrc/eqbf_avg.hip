@@ -163,6 +163,17 @@ __device__ __forceinline__ int first_max(double v0, double mx, double lmax, int 
   return cand >= n ? 0 : cand;
 }
 
+/* Posterior of a dimension of weight w and log10 BF d: its term t of the SNP's
+ * sum over that sum, against mx; where the sum leaves the normal numbers (the
+ * largest d has weight 0, or a weight is negative), the reference's expression. */
+__device__ __noinline__ double post_apart(double w, double d, double mx, double sum) {
+  return exp10(log10(w) + d - l10_round(mx + log10(sum)));
+}
+__device__ __forceinline__ double post_of(double w, double t, double sum, double d, double mx) {
+  if (__builtin_expect(!(sum > 1e-290) || !(w >= 0.0), 0)) return post_apart(w, d, mx, sum);
+  return t / sum;
+}
+
 constexpr int kAvgWaves = 4;
 constexpr int kAvgRow = 16; /* longest row that a lane holds in registers (AvgArgs::gw_row) */
 
@@ -260,7 +271,7 @@ __global__ void __launch_bounds__(64 * kAvgWaves) avg_pair_kernel(const AvgArgs 
       for (int k = gl; on && k < D; k += w) {
         const double wk = (k == gl) ? dw0 : a.dw[k];
         const double t = (k == gl) ? tk : wk * dm::exp10_sum(dims[k] - mx);
-        double v = wk >= 0.0 ? t / sum : NAN; /* the reference takes the weight's logarithm */
+        double v = post_of(wk, t, sum, (k == gl) ? dk : dims[k], mx);
         if (v > 1.0) v = 1.0;
         pd[k] = v;
         if (k == gl) pk = v;
@@ -329,7 +340,7 @@ avg_rows_kernel(const AvgArgs a, int w, int n_it) {
     const double sum = gsum(isnan(d) ? 0.0 : t, w);
     int best;
     if (dims_post) {
-      double v = dw0 >= 0.0 ? t / sum : NAN; /* the reference takes the weight's logarithm */
+      double v = post_of(dw0, t, sum, d, mx);
       if (v > 1.0) v = 1.0;
       if (on) a.post_dim[(size_t)p * D + gl] = v;
       const double pmax = v > -INFINITY && on ? v : -INFINITY;

@@ -144,3 +144,25 @@ def test_avg_configs_rows_in_registers(eng, orc, D, L, S, want):
     keys = ["dim_bf", "snp_bf", "gene_bf", "best_dim"]
     keys += [k for w, k in zip("abc", ("gene_post", "post_the", "post_an")) if w in want]
     _cmp(got, ref, keys + (["post_dim", "post_sub"] if "d" in want else []))
+
+
+@pytest.mark.parametrize("D,L", [(3, 5), (31, 10), (70, 4)])  # rows in registers, the general form
+def test_avg_configs_largest_dimension_of_no_weight(eng, orc, D, L):
+    """A SNP whose largest configuration has weight 0 and lies more than 308
+    decades above the others: the sum of the weighted terms underflows, and the
+    reference's posteriors are 1 or NaN."""
+    rng = np.random.default_rng(D)
+    off = _genes(rng, 6, 2, 9)
+    NP = int(off[-1])
+    raw = rng.normal(-0.4, 0.7, (NP, D, L))
+    raw[::3, 1] += 400.0
+    raw[1::3, 1] += 295.0  # the sum is small and normal
+    raw[2, 2] += 900.0
+    cw = rng.dirichlet(np.ones(D))
+    cw[1] = 0.0
+    kw = dict(cfg_w=cw, cfg_sub=rng.integers(1, 8, D).astype(np.uint64), pi0=0.3, want=("a", "b", "c", "d", "dims"),
+              n_subgroups=3)
+    gw = rng.dirichlet(np.ones(L))
+    got, ref = eng.avg_bfs(raw, off, gw, **kw), orc.avg_bfs(raw, off, gw, **kw)
+    assert np.sum(ref["post_dim"] == 1.0) > 0
+    _cmp(got, ref, ["dim_bf", "snp_bf", "post_dim", "post_sub", "best_dim"])
