@@ -136,3 +136,25 @@ def test_inss_many_subgroups_and_tiny_errors(eng, orc, S, bfs, NP):
     got = eng.abf_from_sstats(n, sig, beta, se, bfs)
     std, raw, w = orc.abf_from_sstats(n, sig, beta, se, bfs, GL, GS)
     _check(got, std, raw, w, np.ones(NP, bool))
+
+
+@pytest.mark.parametrize("S,bfs", [(1, "gen"), (3, "all"), (9, "sin")])
+def test_inss_standard_errors_whose_square_underflows(eng, orc, S, bfs):
+    """se^2 = 0 with a finite t: log10 of the variance makes the terms -inf, and
+    NaN where phi^2 is 0 too; a NaN beside it gives 0, as in the reference."""
+    rng = np.random.default_rng(S)
+    NP = 70
+    n = np.full((S, NP), 40)
+    sig, se = np.ones((S, NP)), rng.uniform(0.05, 0.4, (S, NP))
+    beta = se * rng.normal(size=(S, NP))
+    se[0, ::2] = 1e-300
+    beta[0, ::2] = rng.choice([-1.5e-300, 1e-300, 3e-300], 35)
+    se[S - 1, ::3] = np.nan
+    got = eng.abf_from_sstats(n, sig, beta, se, bfs)
+    _std, raw, w = orc.abf_from_sstats(n, sig, beta, se, bfs, GL, GS)
+    assert np.isneginf(raw).any()
+    for a, b in ((got.raw, raw), (got.w, w)):
+        assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(np.isinf(a), np.isinf(b))
+        m = np.isfinite(b)
+        assert np.array_equal(a[~m & ~np.isnan(b)], b[~m & ~np.isnan(b)])
+        assert np.max(np.abs(a[m] - b[m]), initial=0) <= 1e-9
