@@ -1188,19 +1188,21 @@ struct P64Lws {
 };
 
 /* Rows with a subgroup whose se^2 underflows (1 / se^2 infinite): its log10 v
- * makes the reference's terms -inf, NaN where phi^2 is 0 as well, and their log10
- * sum NaN; a NaN se beside it gives 0, as everywhere.  Written over the rows. */
+ * makes the reference's terms -inf, NaN where phi^2 is 0 or another t is NaN as
+ * well, and their log10 sum NaN; a NaN se beside it gives 0, as everywhere.
+ * Written over the rows. */
 __device__ __forceinline__ void p64_underflow(const AssocParams& kp, const P64Lds& l, int S, int64_t NP, int64_t p,
                                            bool valid, int lane, int wv) {
   const int64_t n_raw = 3 * (int64_t)kp.GL + (int64_t)kp.n_cfg * kp.GS;
   for (int task = wv; task < 3 + kp.n_cfg; task += P64_WAVES) {
     const uint64_t mk = task < 3 ? ((S >= 64) ? ~0ull : ((1ull << S) - 1ull)) : kp.masks[task - 3];
-    bool odd = valid, any = false;
+    bool odd = valid, any = false, no_t = false;
     for (int s = 0; s < S; ++s) {
       const double iv = l.iv[s * 64 + lane];
       if ((mk >> s) & 1ull) {
         any |= isinf(iv);
         odd &= !isnan(iv);
+        no_t |= isnan(l.e[s * 64 + lane]);
       }
     }
     if (!(odd && any)) continue;
@@ -1210,7 +1212,7 @@ __device__ __forceinline__ void p64_underflow(const AssocParams& kp, const P64Ld
     const int64_t row0 = task < 3 ? (int64_t)task * kp.GL : 3 * (int64_t)kp.GL + (int64_t)(task - 3) * kp.GS;
     for (int gi = 0; kp.raw && gi < n; ++gi) {
       const double p2 = task == 1 ? 0.0 : phi[gi] + (task == 2 ? oma[gi] : 0.0);
-      const double v = p2 > 0.0 ? -INFINITY : NAN;
+      const double v = p2 > 0.0 && !no_t ? -INFINITY : NAN;
       const int64_t ro = raw_index(row0 + gi, p, NP, n_raw, kp.raw_tiled);
       if (kp.raw_f64)
         ((double*)kp.raw)[ro] = v;

@@ -150,6 +150,7 @@ def test_inss_standard_errors_whose_square_underflows(eng, orc, S, bfs):
     se[0, ::2] = 1e-300
     beta[0, ::2] = rng.choice([-1.5e-300, 1e-300, 3e-300], 35)
     se[S - 1, ::3] = np.nan
+    n[S - 1, ::5] = 1  # no z
     got = eng.abf_from_sstats(n, sig, beta, se, bfs)
     _std, raw, w = orc.abf_from_sstats(n, sig, beta, se, bfs, GL, GS)
     assert np.isneginf(raw).any()
