@@ -382,6 +382,7 @@ def perm_leg(args, torch, result):
         # near-ties, then the reference's counting loop on the host
         c = wl.chunk(_abi, 0, g1)
         eng.assoc_uvlr_device(c, aopts, o, sptr)
+        eng.sync()  # torch's copy does not wait for the engine's stream
         npc = int(wl.offs[g1])  # the outputs' leading dimension is this chunk's pair count
         w = out_w.view(-1)[w_all_row * npc:(w_all_row + 1) * npc].cpu().numpy()
         true_d[:g1].copy_(torch.from_numpy(np.fmax.reduceat(w, wl.offs[:g1].astype(np.int64))))
@@ -530,6 +531,7 @@ def perm_alloc_leg(args, torch, result):
 
     t0 = time.perf_counter()
     eng.assoc_uvlr_device(c_all, aopts, o, sptr)
+    eng.sync()  # torch's copy does not wait for the engine's stream
     w_all = out_w[3 + n_cfg + 1].cpu().numpy()
     true = np.maximum.reduceat(w_all, wl.offs[:G].astype(np.int64))
     t_true = time.perf_counter() - t0
@@ -553,6 +555,7 @@ def perm_alloc_leg(args, torch, result):
     t0 = time.perf_counter()
     phase = {}
     eng.assoc_uvlr_device(wl.chunk(_abi, n_train, G), aopts, o, sptr)
+    eng.sync()
     npc = int(wl.offs[G] - wl.offs[n_train])  # the outputs' leading dimension is this chunk's pair count
     w_inf = out_w.view(-1)[(3 + n_cfg + 1) * npc:(3 + n_cfg + 2) * npc].cpu().numpy()
     base = int(wl.offs[n_train])
