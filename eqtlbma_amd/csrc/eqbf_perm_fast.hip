@@ -67,7 +67,7 @@ constexpr int ZT_STRIDE = 3;                             /* every third t-tail n
 constexpr int ZT_NODES = (TZ_NODES - 1) / ZT_STRIDE + 1; /* nodes of the z table      */
 constexpr int ZP = 8;                                    /* terms of z(R) / R in R^2  */
 constexpr float ZP_RMAX = 0.5f;                          /* ... used for R below this */
-constexpr int ZT_ROW = 4 + 2 * ZT_NODES + ZP;            /* floats per z-table row    */
+constexpr int ZT_ROW = 4 + 2 * ZT_NODES + ZP + 1;        /* floats per z-table row    */
 constexpr int PF_SB = 64;            /* SNPs per Bayes-factor work item         */
 constexpr float kLog2_10f = 3.32192809488736235f;
 constexpr double kLog2_10 = 3.32192809488736235;
@@ -275,9 +275,11 @@ __global__ void __launch_bounds__(256) pf_prep_x_kernel(const eqbf_chunk c, cons
 /* After the nodes: |z| / R as a polynomial in R^2 for R <= ZP_RMAX (s = atanh R),
  * the interpolant at ZP Chebyshev nodes in R^2; z(R) / R is smooth in R^2 for
  * every nu (its nearest singularity is R^2 = 1), so that eight terms leave
- * about 1e-10 of it, far below the FP32 result.  Its rounding against 64 bits
- * (nu 10 to 2000, t from 1 to 7): 4e-8 to 7e-8 rms, 2.2e-7 at most; the table
- * has 1.0e-7 and 4.7e-7. */
+ * about 1e-10 of it, far below the FP32 result.  The constant term is kept in two
+ * parts: its rounding alone would be the same relative error in every z of a nu
+ * (5e-8 at nu = 298, of 7e-8 rms).  Rounding against 64 bits (nu 10 to 2000, t
+ * from 1 to 7): 4e-8 to 5e-8 rms, 1.7e-7 at most; the table has 1.0e-7 and
+ * 4.7e-7. */
 __device__ void pf_zeta_poly(const double* __restrict__ tz, int nu, float* __restrict__ out) {
   double x[ZP], d[ZP], c[ZP];
   for (int k = 0; k < ZP; ++k) {
@@ -293,6 +295,25 @@ __device__ void pf_zeta_poly(const double* __restrict__ tz, int nu, float* __res
     c[0] = d[k] - x[k] * c[0];
   }
   for (int k = 0; k < ZP; ++k) out[k] = (float)c[k];
+  out[ZP] = (float)(c[0] - (double)out[0]);
+}
+
+struct PfZeta {
+  float c[ZP], lo;
+};
+__device__ __forceinline__ PfZeta pf_zeta_load(const float* __restrict__ zt) {
+  PfZeta p;
+#pragma unroll
+  for (int k = 0; k < ZP; ++k) p.c[k] = zt[4 + 2 * ZT_NODES + k];
+  p.lo = zt[4 + 2 * ZT_NODES + ZP];
+  return p;
+}
+/* |z| / R at x = R^2 */
+__device__ __forceinline__ float pf_zeta_ratio(const PfZeta& p, float x) {
+  float v = p.c[ZP - 1];
+#pragma unroll
+  for (int k = ZP - 2; k > 0; --k) v = fmaf(v, x, p.c[k]);
+  return p.c[0] + fmaf(v, x, p.lo);
 }
 
 __global__ void pf_zeta_table_kernel(const double* __restrict__ tz, int nu, float* __restrict__ out) {
@@ -482,9 +503,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))
   const YStat y = a.ys[(int64_t)bi * a.S + s];
   const double kc = y.tsum / (double)N, nu = (double)a.nu, inv_yy = 1.0 / y.yy;
   const double k_row = MODE == PF_SEP ? y.scale * y.scale * inv_yy : y.scale * sqrt(inv_yy);
-  float zp[ZP];
-#pragma unroll
-  for (int k = 0; k < ZP; ++k) zp[k] = MODE == PF_SEP ? 0.f : a.zt[4 + 2 * ZT_NODES + k];
+  PfZeta zp = {};
+  if (MODE != PF_SEP) zp = pf_zeta_load(a.zt);
   const int64_t perm = (int64_t)pb * 16 + (lane & 15);
   const bool pvalid = perm < a.nperm;
   const int64_t row_step = (int64_t)a.S * a.NPP;
@@ -563,10 +583,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))
           /* R = |x'y| / sqrt(x'x y'y); |t| / sqrt(nu) = R / sqrt(1 - R^2) */
           const double R = fabs(d) * sc[u][r];
           const float Rf = (float)R, x = Rf * Rf;
-          float z = zp[ZP - 1];
-#pragma unroll
-          for (int k = ZP - 2; k >= 0; --k) z = fmaf(z, x, zp[k]);
-          z = copysignf(z * Rf, (float)d);
+          float z = copysignf(pf_zeta_ratio(zp, x) * Rf, (float)d);
           const bool on = !isnan(R);
           if (__builtin_expect(on && (!(Rf < ZP_RMAX) || x * (float)a.nu < 1e-10f), 0))
             z = pf_zeta_slow(a.zt, a.tz, a.nu, R, d, fb);
@@ -1247,9 +1264,7 @@ __global__ void __launch_bounds__(64 * PFX_WG) pf_max_kernel(const PfMaxArgs x) 
   uint32_t* q2 = q1 + QW;
   const int64_t P0 = a.bpoff[bi], np = a.bpoff[bi + 1] - P0;
   const int npair = (int)((np + 31) / 32);
-  float zp[ZP];
-#pragma unroll
-  for (int k = 0; k < ZP; ++k) zp[k] = a.zt[4 + 2 * ZT_NODES + k];
+  const PfZeta zp = pf_zeta_load(a.zt);
   const int pl = lane & 15;
   const bool pvalid = (int64_t)pb * 16 + pl < a.nperm;
   int n1 = 0, n2 = 0;
@@ -1421,9 +1436,7 @@ __global__ void __launch_bounds__(64 * PFX_WG) pf_max_kernel(const PfMaxArgs x) 
           const int u = k >> 2, r = k & 3;
           dv[k] = pf_fold_narrow(acc[u], r) - sx[u][r] * kc;
           const float Rf = (float)(fabs(dv[k]) * (rs[u][r] * kr)), x2 = Rf * Rf;
-          float v = zp[ZP - 1];
-#pragma unroll
-          for (int i = ZP - 2; i >= 0; --i) v = fmaf(v, x2, zp[i]);
+          const float v = pf_zeta_ratio(zp, x2);
           z[s][k] = __uint_as_float((__float_as_uint(v * Rf) & 0x7fffffffu) |
                                     ((uint32_t)__double2hiint(dv[k]) & 0x80000000u));
           any_slow |= Rf >= ZP_RMAX || Rf < tiny; /* NaN: no SNP */

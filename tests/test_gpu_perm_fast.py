@@ -325,3 +325,23 @@ def test_genes_of_few_and_of_many_snps_in_one_chunk(eng, orc, n_small, nperm):
     assert ("pf_gemm_kernel" in prof) == (n_small == 42)
     assert np.all(np.isnan(gpu[2]))
     _check(gpu, _oracle(orc, hc, tables, gene_table, "join", "all", True), "join")
+
+
+@pytest.mark.parametrize("pbf,use_max", [("all", True), ("all", False), ("gen", True)])
+def test_statistics_against_64_bits(eng, pbf, use_max):
+    # z in FP32 with a relative error of 5e-8 rms (rounding of R, of R^2 and of the
+    # polynomial) moves a log10 BF by z^2 / ln 10 times that: with sum z^2 of 15 to
+    # 25 at the maximum and five subgroups' errors apart, 1.5e-7 to 2.2e-7 rms, and
+    # 1e-7 more in quadrature from the sums of FP32 terms.  An error common to every
+    # z of the gene, as of a rounded leading coefficient (5e-8 at this N), would add
+    # up over the subgroups: 3.8e-7.
+    hc = synth.plain(seed=335, S=5, N=300, n_genes=4, snps_per_gene=200, frac_egenes=0.0)
+    tables = engine.Rng(3).tables(hc.N, 4, 400)
+    gene_table = np.arange(4, dtype=np.int32)
+    _say("[gpu] statistics against 64 bits pbf=%s max=%s" % (pbf, use_max))
+    gpu, prof = _run(eng, hc, tables, gene_table, "join", pbf, use_max)
+    assert "perm_gather_kernel" not in prof
+    ref = eng.perm_stats(hc, tables, gene_table, "join", pbf, use_max, precision="fp64_batched")
+    rms = float(np.sqrt(np.mean((gpu - ref) ** 2)))
+    _say("[gpu]   rms %.3g" % rms)
+    assert rms <= 2.6e-7
